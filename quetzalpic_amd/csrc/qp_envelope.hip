@@ -103,20 +103,46 @@ struct SrcEnv {
     int nx, n1, n2, use_dcur;
     double idy2, idz2, dt, c2dx;
     int e;
-    __device__ double operator()(int, int which, int j, int k) const {
+    template <int E>
+    __device__ void row(int, int which, int j, int k0, int dk, double (&v)[E]) const {
         const double *ac = a + (size_t)which * vol + (size_t)e * nn;
-        const int jm = j == 0 ? n1 - 1 : j - 1, jp = j + 1 == n1 ? 0 : j + 1;
-        const int km = k == 0 ? n2 - 1 : k - 1, kp = k + 1 == n2 ? 0 : k + 1;
-        const size_t t = (size_t)j * n2 + k;
-        const double c = ac[t];
-        const double lap = (ac[(size_t)jp * n2 + k] - 2.0 * c + ac[(size_t)jm * n2 + k]) * idy2 +
-                           (ac[(size_t)j * n2 + kp] - 2.0 * c + ac[(size_t)j * n2 + km]) * idz2;
-        const double x = chi[(size_t)e * nn + t];
-        double v = dt * (x * c - lap);
-        if (e != nx - 1) v -= c2dx * inc[(size_t)((e + 1) & 1) * 2 * nn + (size_t)which * nn + t];
-        if (use_dcur) v += 0.5 * dt * (x - cmid[e]) * inc[(size_t)(e & 1) * 2 * nn + (size_t)which * nn + t];
-        return v;
+        const double *r0 = ac + (size_t)j * n2;
+        const double *rm = ac + (size_t)(j == 0 ? n1 - 1 : j - 1) * n2, *rp = ac + (size_t)(j + 1 == n1 ? 0 : j + 1) * n2;
+        const double *xr = chi + (size_t)e * nn + (size_t)j * n2;
+        const double *ip = inc + (size_t)((e + 1) & 1) * 2 * nn + (size_t)which * nn + (size_t)j * n2;
+        const double *ic = inc + (size_t)(e & 1) * 2 * nn + (size_t)which * nn + (size_t)j * n2;
+        double c[E], cp[E], cm[E], kp[E], km[E], x[E], dp[E], dc[E], mid = 0.0;
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const int k = k0 + dk * r;
+            c[r] = r0[k];
+            cp[r] = rp[k];
+            cm[r] = rm[k];
+            kp[r] = r0[k + 1 == n2 ? 0 : k + 1];
+            km[r] = r0[k == 0 ? n2 - 1 : k - 1];
+            x[r] = xr[k];
+            dp[r] = dc[r] = 0.0;
+        }
+        if (e != nx - 1) {
+#pragma unroll
+            for (int r = 0; r < E; ++r) dp[r] = ip[k0 + dk * r];
+        }
+        if (use_dcur) {
+            mid = cmid[e];
+#pragma unroll
+            for (int r = 0; r < E; ++r) dc[r] = ic[k0 + dk * r];
+        }
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const double lap = (cp[r] - 2.0 * c[r] + cm[r]) * idy2 + (kp[r] - 2.0 * c[r] + km[r]) * idz2;
+            double u = dt * (x[r] * c[r] - lap);
+            u -= c2dx * dp[r];                                  // 0 ahead of the first slice
+            if (use_dcur) u += 0.5 * dt * (x[r] - mid) * dc[r];
+            v[r] = u;
+        }
     }
+    template <int E>
+    __device__ void done(int, int, int, int, int) const {}
 };
 
 // Last row pass: d_e (unnormalised c2r output / (n1 n2)) to the increment

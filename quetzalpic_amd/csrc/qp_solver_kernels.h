@@ -29,10 +29,18 @@ __device__ __forceinline__ bool solver_skip(const Ctl *ctl, int skip_mode) {
     return ctl_skip_b(ctl);
 }
 
+// A source hands out elements k0, k0 + dk, ... of row j (row), all loads before
+// the arithmetic, and is told when they have been read (done).
 struct SrcPlain {
     const double *a;
     int n2;
-    __device__ double operator()(int, int, int j, int k) const { return a[(size_t)j * n2 + k]; }
+    template <int E>
+    __device__ void row(int, int, int j, int k0, int dk, double (&x)[E]) const {
+#pragma unroll
+        for (int r = 0; r < E; ++r) x[r] = a[(size_t)j * n2 + k0 + dk * r];
+    }
+    template <int E>
+    __device__ void done(int, int, int, int, int) const {}
 };
 
 // Real output v of the unnormalised c2r; the reference divides by n1 then n2
@@ -86,10 +94,16 @@ __global__ __launch_bounds__(kSolverThreads) void k_rows_fwd(Src src, double2 *s
     for (int t = threadIdx.x; t < B * n2; t += blockDim.x) {
         const int bb = t / n2, k = t - bb * n2;
         const int ra = 2 * (pair0 + bb), rb = ra + 1;
-        double xa = 0.0, xb = 0.0;
-        if (ra < n1) xa = src(wk, which, ra, k);
-        if (rb < n1) xb = src(wk, which, rb, k);
-        a[t] = make_double2(xa, xb);
+        double xa[1] = {0.0}, xb[1] = {0.0};
+        if (ra < n1) {
+            src.template row<1>(wk, which, ra, k, 1, xa);
+            src.template done<1>(wk, which, ra, k, 1);
+        }
+        if (rb < n1) {
+            src.template row<1>(wk, which, rb, k, 1, xb);
+            src.template done<1>(wk, which, rb, k, 1);
+        }
+        a[t] = make_double2(xa[0], xb[0]);
     }
     __syncthreads();
     const double2 *r = lds_fft(a, b, B, ax, twl, -1);

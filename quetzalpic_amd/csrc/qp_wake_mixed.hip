@@ -590,14 +590,32 @@ struct SrcPsi {
     const Ctl *ctl;
     int slot, n2;
     size_t nn;
-    __device__ double operator()(int wk, int, int j, int k) const {
-        const size_t t = (size_t)j * n2 + k, tw = (size_t)wk * nn + t;
-        const int slice = ctl[wk].slice_of[slot];
-        const double jb = jx_b3 ? jx_b3[(size_t)slice * bstride + t] : 0.0;
-        const double rb = rho_b3 ? rho_b3[(size_t)slice * bstride + t] : 0.0;
-        const double v = acc[tw];
-        acc[tw] = 0.0;
-        return (jb - rb - rho_ion[tw]) + v;
+    template <int E>
+    __device__ void row(int wk, int, int j, int k0, int dk, double (&x)[E]) const {
+        const size_t t = (size_t)j * n2 + k0, tw = (size_t)wk * nn + t;
+        double io[E], jb[E], rb[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            x[r] = acc[tw + dk * r];
+            io[r] = rho_ion[tw + dk * r];
+            jb[r] = rb[r] = 0.0;
+        }
+        if (jx_b3 || rho_b3) {
+            const size_t o = (size_t)ctl[wk].slice_of[slot] * bstride + t;
+#pragma unroll
+            for (int r = 0; r < E; ++r) {
+                if (jx_b3) jb[r] = jx_b3[o + dk * r];
+                if (rho_b3) rb[r] = rho_b3[o + dk * r];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < E; ++r) x[r] = (jb[r] - rb[r] - io[r]) + x[r];
+    }
+    template <int E>
+    __device__ void done(int wk, int, int j, int k0, int dk) const {
+        const size_t tw = (size_t)wk * nn + (size_t)j * n2 + k0;
+#pragma unroll
+        for (int r = 0; r < E; ++r) acc[tw + dk * r] = 0.0;
     }
 };
 
@@ -606,18 +624,46 @@ struct SrcB {
     const double *by, *bz, *jx, *jy, *jz, *jyn, *jzn;
     int n1, n2;
     double D, inv_dx, inv_dy, inv_dz;  // the differences are scaled by reciprocals (no divisions)
-    __device__ double operator()(int wk, int which, int j, int k) const {
-        const size_t go = (size_t)wk * n1 * n2;
-        const size_t t = go + (size_t)j * n2 + k;
+    template <int E>
+    __device__ void row(int wk, int which, int j, int k0, int dk, double (&x)[E]) const {
+        const size_t go = (size_t)wk * n1 * n2, rj = go + (size_t)j * n2;
+        double b[E], jc[E], jn[E], ja[E], jb[E];
         if (which == 0) {
-            const double jn = k < n2 - 1 ? jx[t + 1] : jx[go + (size_t)j * n2];
-            const double djz = (jz[t] - jzn[t]) * inv_dx;
-            return -D * by[t] - (jn - jx[t]) * inv_dz + djz;
+#pragma unroll
+            for (int r = 0; r < E; ++r) {
+                const int k = k0 + dk * r;
+                b[r] = by[rj + k];
+                jc[r] = jx[rj + k];
+                jn[r] = jx[rj + (k < n2 - 1 ? k + 1 : 0)];
+                ja[r] = jz[rj + k];
+                jb[r] = jzn[rj + k];
+            }
+#pragma unroll
+            for (int r = 0; r < E; ++r) {
+                const double djz = (ja[r] - jb[r]) * inv_dx;
+                x[r] = -D * b[r] - (jn[r] - jc[r]) * inv_dz + djz;
+            }
+            return;
         }
-        const double djy = (jy[t] - jyn[t]) * inv_dx;
-        if (j < n1 - 1) return -D * bz[t] + (jx[t + n2] - jx[t]) * inv_dy - djy;
-        return -D * bz[go + k] + (jx[go + k] - jx[t]) * inv_dy - djy;
+        // the last row's source takes bz(0, k) and jx(0, k) (the reference's :563)
+        const size_t rn = j < n1 - 1 ? rj + n2 : go, rb = j < n1 - 1 ? rj : go;
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const int k = k0 + dk * r;
+            b[r] = bz[rb + k];
+            jc[r] = jx[rj + k];
+            jn[r] = jx[rn + k];
+            ja[r] = jy[rj + k];
+            jb[r] = jyn[rj + k];
+        }
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const double djy = (ja[r] - jb[r]) * inv_dx;
+            x[r] = -D * b[r] + (jn[r] - jc[r]) * inv_dy - djy;
+        }
     }
+    template <int E>
+    __device__ void done(int, int, int, int, int) const {}
 };
 
 // psi finalisation: v/n1/n2, minus the border mean (normalize_potential,
@@ -685,12 +731,23 @@ struct SrcCurl {
     const double *jy, *jz;
     int n1, n2;
     double inv_dy, inv_dz;
-    __device__ double operator()(int wk, int, int j, int k) const {
-        const size_t go = (size_t)wk * n1 * n2;
-        const int kp = k + 1 == n2 ? 0 : k + 1, jp = j + 1 == n1 ? 0 : j + 1;
-        const size_t t = go + (size_t)j * n2 + k;
-        return (jy[go + (size_t)j * n2 + kp] - jy[t]) * inv_dz - (jz[go + (size_t)jp * n2 + k] - jz[t]) * inv_dy;
+    template <int E>
+    __device__ void row(int wk, int, int j, int k0, int dk, double (&x)[E]) const {
+        const size_t go = (size_t)wk * n1 * n2, rj = go + (size_t)j * n2, rn = go + (size_t)(j + 1 == n1 ? 0 : j + 1) * n2;
+        double yc[E], yn[E], zc[E], zn[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const int k = k0 + dk * r;
+            yc[r] = jy[rj + k];
+            yn[r] = jy[rj + (k + 1 == n2 ? 0 : k + 1)];
+            zc[r] = jz[rj + k];
+            zn[r] = jz[rn + k];
+        }
+#pragma unroll
+        for (int r = 0; r < E; ++r) x[r] = (yn[r] - yc[r]) * inv_dz - (zn[r] - zc[r]) * inv_dy;
     }
+    template <int E>
+    __device__ void done(int, int, int, int, int) const {}
 };
 
 struct SinkMember {
