@@ -152,6 +152,7 @@ struct SinkEnv {
     double *inc;
     size_t vol, nn;
     int n1, n2, e;
+    __device__ void prep(int) {}
     __device__ void begin(int) {}
     __device__ void operator()(int, int which, int j, int k, double v) const {
         const size_t t = (size_t)j * n2 + k;

@@ -28,6 +28,52 @@ __device__ __forceinline__ bool solver_skip(const Ctl *ctl, int skip_mode) {
     }
     return ctl_skip_b(ctl);
 }
+// The same in two halves: the flag is loaded at kernel start, next to the data
+// loads, and acted on when they arrive, so that a launch does not begin with a
+// round trip to memory of its own.  (Loads are safe whatever the flag says.)
+__device__ __forceinline__ int solver_skip_flag(const Ctl *ctl, int skip_mode) {
+    if (!ctl || skip_mode == 0) return 0;
+    return skip_mode == 1 ? ctl->stop_acc : ctl->stop_now;
+}
+__device__ __forceinline__ bool solver_skip_act(const Ctl *ctl, int skip_mode, int flag) {
+    if (flag != 0 && skip_mode == 1) ctl_latch(const_cast<Ctl *>(ctl));
+    return flag != 0;
+}
+// Keeps the computation of x ahead of what follows (the compiler would move
+// loads used only behind a branch below it).
+__device__ __forceinline__ void keep_here(double &x) { asm volatile("" : "+v"(x)); }
+template <int E>
+__device__ __forceinline__ void keep_here(double2 (&v)[E]) {
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        keep_here(v[r].x);
+        keep_here(v[r].y);
+    }
+}
+
+// Sum over the wavefront, the same value in every lane: DPP moves inside each
+// 16-lane row (lane ^ 1, lane ^ 2, half-row mirror, row mirror), then the four
+// rows by readlane.  Every lane of the wavefront must call it.
+template <int CTRL>
+__device__ __forceinline__ double dpp_row_d(double x) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffLL), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+__device__ __forceinline__ double readlane_d(double x, int lane) {
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum(double x) {
+    x += dpp_row_d<0xB1>(x);   // quad_perm(1, 0, 3, 2)
+    x += dpp_row_d<0x4E>(x);   // quad_perm(2, 3, 0, 1)
+    x += dpp_row_d<0x141>(x);  // row_half_mirror
+    x += dpp_row_d<0x140>(x);  // row_mirror
+    return (readlane_d(x, 0) + readlane_d(x, 16)) + (readlane_d(x, 32) + readlane_d(x, 48));
+}
 
 // A source hands out elements k0, k0 + dk, ... of row j (row), all loads before
 // the arithmetic, and is told when they have been read (done).
@@ -45,9 +91,13 @@ struct SrcPlain {
 
 // Real output v of the unnormalised c2r; the reference divides by n1 then n2
 // (src/System_3d.cpp:361).
+//
+// A sink is prepared (prep: loads of its own are issued) ahead of the transform
+// and begun (begin) after it, before it takes the outputs.
 struct SinkScaled {
     double *dst;
     int n1, n2;
+    __device__ void prep(int) {}
     __device__ void begin(int) {}
     __device__ void operator()(int, int, int j, int k, double v) const { dst[(size_t)j * n2 + k] = v / n1 / n2; }
 };
@@ -56,6 +106,7 @@ struct SinkScaled {
 struct SinkRaw {
     double *dst;
     int n2;
+    __device__ void prep(int) {}
     __device__ void begin(int) {}
     __device__ void operator()(int, int, int j, int k, double v) const { dst[(size_t)j * n2 + k] = v; }
 };
@@ -67,6 +118,7 @@ struct SinkBCheck {
     double thr;
     Ctl *ctl;
     int slice;
+    __device__ void prep(int) {}
     __device__ void begin(int) {}
     __device__ void operator()(int wk, int, int j, int k, double v) const {
         const double b = v / n1 / n2;
@@ -193,6 +245,7 @@ __global__ __launch_bounds__(kSolverThreads) void k_rows_inv(const double2 *spec
     const int which = blockIdx.y % nspec, wk = blockIdx.y / nspec;
     if (solver_skip(ctl ? ctl + wk : nullptr, skip_mode)) return;
     const double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
+    sink.prep(wk);
     sink.begin(wk);
     extern __shared__ double2 lds[];
     double2 *a = lds, *b = lds + (size_t)B * n2, *twl = lds + (size_t)2 * B * n2;

@@ -676,23 +676,27 @@ struct SinkPsiFinal {
     double b;
     size_t bstride;
     double scale;  // 1 / (n1 n2): the unnormalised c2r output times this (exact for 2^p sides)
-    // Every wavefront sums the partial sums itself (no block barrier); lane 0's
-    // result is broadcast, so every lane and every block uses the same value.
-    __device__ void begin(int wk) {
-        const double *bp = bpart + wk * bstride;
-        double s1 = 0.0, s2 = 0.0;
-        for (int i = threadIdx.x & 63; i < ncb; i += 64) {
-            s1 += bp[2 * i];
-            s2 += bp[2 * i + 1];
+    double s1, s2, g00;  // a lane's share of the two sums; G00
+    // Every wavefront sums the partial sums itself (no block barrier), in the same
+    // order, so every block uses the same mean.  The loads go out before the
+    // transform, four at a time; the sum over the lanes follows it.
+    __device__ void prep(int wk) {
+        const double2 *bp = reinterpret_cast<const double2 *>(bpart + wk * bstride);
+        s1 = s2 = 0.0;
+        for (int i0 = threadIdx.x & 63; i0 < ncb; i0 += 256) {
+            double2 t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[u] = bp[i0 + 64 * u < ncb ? i0 + 64 * u : ncb - 1];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                s1 += i0 + 64 * u < ncb ? t[u].x : 0.0;
+                s2 += i0 + 64 * u < ncb ? t[u].y : 0.0;
+            }
         }
-        for (int off = 32; off > 0; off >>= 1) {
-            s1 += __shfl_xor(s1, off);
-            s2 += __shfl_xor(s2, off);
-        }
-        s1 = __shfl(s1, 0);
-        s2 = __shfl(s2, 0);
-        const double g00 = bp[2 * ncb];
-        const double sraw = s1 + (double)n2 * g00 - s2;
+        g00 = bp[ncb].x;
+    }
+    __device__ void begin(int) {
+        const double sraw = wave_sum(s1) + (double)n2 * g00 - wave_sum(s2);
         b = sraw / n1 / n2 / (n1 + n2 - 1);
     }
     __device__ void operator()(int wk, int, int j, int k, double v) const {
@@ -710,6 +714,7 @@ struct SinkBPair {
     Ctl *ctl;
     int slot;
     double scale;  // 1 / (n1 n2)
+    __device__ void prep(int) {}
     __device__ void begin(int) {}
     __device__ void operator()(int wk, int which, int j, int k, double v) const {
         const double b = v * scale;
@@ -754,6 +759,7 @@ struct SinkMember {
     double *dst;
     int n1, n2;
     double scale;  // 1 / (n1 n2)
+    __device__ void prep(int) {}
     __device__ void begin(int) {}
     __device__ void operator()(int wk, int, int j, int k, double v) const {
         dst[(size_t)wk * n1 * n2 + (size_t)j * n2 + k] = v * scale;

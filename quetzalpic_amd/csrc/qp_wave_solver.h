@@ -44,11 +44,9 @@ struct WfCfg {
 // Sum of three values over a block of TB threads (every thread gets the sums).
 template <int TB>
 __device__ __forceinline__ void block_sum3(double &a, double &b, double &c) {
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off);
-        b += __shfl_xor(b, off);
-        c += __shfl_xor(c, off);
-    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    c = wave_sum(c);
     if constexpr (TB > 64) {
         __shared__ double part[3][TB / 64];
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -81,7 +79,8 @@ __device__ __forceinline__ void wrows_fwd_body(const Src &src, double2 *spec0, d
                                                double2 *twl) {
     using W = WfShape<N2, E, TB>;
     const int which = by % nspec, wk = by / nspec;
-    if (solver_skip(ctl ? ctl + wk : nullptr, skip_mode)) return;
+    if (ctl) ctl += wk;
+    const int skip = solver_skip_flag(ctl, skip_mode);
     double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
     const int tid = threadIdx.x;
     const int tt = tid / W::L, j = tid % W::L;
@@ -99,15 +98,16 @@ __device__ __forceinline__ void wrows_fwd_body(const Src &src, double2 *spec0, d
     if (rb < n1) {
         src.template row<E>(wk, which, ra, j, W::L, xa);
         src.template row<E>(wk, which, rb, j, W::L, xb);
-        src.template done<E>(wk, which, ra, j, W::L);
-        src.template done<E>(wk, which, rb, j, W::L);
     } else if (ra < n1) {
         src.template row<E>(wk, which, ra, j, W::L, xa);
-        src.template done<E>(wk, which, ra, j, W::L);
     }
     double2 v[E];
 #pragma unroll
     for (int r = 0; r < E; ++r) v[r] = make_double2(xa[r], xb[r]);
+    keep_here(v);
+    if (solver_skip_act(ctl, skip_mode, skip)) return;
+    if (ra < n1) src.template done<E>(wk, which, ra, j, W::L);
+    if (rb < n1) src.template done<E>(wk, which, rb, j, W::L);
     wave_fft<N2, E, -1>(v, sb0 + tt * W::PADN, sb1 + tt * W::PADN, tw, j);
     // Z in natural order to LDS (after the barrier no lane reads sb0 any more)
     double2 *zb = sb0;
@@ -160,7 +160,8 @@ __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int n
                                            double2 *twl) {
     using W = WfShape<N1, E, TB>;
     const int which = by % nspec, wk = by / nspec;
-    if (solver_skip(ctl ? ctl + wk : nullptr, skip_mode)) return;
+    if (ctl) ctl += wk;
+    const int skip = solver_skip_flag(ctl, skip_mode);
     double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
     if (bpart) bpart += wk * bstride;
     const int tid = threadIdx.x;
@@ -178,6 +179,8 @@ __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int n
         lm[r] = lam1[j + W::L * r];
     }
     const double l2 = valid ? lam2[l] : 0.0;
+    keep_here(v);
+    if (solver_skip_act(ctl, skip_mode, skip)) return;
     double2 *b0 = sb0 + tt * W::PADN, *b1 = sb1 + tt * W::PADN;
     wave_fft<N1, E, -1>(v, b0, b1, tw, j);
 #pragma unroll
@@ -190,14 +193,24 @@ __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int n
             v[m].y *= inv;
         }
     }
+    // The border-mean sums are formed here and reduced behind the last stores.
+    double s1 = 0.0, s2 = 0.0, g00 = 0.0;
     if (bpart) {
         const double wl = (l == 0 || 2 * l == n2) ? 1.0 : 2.0;
         double g = 0.0;
 #pragma unroll
         for (int m = 0; m < E; ++m) g += v[m].x;
-        double s1 = (valid && j == 0) ? wl * (double)N1 * v[0].x : 0.0;
-        double s2 = valid ? wl * g : 0.0;
-        double g00 = (l == 0) ? g : 0.0;
+        s1 = (valid && j == 0) ? wl * (double)N1 * v[0].x : 0.0;
+        s2 = valid ? wl * g : 0.0;
+        g00 = (l == 0) ? g : 0.0;
+    }
+    wave_fft<N1, E, +1>(v, b0, b1, tw, j);
+    if (valid) {
+        double2 *out = spec + (size_t)l * N1;
+#pragma unroll
+        for (int m = 0; m < E; ++m) out[j + W::L * m] = v[m];
+    }
+    if (bpart) {
         block_sum3<TB>(s1, s2, g00);
         if (tid == 0) {
             bpart[2 * bx] = s1;
@@ -205,11 +218,6 @@ __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int n
             if (bx == 0) bpart[2 * gx] = g00;
         }
     }
-    wave_fft<N1, E, +1>(v, b0, b1, tw, j);
-    if (!valid) return;
-    double2 *out = spec + (size_t)l * N1;
-#pragma unroll
-    for (int m = 0; m < E; ++m) out[j + W::L * m] = v[m];
 }
 
 template <int N1, int E, int TB>
@@ -233,9 +241,9 @@ __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const doubl
                                                double2 *twl) {
     using W = WfShape<N2, E, TB>;
     const int which = by % nspec, wk = by / nspec;
-    if (solver_skip(ctl ? ctl + wk : nullptr, skip_mode)) return;
+    if (ctl) ctl += wk;
+    const int skip = solver_skip_flag(ctl, skip_mode);
     const double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
-    sink.begin(wk);
     const int tid = threadIdx.x;
     const int tt = tid / W::L, j = tid % W::L;
     WfTw<N2, E, TB> tw;
@@ -260,23 +268,38 @@ __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const doubl
             sb1[(r2 >> 1) * W::PADN + (r2 & 1) * NHF + f] =
                 row < n1 ? spec[(size_t)f * n1 + row] : make_double2(0.0, 0.0);
         }
+        sink.prep(wk);
+        if (solver_skip_act(ctl, skip_mode, skip)) return;
         __syncthreads();
     }
     const double2 *st = sb1 + tt * W::PADN;
-    double2 v[E];
+    double2 v[E], u[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int k = j + W::L * r;
+        const int kk = k > N2 / 2 ? N2 - k : k;
+        if constexpr (staged) {
+            v[r] = st[kk];
+            u[r] = st[NHF + kk];
+        } else {
+            // rows beyond n1 read row n1 - 1 and go nowhere
+            v[r] = spec[(size_t)kk * n1 + (ra < n1 ? ra : n1 - 1)];
+            u[r] = spec[(size_t)kk * n1 + (rb < n1 ? rb : n1 - 1)];
+        }
+    }
+    if constexpr (!staged) {
+        sink.prep(wk);
+        keep_here(v);
+        keep_here(u);
+        if (solver_skip_act(ctl, skip_mode, skip)) return;
+    }
 #pragma unroll
     for (int r = 0; r < E; ++r) {
         const int k = j + W::L * r;
         const bool cj = k > N2 / 2;
         const int kk = cj ? N2 - k : k;
-        double2 X = make_double2(0.0, 0.0), Y = X;
-        if constexpr (staged) {
-            X = st[kk];
-            Y = st[NHF + kk];
-        } else {
-            if (ra < n1) X = spec[(size_t)kk * n1 + ra];
-            if (rb < n1) Y = spec[(size_t)kk * n1 + rb];
-        }
+        double2 X = v[r], Y = u[r];
+        if (rb >= n1) Y = make_double2(0.0, 0.0);
         if (cj) {
             X.y = -X.y;
             Y.y = -Y.y;
@@ -288,6 +311,7 @@ __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const doubl
         v[r] = make_double2(X.x - Y.y, X.y + Y.x);
     }
     wave_fft<N2, E, +1>(v, sb0 + tt * W::PADN, sb1 + tt * W::PADN, tw, j);
+    sink.begin(wk);
     if (ra >= n1) return;
 #pragma unroll
     for (int m = 0; m < E; ++m) {
