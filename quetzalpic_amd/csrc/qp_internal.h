@@ -83,7 +83,8 @@ struct Ctl {
     int stop_slice;
     int slice_of[2];   // mixed path: slice index for the even / odd slice step
     unsigned ovf;      // mixed path: particle blocks whose deposit window exceeded the LDS capacity
-    int pad[2];
+    int iter;          // mixed path: predictor-corrector iteration of the slice step (k_mx_B)
+    int stop_iter;     // mixed path: the iteration whose B solve tripped the stop rule
     double border[4];  // plain path: border mean of the last psi solve
 };
 

@@ -20,9 +20,14 @@
 //
 // The 35 particle sweeps of a reference slice (src/System_3d.cpp:328-619)
 // become 2K+1 launches: A (commit + advance + psi source deposit), then per
-// iteration B (gamma, predictor, half step, psi_middle source deposit) and
-// C (transverse current at the half step, gamma/px, jx deposits; chi in the
-// first iteration of a slice, rho in the last).
+// iteration B (gamma, predictor, half step, psi_middle source deposit, then
+// gamma/px of the new p* and the jx deposit; chi in the first iteration of a
+// slice, rho in the last) and C (transverse current at the half step).  The node
+// deposits sit in B because B holds their inputs: C then gathers psi_middle only
+// and reads 1/(1 + psi) (8 B) where it gathered psi and <a^2>, divided and read p
+// (16 B).  With the shared window (see k_mx_B) one iteration's B + C took 77 + 48 us
+// against 83 + 70 us at 1024^2 with 4.2 M particles, 23 + 16 against 26 + 22 us at
+// 512^2 with 1 M.
 #pragma once
 
 #include "qp_solver_kernels.h"
@@ -57,11 +62,19 @@ struct MxPart {
     double2 *p;    // p_y, p_z
     double *w;
     double2 *ps;   // p* (y, z)
+    double *iv;    // 1/(1 + psi) at the slice's position, from the first B to every C of a slice
+    int4 *wq;      // per particle block: the node window of its cells (origin j, k; rows,
+                   // columns), from A to the slice's B and C
     int np;
     int pstride;
     const int *npw;
 };
 
+// Window slot of a particle block (blocks of one member start at its own slots).
+template <int PT>
+__device__ __forceinline__ int mx_blk(const MxPart &P, int wk, int bx) {
+    return wk * (P.pstride / PT) + bx;
+}
 __device__ __forceinline__ int mx_np(const MxPart &P, int wk) { return P.npw ? P.npw[wk] : P.np; }
 
 // Slice-dependent inputs resolved on the device from the slice counter.
@@ -73,7 +86,10 @@ struct MxSliceIn {
     int slot;               // which ctl->slice_of[] entry holds this step's slice
 };
 
-__device__ __forceinline__ int mx_slice(const Ctl *c, const MxSliceIn &si) { return c->slice_of[si.slot]; }
+// (readfirstlane: the same in every lane, kept in a scalar register)
+__device__ __forceinline__ int mx_slice(const Ctl *c, const MxSliceIn &si) {
+    return __builtin_amdgcn_readfirstlane(c->slice_of[si.slot]);
+}
 // <a^2> plane of the block's member (go = member * nn; the 3D array and the
 // bunch sources exist for single wakes only).
 __device__ __forceinline__ const double *mx_asq(const Ctl *c, const MxSliceIn &si, size_t nn, size_t go) {
@@ -119,17 +135,14 @@ __device__ __forceinline__ void split_coord(double Y, int n, int &j, uint32_t &o
 // addition (the reference's y += l); fmod stays for anything further out.
 __device__ __forceinline__ double wrap_cells(double Y, int n) {
     const double dn = (double)n;
-    if (Y >= 0.0 && Y < dn) return Y;
-    if (Y >= dn && Y < 2.0 * dn) {
-        Y -= dn;
-    } else if (Y < 0.0 && Y >= -dn) {
-        Y += dn;
-    } else {
-        Y = fmod(Y, dn);
-        if (Y < 0) Y += dn;
+    // selects for the common cases, one branch for the rest (and NaN)
+    double r = Y >= dn ? Y - dn : Y;
+    r = Y < 0.0 ? Y + dn : r;
+    if (!(Y >= -dn && Y < 2.0 * dn)) {
+        r = fmod(Y, dn);
+        if (r < 0) r += dn;
     }
-    if (Y >= dn) Y = 0.0;
-    return Y;
+    return r >= dn ? 0.0 : r;
 }
 
 // Element i of a grid through a 32-bit byte offset from the (uniform) base:
@@ -324,8 +337,8 @@ __device__ __forceinline__ int wave_max(int v) {
 // rmin/rmax/cmin/cmax: this thread's relative node range (INT_MAX / INT_MIN
 // when the thread deposits nothing).  Relative indices come from rel_idx, so
 // they lie in [-n/2, n - n/2].
-// `sh` is 4*(blockDim/64)+2 ints of LDS.  The window is the same in every lane
-// (kept in scalar registers).
+// `sh` is 4*(blockDim/64) ints of LDS, not written again before a later barrier.
+// The window is the same in every lane (kept in scalar registers).
 template <int CAP>
 __device__ inline Win block_window(int rmin, int rmax, int cmin, int cmax, int jref, int kref, int n1, int n2,
                                    int *sh) {
@@ -348,7 +361,6 @@ __device__ inline Win block_window(int rmin, int rmax, int cmin, int cmax, int j
         c = min(c, sh[4 * i + 2]);
         d = max(d, sh[4 * i + 3]);
     }
-    __syncthreads();
     a = __builtin_amdgcn_readfirstlane(a);
     b = __builtin_amdgcn_readfirstlane(b);
     c = __builtin_amdgcn_readfirstlane(c);
@@ -373,10 +385,36 @@ __device__ inline Win block_window(int rmin, int rmax, int cmin, int cmax, int j
     return w;
 }
 
+// A window kept for a later launch of the same block, with `lo` rows and columns
+// more ahead of it and `hi` more behind it (each below the grid's sides).
+template <int CAP>
+__device__ __forceinline__ Win win_load(const int4 *t, int blk, int lo, int hi, int n1, int n2) {
+    const int4 d = t[blk];
+    Win w;
+    w.j0 = __builtin_amdgcn_readfirstlane(d.x) - lo;
+    w.k0 = __builtin_amdgcn_readfirstlane(d.y) - lo;
+    w.wj = __builtin_amdgcn_readfirstlane(d.z);
+    w.wk = __builtin_amdgcn_readfirstlane(d.w);
+    if (w.wj == 0) {  // a block without particles
+        w.j0 = w.k0 = 0;
+        w.lds = true;
+        return w;
+    }
+    if (w.j0 < 0) w.j0 += n1;
+    if (w.k0 < 0) w.k0 += n2;
+    w.wj += lo + hi;
+    w.wk += lo + hi;
+    w.lds = (w.wj <= n1 && w.wk <= n2 && w.wj * w.wk <= CAP);
+    return w;
+}
+__device__ __forceinline__ void win_store(int4 *t, int blk, const Win &w) {
+    if (threadIdx.x == 0) t[blk] = make_int4(w.j0, w.k0, w.wj, w.wk);
+}
+
 // Count a block that deposits but whose window exceeds its capacity (it falls back
 // to global atomics): one atomic per such block, none otherwise.
-__device__ __forceinline__ void win_note_overflow(const Win &w, Ctl *ctl) {
-    if (!w.lds && w.wj > 0 && threadIdx.x == 0) atomicAdd(&ctl->ovf, 1u);
+__device__ __forceinline__ void win_note_overflow(bool fits, Ctl *ctl) {
+    if (!fits && threadIdx.x == 0) atomicAdd(&ctl->ovf, 1u);
 }
 
 // Window slot of node (j, k) for a CIC stencil whose other nodes are (j + 1, k),

@@ -8,10 +8,12 @@
 //                 normalize_potential + clamp applied in the last pass (:355-365)
 //             per iteration k = 1..K:
 //               B  gamma (S4 for k = 1, else P6 recomputed from p, p*_{k-1}),
-//                  predictor P1, half step P2, psi_middle source deposit P3
+//                  predictor P1, half step P2, psi_middle source deposit P3,
+//                  gamma/px P6 and the rho/jx/chi deposits P7 (they need the new p*
+//                  and the fields B has gathered, not psi_middle)
 //               psi_middle solve (:459-469)
 //               C  half-step position recomputed from the same inputs, j_perp*
-//                  deposit P4, gamma/px P6, rho/jx/chi deposits P7
+//                  deposit P4
 //               B_y and B_z Helmholtz solves in one set of launches, sources
 //                  (P5, P8, P9) assembled in the row pass, stop rule in the
 //                  last pass (:529-580)
@@ -47,14 +49,14 @@ namespace qp {
 // ------------------------------------------------------------------ A phase
 // Commit and advance (src/System_3d.cpp:593-608), then deposit -n at the new
 // position into the psi source accumulator (:349-353).  The grid part
-// evaluates the laser plane of slice i and, for S-phase slices, initialises
-// rho/jx/chi (:381-388).
+// evaluates the laser plane of slice i and initialises the slice's rho, chi and
+// first jx (:381-388).  The block's cell window is kept for the B phase.
 // Batches: blockIdx.y is the member; its grids sit at + member * nn, its
 // particles at + member * pstride, its control block at ctl + member.
 template <int PT, int CAP>
 __device__ __forceinline__ void mx_A(MxPart P, MxGeom g, MxSliceIn si, const double *psim, double *src_acc,
                                               double *asq2, const LaserGauss *Ls, int laser, double *rho, double *jx,
-                                              double *chi, int init_rho, int advance, Ctl *ctl, int bx, int wk, int gx) {
+                                              double *chi, int advance, Ctl *ctl, int bx, int wk, int gx) {
     // The particle's state is loaded before the control block is checked: the
     // index stays inside the member's allocation (pstride is a whole number of
     // blocks), so these loads share a round trip with the control block's.
@@ -114,7 +116,8 @@ __device__ __forceinline__ void mx_A(MxPart P, MxGeom g, MxSliceIn si, const dou
     int rmin = INT_MAX, rmax = INT_MIN, cmin = INT_MAX, cmax = INT_MIN;
     if (valid) range_add(q.j, q.k, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
     const Win win = block_window<CAP>(rmin, rmax, cmin, cmax, jref, kref, n1, n2, sh);
-    win_note_overflow(win, ctl);
+    win_store(P.wq, mx_blk<PT>(P, wk, bx), win);
+    win_note_overflow(win.lds, ctl);
     win_zero<CAP>(lds, 1, win);
     __syncthreads();
     {
@@ -125,38 +128,33 @@ __device__ __forceinline__ void mx_A(MxPart P, MxGeom g, MxSliceIn si, const dou
         double a[4];
         cic_w(-w, yf, zf, a);
         bool act = valid;
-        quad_fold<4>(j1 * n2 + k1, act, a);
+        quad_fold<4>((j1 << 16) | k1, act, a);
         if (act) dep4w(lds, win, src_acc, n1, n2, j1, j2, k1, k2, a[0], a[1], a[2], a[3]);
     }
     __syncthreads();
     double *gl[1] = {src_acc};
     win_flush<CAP>(lds, gl, 1, win, n1, n2);
-    // The slice's laser plane and the S-phase initial rho / jx / chi last, so that
-    // these stores do not queue ahead of the particle loads (nothing in this kernel
-    // reads them).
-    if (laser || init_rho) {
-        const double *rb = si.rho_b3 ? si.rho_b3 + (size_t)slice * si.bstride : nullptr;
-        const double *jb = si.jx_b3 ? si.jx_b3 + (size_t)slice * si.bstride : nullptr;
-        for (size_t t = (size_t)bx * PT + threadIdx.x; t < nn; t += (size_t)gx * PT) {
-            if (laser) {
-                const int j = (int)(t / n2), k = (int)(t % n2);
-                const double x = slice * g.dx, y = j * g.d1, z = k * g.d2;
-                asq2[t] = L.amp * exp(-(x - L.x0) * (x - L.x0) / L.wx / L.wx - (y - L.y0) * (y - L.y0) / L.wy / L.wy -
-                                      (z - L.z0) * (z - L.z0) / L.wz / L.wz);
-            }
-            if (init_rho) {
-                rho[t] = rb ? rb[t] : 0.0;
-                jx[t] = jb ? jb[t] : 0.0;
-                chi[t] = 0.0;
-            }
+    // The slice's laser plane and initial rho / jx / chi last, so that these stores
+    // do not queue ahead of the particle loads (nothing in this kernel reads them).
+    const double *rb = si.rho_b3 ? si.rho_b3 + (size_t)slice * si.bstride : nullptr;
+    const double *jb = si.jx_b3 ? si.jx_b3 + (size_t)slice * si.bstride : nullptr;
+    for (size_t t = (size_t)bx * PT + threadIdx.x; t < nn; t += (size_t)gx * PT) {
+        if (laser) {
+            const int j = (int)(t / n2), k = (int)(t % n2);
+            const double x = slice * g.dx, y = j * g.d1, z = k * g.d2;
+            asq2[t] = L.amp * exp(-(x - L.x0) * (x - L.x0) / L.wx / L.wx - (y - L.y0) * (y - L.y0) / L.wy / L.wy -
+                                  (z - L.z0) * (z - L.z0) / L.wz / L.wz);
         }
+        rho[t] = rb ? rb[t] : 0.0;
+        jx[t] = jb ? jb[t] : 0.0;
+        chi[t] = 0.0;
     }
 }
 template <int PT, int CAP>
 __global__ __launch_bounds__(PT) void k_mx_A(MxPart P, MxGeom g, MxSliceIn si, const double *psim, double *src_acc,
                                               double *asq2, const LaserGauss *Ls, int laser, double *rho, double *jx,
-                                              double *chi, int init_rho, int advance, Ctl *ctl) {
-    mx_A<PT, CAP>(P, g, si, psim, src_acc, asq2, Ls, laser, rho, jx, chi, init_rho, advance, ctl, blockIdx.x, blockIdx.y,
+                                              double *chi, int advance, Ctl *ctl) {
+    mx_A<PT, CAP>(P, g, si, psim, src_acc, asq2, Ls, laser, rho, jx, chi, advance, ctl, blockIdx.x, blockIdx.y,
          gridDim.x);
 }
 
@@ -166,15 +164,37 @@ __device__ __forceinline__ double gamma_of(double p2, double a, double ps, doubl
     return 0.5 * (1 + p2 + a + (1 + ps) * (1 + ps)) * inv1ps;
 }
 
-template <int PT, int CAP>
+// One template per slice role: RHO in the last iteration of a slice, CHI in the
+// first.  Within a slice only jx feeds the next field solve; rho and chi are read
+// only by the slice's output.  rho depends on the iteration's p*, so only the
+// last iteration deposits it.  chi = -n/(1+psi) at the slice's old positions is
+// the same in every iteration (:526), so the first deposits it; a pass that stops
+// in a later iteration then still has it.
+// Waves per SIMD the B phase is bounded to, where the LDS of as many blocks fits a CU
+// (160 KB).  Unbounded the compiler takes 88 VGPRs (5 waves: 109 us at 1024^2 against
+// 89 us).  The first iteration fits 64 VGPRs (8 waves) without scratch, the others,
+// which also hold the previous p*, 72 (7 waves).
+constexpr int b_lds(int CAP, bool RHO, bool CHI) {  // doubles: the staged grids or the deposit windows
+    return std::max(4 * kGwCap, (2 + RHO + CHI) * CAP);
+}
+constexpr int b_waves(int PT, int CAP, bool RHO, bool CHI) {
+    return std::min(CHI ? 8 : 7, 163840 / (8 * b_lds(CAP, RHO, CHI) + 256) * PT / 256);
+}
+// One window serves the launch: rows and columns -1 .. +2 around the block's cells,
+// from the cell window that the A phase kept.  It holds every node of the gathers and
+// of the deposits at the cells, and those of the half-step deposit unless the half step
+// leaves its cell by more than one (such a particle deposits with global atomics).  So
+// the launch starts with the window's grid loads beside the particle loads, and finds
+// no window of its own: no reductions over the block, two barriers fewer, one flush.
+template <int PT, int CAP, bool RHO, bool CHI>
 __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const double *psi, const double *by,
                                               const double *bz, double *src_acc, double *rho, double *jx,
-                                              double *chi, double *jyn, double *jzn, int first_iter, int init_rho,
+                                              double *jx_next, double *chi, double *jyn, double *jzn, int it,
                                               Ctl *ctl, int bx, int wk, int gx) {
+    constexpr int G = 1 + (RHO ? 1 : 0) + (CHI ? 1 : 0);  // node grids
+    __shared__ double lds[b_lds(CAP, RHO, CHI)];  // the staged grids, then (behind a barrier) the deposit windows
     ctl += wk;
-    MX_SKIP(ctl);
-    __shared__ double lds[CAP];
-    __shared__ int sh[4 * (PT / 64) + 2];
+    const int stop = ctl->stop_acc;
     const int n1 = g.n1, n2 = g.n2;
     const size_t nn = (size_t)n1 * n2, go = (size_t)wk * nn;
     psi += go;
@@ -186,56 +206,39 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
     chi += go;
     jyn += go;
     jzn += go;
-    const int slice = mx_slice(ctl, si);
-    const double *asq = mx_asq(ctl, si, nn, go);
     const int lp = bx * PT + threadIdx.x;
     const bool valid = lp < mx_np(P, wk);
     const unsigned p = (unsigned)(wk * P.pstride + lp);
-    Pos q{0, 0, 0.0, 0.0}, qm{0, 0, 0.0, 0.0};
-    double w = 0.0;
-    double2 pp = make_double2(0.0, 0.0), pst = pp;
-    if (valid) {
-        q = load_pos(P, p);
-        w = P.w[p];
-        pp = P.p[p];
-        pst = P.ps[p];  // P6 of the previous iteration (:503-505); unused in the first
+    Pos qm{0, 0, 0.0, 0.0};
+    double vjx = 0.0, vrho = 0.0, vchi = 0.0;
+    // loaded with the stop flag (the index stays inside the member's allocation)
+    const Pos q = load_pos(P, p);
+    const double w = P.w[p];
+    const double2 pp = P.p[p];
+    double2 pst = make_double2(0.0, 0.0);
+    if (!CHI) pst = P.ps[p];  // P6 of the previous iteration (:503-505)
+    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 1, 1, n1, n2);
+    if (stop) {
+        ctl_latch(ctl);
+        return;
     }
-    // Gather window: rows and columns -1 .. +2 around the block's cells hold every
-    // node of the value + gradient stencils and of the staggered B stencils.
-    __shared__ double gw[4 * kGwCap];
-    Win gwn;
-    {
-        if (threadIdx.x == 0) {
-            sh[4 * (PT / 64)] = q.j;
-            sh[4 * (PT / 64) + 1] = q.k;
-        }
-        __syncthreads();
-        const int jref = sh[4 * (PT / 64)], kref = sh[4 * (PT / 64) + 1];
-        int rmin = INT_MAX, rmax = INT_MIN, cmin = INT_MAX, cmax = INT_MIN;
-        if (valid) {
-            const int r = rel_idx(q.j, jref, n1), c = rel_idx(q.k, kref, n2);
-            rmin = r - 1;
-            rmax = r + 2;
-            cmin = c - 1;
-            cmax = c + 2;
-        }
-        gwn = block_window<kGwCap>(rmin, rmax, cmin, cmax, jref, kref, n1, n2, sh);
-        if (gwn.lds) {
-            const double *src[4] = {psi, asq, by, bz};
-            gwin_load<4>(gw, kGwCap, src, gwn, n1, n2);
-        }
-        __syncthreads();
+    const double *asq = mx_asq(ctl, si, nn, go);
+    const bool staged = win.lds && win.wj * win.wk <= kGwCap;
+    if (staged) {
+        const double *src[4] = {psi, asq, by, bz};
+        gwin_load<4>(lds, kGwCap, src, win, n1, n2);
     }
+    __syncthreads();
+    int r = 0, c = 0;  // the particle's cell in the window
+    gwin_rc(win, q.j, q.k, n1, n2, r, c);
     if (valid) {
         ValGrad ga, gp;
         double byp, bzp;
-        if (gwn.lds) {
-            int r, c;
-            gwin_rc(gwn, q.j, q.k, n1, n2, r, c);
-            gp = lg_vg(gw, gwn.wk, r, c, q.fy, q.fz, g.inv_d1, g.inv_d2);
-            ga = lg_vg(gw + kGwCap, gwn.wk, r, c, q.fy, q.fz, g.inv_d1, g.inv_d2);
-            byp = lg_hz(gw + 2 * kGwCap, gwn.wk, r, c, q.fy, q.fz);
-            bzp = lg_hy(gw + 3 * kGwCap, gwn.wk, r, c, q.fy, q.fz);
+        if (staged) {
+            gp = lg_vg(lds, win.wk, r, c, q.fy, q.fz, g.inv_d1, g.inv_d2);
+            ga = lg_vg(lds + kGwCap, win.wk, r, c, q.fy, q.fz, g.inv_d1, g.inv_d2);
+            byp = lg_hz(lds + 2 * kGwCap, win.wk, r, c, q.fy, q.fz);
+            bzp = lg_hy(lds + 3 * kGwCap, win.wk, r, c, q.fy, q.fz);
         } else {
             ga = mx_gather_vg(asq, q, n1, n2, g.inv_d1, g.inv_d2);
             gp = mx_gather_vg(psi, q, n1, n2, g.inv_d1, g.inv_d2);
@@ -247,8 +250,7 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
         const double inv1ps = 1.0 / (1 + ps);  // the FP64 1/(1+psi) factor
         const double pys = pst.x, pzs = pst.y;
         // S4 (:373-374) in the first iteration, the half-step momentum after it
-        const double p2 = first_iter ? py * py + pz * pz
-                                     : 0.25 * (py + pys) * (py + pys) + 0.25 * (pz + pzs) * (pz + pzs);
+        const double p2 = CHI ? py * py + pz * pz : 0.25 * (py + pys) * (py + pys) + 0.25 * (pz + pzs) * (pz + pzs);
         const double gm = gamma_of(p2, a, ps, inv1ps);
         const double day = ga.dy, daz = ga.dz, dpy = gp.dy, dpz = gp.dz;
         const double dx = g.dx;
@@ -260,23 +262,32 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
         pzn += s * gm * dpz;
         pzn += dx * byp;
         P.ps[p] = make_double2(pyn, pzn);
+        if (CHI) P.iv[p] = inv1ps;
         // P2 (:439-442)
         double Ym = (q.j + q.fy) + (0.5 * s * pyn) * g.inv_d1;
         double Zm = (q.k + q.fz) + (0.5 * s * pzn) * g.inv_d2;
         qm = pos_from_cells(wrap_cells(Ym, n1), wrap_cells(Zm, n2), n1, n2);
+        // P6 (:501-506), P7 (:523-526) with vx = px/gamma and 1/(1-vx) = gamma/(gamma-px) =
+        // gamma/(1+psi) (gamma - px = 1 + psi exactly, from the two closed forms): n vx/(1-vx) =
+        // n px/(1+psi), n/(1-vx) = n gamma/(1+psi), -n/((1-vx) gamma) = -n/(1+psi).
+        // No divisions, and no cancellation in gamma - px near psi -> -1.
+        const double h2 = 0.25 * (py + pyn) * (py + pyn) + 0.25 * (pz + pzn) * (pz + pzn);
+        const double px = 0.5 * (1 + h2 + a - (1 + ps) * (1 + ps)) * inv1ps;
+        vjx = w * px * inv1ps;
+        if (RHO) vrho = w * gamma_of(h2, a, ps, inv1ps) * inv1ps;
+        if (CHI) vchi = -w * inv1ps;
     }
-    if (threadIdx.x == 0) {
-        sh[4 * (PT / 64)] = qm.j;
-        sh[4 * (PT / 64) + 1] = qm.k;
+    __syncthreads();  // the gathers from LDS are done
+    win_note_overflow(win.lds, ctl);
+    win_zero<CAP>(lds, 1 + G, win);
+    __syncthreads();
+    double *gl[4] = {src_acc};  // deposited grids in window order
+    {
+        int ig = 1;
+        if (RHO) gl[ig++] = rho;
+        gl[ig++] = jx;
+        if (CHI) gl[ig] = chi;
     }
-    __syncthreads();
-    const int jref = sh[4 * (PT / 64)], kref = sh[4 * (PT / 64) + 1];
-    int rmin = INT_MAX, rmax = INT_MIN, cmin = INT_MAX, cmax = INT_MIN;
-    if (valid) range_add(qm.j, qm.k, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
-    const Win win = block_window<CAP>(rmin, rmax, cmin, cmax, jref, kref, n1, n2, sh);
-    win_note_overflow(win, ctl);
-    win_zero<CAP>(lds, 1, win);
-    __syncthreads();
     {  // P3 (:453-457)
         int j1, j2, k1, k2;
         double yf, zf;
@@ -285,81 +296,82 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
         double a[4];
         cic_w(-w, yf, zf, a);
         bool act = valid;
-        quad_fold<4>(j1 * n2 + k1, act, a);
+        quad_fold<4>((j1 << 16) | k1, act, a);
         if (act) dep4w(lds, win, src_acc, n1, n2, j1, j2, k1, k2, a[0], a[1], a[2], a[3]);
     }
-    __syncthreads();
-    double *gl[1] = {src_acc};
-    win_flush<CAP>(lds, gl, 1, win, n1, n2);
-    // Last, so that these stores do not queue ahead of the particle loads (nothing
-    // in this kernel reads the grids).
-    {  // jx = jx_bunch(i), jy* = jz* = 0 before the C phase (:473-478, :511-518); rho =
-       // rho_bunch(i) before the C phase that deposits rho (the last), chi = 0 before the
-       // one that deposits chi (the first)
-        const double *rb = si.rho_b3 ? si.rho_b3 + (size_t)slice * si.bstride : nullptr;
-        const double *jb = si.jx_b3 ? si.jx_b3 + (size_t)slice * si.bstride : nullptr;
-        for (size_t t = (size_t)bx * PT + threadIdx.x; t < nn; t += (size_t)gx * PT) {
-            if (init_rho) rho[t] = rb ? rb[t] : 0.0;
-            jx[t] = jb ? jb[t] : 0.0;
-            if (first_iter) chi[t] = 0.0;
-            jyn[t] = 0.0;
-            jzn[t] = 0.0;
-        }
+    {  // P7
+        int j1, j2, k1, k2;
+        double yf, zf;
+        ax_node(q.j, q.fy, n1, j1, j2, yf);
+        ax_node(q.k, q.fz, n2, k1, k2, zf);
+        double a[4 * G];
+        int ig = 0;
+        if (RHO) cic_w(vrho, yf, zf, a + 4 * ig++);
+        cic_w(vjx, yf, zf, a + 4 * ig++);
+        if (CHI) cic_w(vchi, yf, zf, a + 4 * ig);
+        // the quad fold also pays in VALU-bound batches: without it the same-address
+        // LDS conflicts cost more (256^2 x 10 members: 61.4 us folded, 86.8 us not)
+        bool act = valid;
+        quad_fold<4 * G>((j1 << 16) | k1, act, a);
+        if (act) dep4w_multi<G, CAP>(lds + CAP, win, gl + 1, n1, n2, j1, j2, k1, k2, a);
     }
+    __syncthreads();
+    win_flush<CAP>(lds, gl, 1 + G, win, n1, n2);
+    // Last, so that these stores do not queue ahead of the particle loads (nothing
+    // in this kernel reads the grids): jy* = jz* = 0 before the C phase (:473-478) and
+    // jx = jx_bunch(i) before the next iteration deposits (:511-518)
+    const double *jb = si.jx_b3 ? si.jx_b3 + (size_t)mx_slice(ctl, si) * si.bstride : nullptr;
+    if (jx_next) jx_next += go;
+    for (size_t t = (size_t)bx * PT + threadIdx.x; t < nn; t += (size_t)gx * PT) {
+        if (jx_next) jx_next[t] = jb ? jb[t] : 0.0;
+        jyn[t] = 0.0;
+        jzn[t] = 0.0;
+    }
+    if (bx == 0 && threadIdx.x == 0) ctl->iter = it;
 }
-template <int PT, int CAP>
-__global__ __launch_bounds__(PT) void k_mx_B(MxPart P, MxGeom g, MxSliceIn si, const double *psi, const double *by,
+template <int PT, int CAP, bool RHO, bool CHI>
+__global__ __launch_bounds__(PT, b_waves(PT, CAP, RHO, CHI)) void k_mx_B(MxPart P, MxGeom g, MxSliceIn si, const double *psi, const double *by,
                                               const double *bz, double *src_acc, double *rho, double *jx,
-                                              double *chi, double *jyn, double *jzn, int first_iter, int init_rho,
+                                              double *jx_next, double *chi, double *jyn, double *jzn, int it,
                                               Ctl *ctl) {
-    mx_B<PT, CAP>(P, g, si, psi, by, bz, src_acc, rho, jx, chi, jyn, jzn, first_iter, init_rho, ctl, blockIdx.x,
+    mx_B<PT, CAP, RHO, CHI>(P, g, si, psi, by, bz, src_acc, rho, jx, jx_next, chi, jyn, jzn, it, ctl, blockIdx.x,
          blockIdx.y, gridDim.x);
 }
 
 // ------------------------------------------------------------------ C phase
-// Grids jy*, jz*, jx, and rho (RHO) and chi (CHI).  Within a slice only jx and
-// j* feed the next field solve; rho and chi are read only by the slice's
-// output.  rho depends on the iteration's p*, so only the last iteration
-// deposits it.  chi = -n/(1+psi) at the slice's old positions is the same in
-// every iteration (:526), so the first iteration deposits it.  A pass that
-// stops in a later iteration then still has it, and no iteration repeats it.
-// Second launch bound (waves per SIMD): C fits 80 VGPRs at 6 waves without
-// spills (5 otherwise), which hides more of its gather -> deposit -> flush chain
-// in batches (256^2 x 10 members: 69.8 -> 65.9 us).  The same bound on B
-// (56 VGPRs, 8 waves) made it slower (77.9 -> 83.2 us) and is not used.
-template <int PT, int CAP, bool RHO, bool CHI>
-__device__ __forceinline__ void mx_C(MxPart P, MxGeom g, MxSliceIn si, const double *psi,
-                                              const double *psim, double *rho, double *jx, double *chi,
-                                              double *jyn, double *jzn, Ctl *ctl, double *lds, int bx, int wk) {
-    constexpr int G = 1 + (RHO ? 1 : 0) + (CHI ? 1 : 0);  // node grids
+// jy*, jz* at the half-step positions.  The deposit window is the block's cell window
+// with the row and column each side that a half step reaches, and one more ahead (the
+// half-cell stencils start at cell or cell - 1).
+template <int PT, int CAP>
+__device__ __forceinline__ void mx_C(MxPart P, MxGeom g, const double *psim, double *jyn, double *jzn, Ctl *ctl, int bx,
+                                     int wk) {
+    __shared__ double lds[2 * CAP];
     ctl += wk;
-    MX_SKIP(ctl);
-    __shared__ int sh[4 * (PT / 64) + 2];
+    const int stop = ctl->stop_acc;
     const int n1 = g.n1, n2 = g.n2;
-    const size_t nn = (size_t)n1 * n2, go = (size_t)wk * nn;
-    psi += go;
+    const size_t go = (size_t)wk * n1 * n2;
     psim += go;
-    rho += go;
-    jx += go;
-    chi += go;
     jyn += go;
     jzn += go;
-    const double *asq = mx_asq(ctl, si, nn, go);
     const int lp = bx * PT + threadIdx.x;
     const bool valid = lp < mx_np(P, wk);
     const unsigned p = (unsigned)(wk * P.pstride + lp);
-    Pos q{0, 0, 0.0, 0.0}, qm{0, 0, 0.0, 0.0};
-    double vjy = 0, vjz = 0, vjx = 0, vrho = 0, vchi = 0;
+    // loaded with the stop flag (the index stays inside the member's allocation)
+    const Pos q = load_pos(P, p);
+    Pos qm{0, 0, 0.0, 0.0};
+    double vjy = 0, vjz = 0;
+    const double w = P.w[p], iv = P.iv[p];
+    const double2 pst = P.ps[p];
+    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 2, 1, n1, n2);
+    if (stop) {
+        ctl_latch(ctl);
+        return;
+    }
+    win_note_overflow(win.lds, ctl);
+    win_zero<CAP>(lds, 2, win);
     if (valid) {
-        q = load_pos(P, p);
-        const double w = P.w[p];
-        const double2 pp = P.p[p];
-        const double2 pst = P.ps[p];
-        const double py = pp.x, pz = pp.y;
         const double pys = pst.x, pzs = pst.y;
-        const double ps = mx_gather(psi, q, n1, n2);
-        const double inv1ps = 1.0 / (1 + ps);
-        const double s = g.dx * inv1ps;
+        const double s = g.dx * iv;
         double Ym = (q.j + q.fy) + (0.5 * s * pys) * g.inv_d1;
         double Zm = (q.k + q.fz) + (0.5 * s * pzs) * g.inv_d2;
         qm = pos_from_cells(wrap_cells(Ym, n1), wrap_cells(Zm, n2), n1, n2);
@@ -367,77 +379,29 @@ __device__ __forceinline__ void mx_C(MxPart P, MxGeom g, MxSliceIn si, const dou
         const double wm = w / (1 + psm);
         vjy = wm * pys;
         vjz = wm * pzs;
-        const double a = mx_gather(asq, q, n1, n2);  // P6 (:501-506)
-        const double p2 = 0.25 * (py + pys) * (py + pys) + 0.25 * (pz + pzs) * (pz + pzs);
-        const double px = 0.5 * (1 + p2 + a - (1 + ps) * (1 + ps)) * inv1ps;
-        // P7 (:523-526) with vx = px/gamma and 1/(1-vx) = gamma/(gamma-px) = gamma/(1+psi)
-        // (gamma - px = 1 + psi exactly, from the two closed forms): n vx/(1-vx) =
-        // n px/(1+psi), n/(1-vx) = n gamma/(1+psi), -n/((1-vx) gamma) = -n/(1+psi).
-        // No divisions, and no cancellation in gamma - px near psi -> -1.
-        vjx = w * px * inv1ps;
-        if (RHO) vrho = w * gamma_of(p2, a, ps, inv1ps) * inv1ps;
-        if (CHI) vchi = -w * inv1ps;
-    }
-    if (threadIdx.x == 0) {
-        sh[4 * (PT / 64)] = q.j;
-        sh[4 * (PT / 64) + 1] = q.k;
     }
     __syncthreads();
-    const int jref = sh[4 * (PT / 64)], kref = sh[4 * (PT / 64) + 1];
-    int ya1, ya2, za1, za2, yb1, yb2, zb1, zb2, yc1, yc2, zc1, zc2;
-    double yaf, zaf, ybf, zbf, ycf, zcf;
+    int ya1, ya2, za1, za2, yb1, yb2, zb1, zb2;
+    double yaf, zaf, ybf, zbf;
     ax_half(qm.j, qm.fy, n1, ya1, ya2, yaf);  // jy* on the (dy/2, 0) grid
     ax_node(qm.k, qm.fz, n2, za1, za2, zaf);
     ax_node(qm.j, qm.fy, n1, yb1, yb2, ybf);  // jz* on the (0, dz/2) grid
     ax_half(qm.k, qm.fz, n2, zb1, zb2, zbf);
-    ax_node(q.j, q.fy, n1, yc1, yc2, ycf);    // jx, rho, chi on the nodes
-    ax_node(q.k, q.fz, n2, zc1, zc2, zcf);
-    int rmin = INT_MAX, rmax = INT_MIN, cmin = INT_MAX, cmax = INT_MIN;
-    if (valid) {
-        range_add(ya1, za1, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
-        range_add(yb1, zb1, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
-        range_add(yc1, zc1, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
-    }
-    const Win win = block_window<CAP>(rmin, rmax, cmin, cmax, jref, kref, n1, n2, sh);
-    win_note_overflow(win, ctl);
-    win_zero<CAP>(lds, 2 + G, win);
+    double aa[4], ab[4];
+    cic_w(vjy, yaf, zaf, aa);
+    cic_w(vjz, ybf, zbf, ab);
+    bool fa = valid, fb = valid;
+    quad_fold<4>((ya1 << 16) | za1, fa, aa);
+    quad_fold<4>((yb1 << 16) | zb1, fb, ab);
+    if (fa) dep4w(lds, win, jyn, n1, n2, ya1, ya2, za1, za2, aa[0], aa[1], aa[2], aa[3]);
+    if (fb) dep4w(lds + CAP, win, jzn, n1, n2, yb1, yb2, zb1, zb2, ab[0], ab[1], ab[2], ab[3]);
     __syncthreads();
-    double *gc[3];  // node grids in deposit order
-    {
-        int ig = 0;
-        if (RHO) gc[ig++] = rho;
-        gc[ig++] = jx;
-        if (CHI) gc[ig] = chi;
-    }
-    {
-        double aa[4], ab[4], ac[4 * G];
-        cic_w(vjy, yaf, zaf, aa);
-        cic_w(vjz, ybf, zbf, ab);
-        int ig = 0;
-        if (RHO) cic_w(vrho, ycf, zcf, ac + 4 * ig++);
-        cic_w(vjx, ycf, zcf, ac + 4 * ig++);
-        if (CHI) cic_w(vchi, ycf, zcf, ac + 4 * ig);
-        // the quad fold also pays in VALU-bound batches: without it the same-address
-        // LDS conflicts cost more (256^2 x 10 members: 61.4 us folded, 86.8 us not)
-        bool fa = valid, fb = valid, fc = valid;
-        quad_fold<4>(ya1 * n2 + za1, fa, aa);
-        quad_fold<4>(yb1 * n2 + zb1, fb, ab);
-        quad_fold<4 * G>(yc1 * n2 + zc1, fc, ac);
-        if (fa) dep4w(lds, win, jyn, n1, n2, ya1, ya2, za1, za2, aa[0], aa[1], aa[2], aa[3]);
-        if (fb) dep4w(lds + CAP, win, jzn, n1, n2, yb1, yb2, zb1, zb2, ab[0], ab[1], ab[2], ab[3]);
-        if (fc) dep4w_multi<G, CAP>(lds + 2 * CAP, win, gc, n1, n2, yc1, yc2, zc1, zc2, ac);
-    }
-    __syncthreads();
-    double *gl[2 + G] = {jyn, jzn};
-    for (int i = 0; i < G; ++i) gl[2 + i] = gc[i];
-    win_flush<CAP>(lds, gl, 2 + G, win, n1, n2);
+    double *gl[2] = {jyn, jzn};
+    win_flush<CAP>(lds, gl, 2, win, n1, n2);
 }
-template <int PT, int CAP, bool RHO, bool CHI>
-__global__ __launch_bounds__(PT, 6) void k_mx_C(MxPart P, MxGeom g, MxSliceIn si, const double *psi,
-                                              const double *psim, double *rho, double *jx, double *chi,
-                                              double *jyn, double *jzn, Ctl *ctl) {
-    extern __shared__ double ldsd[];
-    mx_C<PT, CAP, RHO, CHI>(P, g, si, psi, psim, rho, jx, chi, jyn, jzn, ctl, ldsd, blockIdx.x, blockIdx.y);
+template <int PT, int CAP>
+__global__ __launch_bounds__(PT) void k_mx_C(MxPart P, MxGeom g, const double *psim, double *jyn, double *jzn, Ctl *ctl) {
+    mx_C<PT, CAP>(P, g, psim, jyn, jzn, ctl, blockIdx.x, blockIdx.y);
 }
 
 // -------------------------------------------------- S phase (slice 0, K = 0)
@@ -488,7 +452,7 @@ __device__ __forceinline__ void mx_S(MxPart P, MxGeom g, MxSliceIn si, const dou
     int rmin = INT_MAX, rmax = INT_MIN, cmin = INT_MAX, cmax = INT_MIN;
     if (valid) range_add(y1, z1, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
     const Win win = block_window<CAP>(rmin, rmax, cmin, cmax, jref, kref, n1, n2, sh);
-    win_note_overflow(win, ctl);
+    win_note_overflow(win.lds, ctl);
     win_zero<CAP>(lds, 3, win);
     __syncthreads();
     {
@@ -497,7 +461,7 @@ __device__ __forceinline__ void mx_S(MxPart P, MxGeom g, MxSliceIn si, const dou
         cic_w(vjx, yf, zf, ac + 4);
         cic_w(vchi, yf, zf, ac + 8);
         bool act = valid;
-        quad_fold<12>(y1 * n2 + z1, act, ac);
+        quad_fold<12>((y1 << 16) | z1, act, ac);
         if (act) {
             double *const gc[3] = {rho, jx, chi};
             dep4w_multi<3, CAP>(lds, win, gc, n1, n2, y1, y2, z1, z2, ac);
@@ -722,6 +686,7 @@ struct SinkBPair {
         if (fabs(b) > thr || isnan(b)) {
             ctl[wk].stop_acc = 1;
             ctl[wk].stop_slice = ctl[wk].slice_of[slot];
+            ctl[wk].stop_iter = ctl[wk].iter;
         }
     }
 };
@@ -963,15 +928,22 @@ struct GArgsB {
     MxGeom g;
     MxSliceIn si;
     const double *psi, *by, *bz;
-    double *src_acc, *rho, *jx, *chi, *jyn, *jzn;
+    double *src_acc, *rho, *jx, *jx_next, *chi, *jyn, *jzn;
     Ctl *ctl;
 };
 struct GArgsC {
     MxPart P;
     MxGeom g;
+    const double *psim;
+    double *jyn, *jzn;
+    Ctl *ctl;
+};
+struct GArgsS {
+    MxPart P;
+    MxGeom g;
     MxSliceIn si;
-    const double *psi, *psim;
-    double *rho, *jx, *chi, *jyn, *jzn;
+    const double *psi;
+    double *rho, *jx, *chi;
     Ctl *ctl;
 };
 struct GArgsOut {
@@ -1012,40 +984,37 @@ struct GArgsRowsI {
 
 // The group kernels read their arguments from the table (not the kernel
 // argument segment): left alone the compiler holds more of them in vector
-// registers than the single-batch kernels do (B 88 VGPRs and 5 waves per SIMD
-// against 70 and 7, A 68 against 50).  The bounds restore 7 and 8 waves at
-// 256 threads without scratch (B 66, A 64 VGPRs).
+// registers than the single-batch kernels do (A 68 against 50).  The bounds keep
+// 7 or 8 waves at 256 threads without scratch (B as k_mx_B, A 64 VGPRs).
 template <int PT, int CAP>
-__global__ __launch_bounds__(PT, 8) void kg_mx_A(GrpMap m, const GArgsA *__restrict__ t, int init_rho, int advance) {
+__global__ __launch_bounds__(PT, 8) void kg_mx_A(GrpMap m, const GArgsA *__restrict__ t, int advance) {
     int b, bx, wk;
     grp_locate(m, b, bx, wk);
     const GArgsA &a = t[b];
-    mx_A<PT, CAP>(a.P, a.g, a.si, a.psim, a.src_acc, a.asq2, a.Ls, a.laser, a.rho, a.jx, a.chi, init_rho, advance, a.ctl, bx, wk,
+    mx_A<PT, CAP>(a.P, a.g, a.si, a.psim, a.src_acc, a.asq2, a.Ls, a.laser, a.rho, a.jx, a.chi, advance, a.ctl, bx, wk,
          m.gx[b]);
 }
-template <int PT, int CAP>
-__global__ __launch_bounds__(PT, 7) void kg_mx_B(GrpMap m, const GArgsB *__restrict__ t, int first_iter, int init_rho) {
+template <int PT, int CAP, bool RHO, bool CHI>
+__global__ __launch_bounds__(PT, b_waves(PT, CAP, RHO, CHI)) void kg_mx_B(GrpMap m, const GArgsB *__restrict__ t, int it) {
     int b, bx, wk;
     grp_locate(m, b, bx, wk);
     const GArgsB &a = t[b];
-    mx_B<PT, CAP>(a.P, a.g, a.si, a.psi, a.by, a.bz, a.src_acc, a.rho, a.jx, a.chi, a.jyn, a.jzn, first_iter, init_rho, a.ctl,
-         bx, wk, m.gx[b]);
+    mx_B<PT, CAP, RHO, CHI>(a.P, a.g, a.si, a.psi, a.by, a.bz, a.src_acc, a.rho, a.jx, RHO ? nullptr : a.jx_next, a.chi,
+                            a.jyn, a.jzn, it, a.ctl, bx, wk, m.gx[b]);
 }
-template <int PT, int CAP, bool RHO, bool CHI>
-__global__ __launch_bounds__(PT, 6) void kg_mx_C(GrpMap m, const GArgsC *__restrict__ t) {
-    extern __shared__ double ldsd[];
-    int b, bx, wk;
-    grp_locate(m, b, bx, wk);
-    const GArgsC &a = t[b];
-    mx_C<PT, CAP, RHO, CHI>(a.P, a.g, a.si, a.psi, a.psim, a.rho, a.jx, a.chi, a.jyn, a.jzn, a.ctl, ldsd, bx, wk);
-}
-// S phase: the C table carries the same pointers (psi, rho, jx, chi).
 template <int PT, int CAP>
-__global__ __launch_bounds__(PT) void kg_mx_S(GrpMap m, const GArgsC *__restrict__ t) {
-    extern __shared__ double ldsd[];
+__global__ __launch_bounds__(PT, 8) void kg_mx_C(GrpMap m, const GArgsC *__restrict__ t) {
     int b, bx, wk;
     grp_locate(m, b, bx, wk);
     const GArgsC &a = t[b];
+    mx_C<PT, CAP>(a.P, a.g, a.psim, a.jyn, a.jzn, a.ctl, bx, wk);
+}
+template <int PT, int CAP>
+__global__ __launch_bounds__(PT) void kg_mx_S(GrpMap m, const GArgsS *__restrict__ t) {
+    extern __shared__ double ldsd[];
+    int b, bx, wk;
+    grp_locate(m, b, bx, wk);
+    const GArgsS &a = t[b];
     mx_S<PT, CAP>(a.P, a.g, a.si, a.psi, a.rho, a.jx, a.chi, a.ctl, ldsd, bx, wk);
 }
 __global__ void kg_mx_out(GrpMap m, const GArgsOut *__restrict__ t, int with_ex, int slot, int final_step) {
@@ -1147,6 +1116,10 @@ struct MixedState {
     double *bpart = nullptr;
     size_t bstride = 0;     // partial sums per member
     double *jbuf[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [parity][y/z], nw planes each
+    // rho by slice parity and jx by iteration parity: a launch that deposits finds
+    // its plane cleared by an earlier one, and a pass that stops keeps the planes of
+    // the step it stopped in.  [0] are the wake's own, [1] belong to this state.
+    double *rho2[2] = {nullptr, nullptr}, *jx2[2] = {nullptr, nullptr};
     std::vector<int> h_perm;
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     unsigned graph_epoch = 0;  // Wake::inputs_epoch the graphs were captured at
@@ -1177,7 +1150,7 @@ static hipError_t copy_wait(void *dst, const void *src, size_t bytes, hipMemcpyK
 }
 
 static void free_part(MxPart &P) {
-    void *arrs[] = {P.cell, P.off, P.p, P.w, P.ps};
+    void *arrs[] = {P.cell, P.off, P.p, P.w, P.ps, P.iv, P.wq};
     for (void *a : arrs)
         if (a) (void)hipFree(a);
     P = MxPart{};
@@ -1192,6 +1165,13 @@ static int alloc_part(MxPart &P, size_t n) {
     QP_HIP_CHECK(hipMalloc(&P.ps, 16 * n));
     return QP_OK;
 }
+// The scratch of a slice step beside the live particles: 1/(1 + psi) and the windows of
+// the particle blocks (at the smallest tile's 128 particles a block).
+static int alloc_scratch(MxPart &P, size_t n) {
+    QP_HIP_CHECK(hipMalloc(&P.iv, 8 * n));
+    QP_HIP_CHECK(hipMalloc(&P.wq, sizeof(int4) * (n / 128 + 1)));
+    return QP_OK;
+}
 
 void wake_destroy_mixed(Wake *w) {
     MixedState *m = mstate(w);
@@ -1200,7 +1180,7 @@ void wake_destroy_mixed(Wake *w) {
     free_part(m->Q);
     free_part(m->I);
     void *arrs[] = {m->perm,       m->perm2,      m->perm0,      m->npw,        m->count,     m->cursor,
-                    m->totals,     m->bpart,      m->jbuf[0][0], m->jbuf[0][1], m->jbuf[1][0], m->jbuf[1][1]};
+                    m->totals,     m->bpart,      m->rho2[1],    m->jx2[1],     m->jbuf[0][0], m->jbuf[0][1], m->jbuf[1][0], m->jbuf[1][1]};
     for (void *a : arrs)
         if (a) (void)hipFree(a);
     for (auto &g : m->gexec)
@@ -1241,6 +1221,10 @@ static int ensure_state(Wake *w) {
         QP_HIP_CHECK(hipMalloc(&m->bpart, sizeof(double) * m->bstride * nw));
         for (int a = 0; a < 2; ++a)
             for (int b = 0; b < 2; ++b) QP_HIP_CHECK(hipMalloc(&m->jbuf[a][b], sizeof(double) * nn * nw));
+        m->rho2[0] = w->rho;
+        m->jx2[0] = w->jx;
+        QP_HIP_CHECK(hipMalloc(&m->rho2[1], sizeof(double) * nn * nw));
+        QP_HIP_CHECK(hipMalloc(&m->jx2[1], sizeof(double) * nn * nw));
         const int ntk = (w->p.nz + kTile - 1) / kTile, ntj = (w->p.ny + kTile - 1) / kTile;
         const size_t nbins = (size_t)ntk * ntj * kTileBins;
         QP_HIP_CHECK(hipMalloc(&m->count, sizeof(unsigned) * nbins));
@@ -1258,6 +1242,7 @@ static int ensure_state(Wake *w) {
         if (m->perm2) (void)hipFree(m->perm2);
         if (m->perm0) (void)hipFree(m->perm0);
         QP_TRY(alloc_part(m->P, need));
+        QP_TRY(alloc_scratch(m->P, need));
         QP_TRY(alloc_part(m->Q, need));
         QP_TRY(alloc_part(m->I, need));
         QP_HIP_CHECK(hipMalloc(&m->perm, sizeof(int) * need));
@@ -1429,6 +1414,19 @@ int with_tile(int pt, int cap, F &&f) {
     return QP_ERR_ARG;
 }
 
+// f(bool_constant<RHO>, bool_constant<CHI>) for run-time flags.
+template <class F>
+int with_flags(bool rho, bool chi, F &&f) {
+    if (rho) return chi ? f(std::true_type{}, std::true_type{}) : f(std::true_type{}, std::false_type{});
+    return chi ? f(std::false_type{}, std::true_type{}) : f(std::false_type{}, std::false_type{});
+}
+
+// The planes slice i's step leaves rho and jx in (run in full).
+const double *rho_of(const MixedState *m, int i) { return m->rho2[i & 1]; }
+const double *jx_of(const Wake *w, const MixedState *m, int i) {
+    return m->jx2[(i == 0 || w->p.K == 0) ? 0 : (w->p.K - 1) & 1];
+}
+
 #define MLAUNCH(kern, grid, block, lds, ...)                                            \
     do {                                                                                \
         hipLaunchKernelGGL(kern, grid, dim3(block), lds, s, __VA_ARGS__);               \
@@ -1473,7 +1471,7 @@ int psi_solve(MxRun &R, hipStream_t s, int slot, double *dst) {
     return QP_OK;
 }
 
-int b_solve(MxRun &R, hipStream_t s, int slot) {
+int b_solve(MxRun &R, hipStream_t s, int slot, const double *jx) {
     Wake *w = R.w;
     const Solver2d &S = w->S;
     MixedState *m = R.m;
@@ -1481,7 +1479,7 @@ int b_solve(MxRun &R, hipStream_t s, int slot) {
     const int nw = R.nw;
     double *jy = m->jbuf[1 - slot][0], *jz = m->jbuf[1 - slot][1];
     double *jyn = m->jbuf[slot][0], *jzn = m->jbuf[slot][1];
-    SrcB src{w->by, w->bz, w->jx, jy, jz, jyn, jzn, S.n1, S.n2, p.D, 1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
+    SrcB src{w->by, w->bz, jx, jy, jz, jyn, jzn, S.n1, S.n2, p.D, 1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
     SinkBPair snk{w->by, w->bz, S.n1, S.n2, p.b_threshold, w->ctl, slot, 1.0 / ((double)S.n1 * S.n2)};
     if (S.wave) {
         prof_begin(w, "solve");
@@ -1552,13 +1550,14 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
     if (w->bunch) QP_TRY(bunch_slice_sources(w->bunch, (const Ctl *)w->ctl, slot, 0, s));
     prof_begin(w, "push_A");
     MLAUNCH((k_mx_A<PT, CAP>), pg, PT, 0, m->P, R.g, si, (const double *)w->psim, w->src, w->asq2,
-            (const LaserGauss *)w->d_laser, laser, w->rho, w->jx, w->chi, s_phase ? 1 : 0,
+            (const LaserGauss *)w->d_laser, laser, m->rho2[slot], m->jx2[0], w->chi,
             first ? 0 : (p.K == 0 ? 2 : 1), w->ctl);
     prof_end(w, "push_A");
     QP_TRY(psi_solve(R, s, slot, psi));
     if (s_phase) {
         prof_begin(w, "push_S");
-        MLAUNCH((k_mx_S<PT, CAP>), pg, PT, R.ldsS, m->P, R.g, si, (const double *)psi, w->rho, w->jx, w->chi, w->ctl);
+        MLAUNCH((k_mx_S<PT, CAP>), pg, PT, R.ldsS, m->P, R.g, si, (const double *)psi, m->rho2[slot], m->jx2[0],
+                w->chi, w->ctl);
         prof_end(w, "push_S");
         if (p.longitudinal_b) QP_TRY(bx_solve(R, s, slot));
         if (w->env)
@@ -1566,29 +1565,22 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
         if (i == 0) return QP_OK;
     } else {
         for (int it = 0; it < p.K; ++it) {
-            prof_begin(w, "push_B");
             const bool first_it = it == 0, last_it = it == p.K - 1;
-            MLAUNCH((k_mx_B<PT, CAP>), pg, PT, 0, m->P, R.g, si, (const double *)psi, (const double *)w->by,
-                    (const double *)w->bz, w->src, w->rho, w->jx, w->chi, m->jbuf[slot][0], m->jbuf[slot][1],
-                    first_it ? 1 : 0, last_it ? 1 : 0, w->ctl);
+            double *jx = m->jx2[it & 1], *jx_next = last_it ? nullptr : m->jx2[(it + 1) & 1];
+            prof_begin(w, "push_B");
+            QP_TRY(with_flags(last_it, first_it, [&](auto RH, auto CH) {
+                MLAUNCH((k_mx_B<PT, CAP, decltype(RH)::value, decltype(CH)::value>), pg, PT, 0, m->P, R.g, si,
+                        (const double *)psi, (const double *)w->by, (const double *)w->bz, w->src, m->rho2[slot], jx,
+                        jx_next, w->chi, m->jbuf[slot][0], m->jbuf[slot][1], it, w->ctl);
+                return QP_OK;
+            }));
             prof_end(w, "push_B");
             QP_TRY(psi_solve(R, s, slot, w->psim));
             prof_begin(w, "push_C");
-            const size_t ldsc = sizeof(double) * CAP * (3 + (first_it ? 1 : 0) + (last_it ? 1 : 0));
-            if (first_it && last_it)
-                MLAUNCH((k_mx_C<PT, CAP, true, true>), pg, PT, ldsc, m->P, R.g, si, (const double *)psi,
-                        (const double *)w->psim, w->rho, w->jx, w->chi, m->jbuf[slot][0], m->jbuf[slot][1], w->ctl);
-            else if (first_it)
-                MLAUNCH((k_mx_C<PT, CAP, false, true>), pg, PT, ldsc, m->P, R.g, si, (const double *)psi,
-                        (const double *)w->psim, w->rho, w->jx, w->chi, m->jbuf[slot][0], m->jbuf[slot][1], w->ctl);
-            else if (last_it)
-                MLAUNCH((k_mx_C<PT, CAP, true, false>), pg, PT, ldsc, m->P, R.g, si, (const double *)psi,
-                        (const double *)w->psim, w->rho, w->jx, w->chi, m->jbuf[slot][0], m->jbuf[slot][1], w->ctl);
-            else
-                MLAUNCH((k_mx_C<PT, CAP, false, false>), pg, PT, ldsc, m->P, R.g, si, (const double *)psi,
-                        (const double *)w->psim, w->rho, w->jx, w->chi, m->jbuf[slot][0], m->jbuf[slot][1], w->ctl);
+            MLAUNCH((k_mx_C<PT, CAP>), pg, PT, 0, m->P, R.g, (const double *)w->psim, m->jbuf[slot][0],
+                    m->jbuf[slot][1], w->ctl);
             prof_end(w, "push_C");
-            QP_TRY(b_solve(R, s, slot));
+            QP_TRY(b_solve(R, s, slot, jx));
         }
         if (p.longitudinal_b) QP_TRY(bx_solve(R, s, slot));
         if (w->env)
@@ -1676,10 +1668,11 @@ int ensure_snapshots(Wake *w, MixedState *m) {
 }
 
 // Snapshot of slice i's output planes and control blocks into device slot d.
-int snapshot(Wake *w, MixedState *m, hipStream_t s, int slot, int d) {
+int snapshot(Wake *w, MixedState *m, hipStream_t s, int i, int d) {
+    const int slot = i & 1;
     const size_t nn = w->nn(), nw = (size_t)w->nw, plane = nn * nw;
     double *dst = m->snap_dev + (size_t)d * m->snap_words;
-    const double *src[kSnapPlanes] = {w->psi_b[slot], w->rho, w->jx, m->jbuf[1 - slot][0], m->jbuf[1 - slot][1],
+    const double *src[kSnapPlanes] = {w->psi_b[slot], rho_of(m, i), jx_of(w, m, i), m->jbuf[1 - slot][0], m->jbuf[1 - slot][1],
                                       w->ex, w->ey, w->ez, w->by, w->bz, w->chi,
                                       w->p.longitudinal_b ? w->bx : nullptr};
     for (int f = 0; f < kSnapPlanes; ++f)
@@ -1819,8 +1812,8 @@ int pass_setup(Wake *w, MxRun &R) {
     QP_HIP_CHECK(hipMemcpyAsync(w->d_laser, hl.data(), sizeof(LaserGauss) * nw, hipMemcpyHostToDevice, s));
     // zero the fields (src/System_3d.cpp:265-316) and the control blocks
     const size_t plane = sizeof(double) * R.nn * nw;
-    double *zero_list[] = {w->psi_b[0], w->psi_b[1], w->psim, w->by, w->bz, w->rho_ion, w->src, w->rho, w->jx,
-                           w->chi, w->ex, w->ey, w->ez, w->asq2, w->bx};
+    double *zero_list[] = {w->psi_b[0], w->psi_b[1], w->psim, w->by, w->bz, w->rho_ion, w->src, m->rho2[0], m->rho2[1],
+                           m->jx2[0], m->jx2[1], w->chi, w->ex, w->ey, w->ez, w->asq2, w->bx};
     for (double *a : zero_list) QP_HIP_CHECK(hipMemsetAsync(a, 0, plane, s));
     for (int a = 0; a < 2; ++a)
         for (int b = 0; b < 2; ++b) QP_HIP_CHECK(hipMemsetAsync(m->jbuf[a][b], 0, plane, s));
@@ -1863,7 +1856,7 @@ int deliver_inline(Wake *w, MxRun &R, batch_cb cb, void *user, int i, std::vecto
             continue;
         }
         ++running;
-        QP_TRY(deliver_member(w, cb, user, mb, i, QP_SLICE_NORMAL, w->psi_b[slot], w->rho, w->jx,
+        QP_TRY(deliver_member(w, cb, user, mb, i, QP_SLICE_NORMAL, w->psi_b[slot], rho_of(m, i), jx_of(w, m, i),
                               m->jbuf[1 - slot][0], m->jbuf[1 - slot][1], w->ex, w->ey, w->ez, w->by, w->bz, w->chi,
                               p.longitudinal_b ? w->bx : nullptr));
     }
@@ -1924,7 +1917,12 @@ int pass_finish(Wake *w, MxRun &R, batch_cb cb, void *user, int i_end, std::vect
             const double *bz0 = stopped ? w->zero2 : w->bz;
             const double *chi0 = stopped ? w->zero2 : w->chi;
             const double *bx0 = p.longitudinal_b ? (stopped ? w->zero2 : w->bx) : nullptr;
-            QP_TRY(deliver_member(w, cb, user, mb, 0, QP_SLICE_FINAL, w->psi_b[cslot], w->rho, w->jx,
+            // rho and jx of the last step: a stopped one ended in iteration stop_iter, where
+            // jx is that iteration's and rho the step's own only after its last iteration
+            const int it = hc[mb].stop_iter;
+            const double *rho0 = stopped ? m->rho2[it == p.K - 1 ? cslot : 1 - cslot] : rho_of(m, 0);
+            const double *jx0 = stopped ? m->jx2[it & 1] : jx_of(w, m, 0);
+            QP_TRY(deliver_member(w, cb, user, mb, 0, QP_SLICE_FINAL, w->psi_b[cslot], rho0, jx0,
                                   m->jbuf[1 - cslot][0], m->jbuf[1 - cslot][1], w->ex, w->ey, w->ez, by0, bz0,
                                   chi0, bx0));
         }
@@ -2105,7 +2103,7 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
             // device slot d was last read by the copy of slice i + 2
             const int d = i & 1;
             QP_HIP_CHECK(hipStreamWaitEvent(s, m->ev_copied[d], 0));
-            QP_TRY(snapshot(w, m, s, slot, d));
+            QP_TRY(snapshot(w, m, s, i, d));
             QP_HIP_CHECK(hipEventRecord(m->ev_done[d], s));
             const int h = (int)(seq++ % kHostSlots);
             {
@@ -2165,14 +2163,15 @@ namespace {
 // captured slice steps hold pointers into it; each run rewrites the contents).
 struct GroupTabs {
     GArgsA A[2][kGroupMax];
-    GArgsB B[2][kGroupMax];
+    GArgsB B[2][2][kGroupMax];   // [slice parity][iteration parity]
     GArgsC C[2][kGroupMax];
+    GArgsS S[2][kGroupMax];
     GArgsOut O[kGroupMax];
     GArgsRowsF<SrcPsi> PF[2][kGroupMax];
     GArgsCols PC[kGroupMax];
     GArgsRowsI<SinkPsiFinal> PI[2][kGroupMax];   // psi of the slice
     GArgsRowsI<SinkPsiFinal> MI[kGroupMax];      // psi_middle
-    GArgsRowsF<SrcB> BF[2][kGroupMax];
+    GArgsRowsF<SrcB> BF[2][2][kGroupMax];
     GArgsCols BC[kGroupMax];
     GArgsRowsI<SinkBPair> BI[2][kGroupMax];
 };
@@ -2220,11 +2219,12 @@ void group_tables(Group *G, std::vector<MxRun> &R, GroupTabs &T, GroupMaps &M) {
         for (int sl = 0; sl < 2; ++sl) {
             const MxSliceIn &si = R[b].si[sl];
             T.A[sl][b] = GArgsA{m->P, R[b].g, si, w->psim, w->src, w->asq2, (const LaserGauss *)w->d_laser,
-                                laser, w->rho, w->jx, w->chi, w->ctl};
-            T.B[sl][b] = GArgsB{m->P, R[b].g, si, w->psi_b[sl], w->by, w->bz, w->src, w->rho, w->jx, w->chi,
-                                m->jbuf[sl][0], m->jbuf[sl][1], w->ctl};
-            T.C[sl][b] = GArgsC{m->P, R[b].g, si, w->psi_b[sl], w->psim, w->rho, w->jx, w->chi,
-                                m->jbuf[sl][0], m->jbuf[sl][1], w->ctl};
+                                laser, m->rho2[sl], m->jx2[0], w->chi, w->ctl};
+            for (int par = 0; par < 2; ++par)
+                T.B[sl][par][b] = GArgsB{m->P, R[b].g, si, w->psi_b[sl], w->by, w->bz, w->src, m->rho2[sl], m->jx2[par],
+                                         m->jx2[1 - par], w->chi, m->jbuf[sl][0], m->jbuf[sl][1], w->ctl};
+            T.C[sl][b] = GArgsC{m->P, R[b].g, w->psim, m->jbuf[sl][0], m->jbuf[sl][1], w->ctl};
+            T.S[sl][b] = GArgsS{m->P, R[b].g, si, w->psi_b[sl], m->rho2[sl], m->jx2[0], w->chi, w->ctl};
             SrcPsi sp{w->src, w->rho_ion, w->rho_b_src(), w->jx_b_src(), w->bsrc_stride(), w->ctl, sl, S.n2, R[b].nn};
             T.PF[sl][b] = GArgsRowsF<SrcPsi>{sp, S.spec[0], S.spec[0], S.n1, S.n2, S.ax2.dev.tw, w->ctl,
                                              R[b].sstride};
@@ -2233,8 +2233,11 @@ void group_tables(Group *G, std::vector<MxRun> &R, GroupTabs &T, GroupMaps &M) {
                                                    R[b].sstride};
             double *jy = m->jbuf[1 - sl][0], *jz = m->jbuf[1 - sl][1];
             double *jyn = m->jbuf[sl][0], *jzn = m->jbuf[sl][1];
-            SrcB sb{w->by, w->bz, w->jx, jy, jz, jyn, jzn, S.n1, S.n2, p.D, 1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
-            T.BF[sl][b] = GArgsRowsF<SrcB>{sb, S.spec[0], S.spec[1], S.n1, S.n2, S.ax2.dev.tw, w->ctl, R[b].sstride};
+            for (int par = 0; par < 2; ++par) {
+                SrcB sb{w->by, w->bz, m->jx2[par], jy, jz, jyn, jzn, S.n1, S.n2, p.D, 1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
+                T.BF[sl][par][b] = GArgsRowsF<SrcB>{sb, S.spec[0], S.spec[1], S.n1, S.n2, S.ax2.dev.tw, w->ctl,
+                                                    R[b].sstride};
+            }
             SinkBPair kb{w->by, w->bz, S.n1, S.n2, p.b_threshold, w->ctl, sl, scale};
             T.BI[sl][b] = GArgsRowsI<SinkBPair>{kb, S.spec[0], S.spec[1], S.n1, S.n2, S.ax2.dev.tw, w->ctl,
                                                 R[b].sstride};
@@ -2328,30 +2331,26 @@ int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
     const int slot = i & 1;
     const bool first = (i == p.nx - 1);
     const bool s_phase = (i == 0) || (p.K == 0);
-    GLAUNCH((kg_mx_A<PT, CAP>), M.part, PT, 0, T->A[slot], s_phase ? 1 : 0, first ? 0 : (p.K == 0 ? 2 : 1));
+    GLAUNCH((kg_mx_A<PT, CAP>), M.part, PT, 0, T->A[slot], first ? 0 : (p.K == 0 ? 2 : 1));
     GSOLVE_T(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
     GSOLVE(kg_cols, M.cols1, 1, T->PC);
     GSOLVE_T(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->PI[slot]);
     if (s_phase) {
-        GLAUNCH((kg_mx_S<PT, CAP>), M.part, PT, sizeof(double) * 3 * CAP, T->C[slot]);
+        GLAUNCH((kg_mx_S<PT, CAP>), M.part, PT, sizeof(double) * 3 * CAP, T->S[slot]);
         if (i == 0) return QP_OK;
     } else {
         for (int it = 0; it < p.K; ++it) {
             const bool first_it = it == 0, last_it = it == p.K - 1;
-            GLAUNCH((kg_mx_B<PT, CAP>), M.part, PT, 0, T->B[slot], first_it ? 1 : 0, last_it ? 1 : 0);
+            QP_TRY(with_flags(last_it, first_it, [&](auto RH, auto CH) {
+                GLAUNCH((kg_mx_B<PT, CAP, decltype(RH)::value, decltype(CH)::value>), M.part, PT, 0, T->B[slot][it & 1],
+                        it);
+                return QP_OK;
+            }));
             GSOLVE_T(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
             GSOLVE(kg_cols, M.cols1, 1, T->PC);
             GSOLVE_T(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->MI);
-            const size_t ldsc = sizeof(double) * CAP * (3 + (first_it ? 1 : 0) + (last_it ? 1 : 0));
-            if (first_it && last_it)
-                GLAUNCH((kg_mx_C<PT, CAP, true, true>), M.part, PT, ldsc, T->C[slot]);
-            else if (first_it)
-                GLAUNCH((kg_mx_C<PT, CAP, false, true>), M.part, PT, ldsc, T->C[slot]);
-            else if (last_it)
-                GLAUNCH((kg_mx_C<PT, CAP, true, false>), M.part, PT, ldsc, T->C[slot]);
-            else
-                GLAUNCH((kg_mx_C<PT, CAP, false, false>), M.part, PT, ldsc, T->C[slot]);
-            GSOLVE_T(kg_rows_fwd, SrcB, M.rows2, 2, T->BF[slot]);
+            GLAUNCH((kg_mx_C<PT, CAP>), M.part, PT, 0, T->C[slot]);
+            GSOLVE_T(kg_rows_fwd, SrcB, M.rows2, 2, T->BF[slot][it & 1]);
             GSOLVE(kg_cols, M.cols2, 2, T->BC);
             GSOLVE_T(kg_rows_inv, SinkBPair, M.rows2, 2, T->BI[slot]);
         }
