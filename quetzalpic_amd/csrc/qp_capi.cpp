@@ -587,7 +587,7 @@ int wake_alloc_common(Wake *w) {
     QP_HIP_CHECK(hipMemset(w->ctl, 0, sizeof(Ctl) * nw));
     QP_HIP_CHECK(hipMalloc(&w->d_laser, sizeof(LaserGauss) * nw));
     QP_HIP_CHECK(hipMemset(w->d_laser, 0, sizeof(LaserGauss) * nw));
-    QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * nn * 12, hipHostMallocDefault));
+    QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * (nn * kOutPlanes + kCtlWords), hipHostMallocDefault));
     QP_HIP_CHECK(hipEventCreate(&w->ev0));
     QP_HIP_CHECK(hipEventCreate(&w->ev1));
     if (p.precision == QP_PREC_MIXED) {
@@ -635,41 +635,6 @@ void prof_end(Wake *w, const char *cls) {
     if (w->prof_ev.size() < 2 * (size_t)(w->prof_count + 1)) return;
     (void)hipEventRecord(w->prof_ev[2 * w->prof_count + 1], w->stream());
     w->prof_count++;
-}
-
-int deliver_slice(Wake *w, qp_slice_cb cb, void *user, int slice, int kind, const double *psi, const double *rho,
-                  const double *jx, const double *jy, const double *jz, const double *ex, const double *ey,
-                  const double *ez, const double *by, const double *bz, const double *chi, const double *bx) {
-    const size_t nn = w->nn();
-    hipStream_t s = w->stream();
-    const double *src[12] = {psi, rho, jx, jy, jz, ex, ey, ez, by, bz, chi, bx};
-    const int nf = bx ? 12 : 11;
-    for (int f = 0; f < nf; ++f)
-        QP_HIP_CHECK(hipMemcpyAsync(w->h_out + f * nn, src[f] ? src[f] : w->zero2, sizeof(double) * nn,
-                                    hipMemcpyDeviceToHost, s));
-    QP_HIP_CHECK(hipStreamSynchronize(s));
-    qp_slice_view v;
-    v.slice = slice;
-    v.kind = kind;
-    const double *h = w->h_out;
-    v.psi = h;
-    v.rho = h + nn;
-    v.jx = h + 2 * nn;
-    v.jy = h + 3 * nn;
-    v.jz = h + 4 * nn;
-    v.ex = h + 5 * nn;
-    v.ey = h + 6 * nn;
-    v.ez = h + 7 * nn;
-    v.by = h + 8 * nn;
-    v.bz = h + 9 * nn;
-    v.chi = h + 10 * nn;
-    v.bx = bx ? h + 11 * nn : nullptr;
-    int r = cb(&v, user);
-    if (r != 0) {
-        set_error("slice callback returned " + std::to_string(r));
-        return QP_ERR_STATE;
-    }
-    return QP_OK;
 }
 
 }  // namespace qp

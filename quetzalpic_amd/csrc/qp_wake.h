@@ -57,7 +57,7 @@ struct Wake {
     double *rho_b3 = nullptr, *jx_b3 = nullptr;  // nx*ny*nz or null
 
     Ctl *ctl = nullptr;                  // nw control blocks
-    double *h_out = nullptr;             // pinned host staging, 12 planes
+    double *h_out = nullptr;             // pinned host staging, 12 planes and a control block
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double last_ms = 0.0;
     // mixed path: particle tile (threads per block, LDS window nodes per grid),
@@ -131,10 +131,22 @@ void prof_begin(Wake *w, const char *cls);
 void prof_end(Wake *w, const char *cls);
 
 // Stage the output planes of slice i to host and call cb (bx may be null).
-int deliver_slice(Wake *w, qp_slice_cb cb, void *user, int slice, int kind, const double *psi,
-                  const double *rho, const double *jx, const double *jy, const double *jz, const double *ex,
-                  const double *ey, const double *ez, const double *by, const double *bz, const double *chi,
-                  const double *bx = nullptr);
+// Per-slice output (qp_output.hip).  The planes of one view, in its order.
+constexpr int kOutPlanes = 12;  // psi, rho, jx, jy, jz, ex, ey, ez, by, bz, chi, bx
+constexpr size_t kCtlWords = sizeof(Ctl) / sizeof(double);
+static_assert(sizeof(Ctl) % sizeof(double) == 0, "control blocks travel as whole doubles");
+struct OutPlanes {
+    const double *p[kOutPlanes];  // device planes; null = a plane of zeros (bx: absent)
+};
+// One launch that copies the planes (`plane` doubles each, side by side at dst) and `nctl`
+// control blocks behind them.
+int pack_planes(const OutPlanes &o, size_t plane, const Ctl *ctl, int nctl, double *dst, hipStream_t s);
+// Stages a view and its control block in the wake's pinned buffer and waits for it.
+int stage_slice(Wake *w, const OutPlanes &o, const Ctl *ctl, Ctl *host_ctl);
+// Hands the staged view to the callback.
+int call_slice(Wake *w, qp_slice_cb cb, void *user, int slice, int kind, bool with_bx);
+// stage_slice + call_slice.
+int deliver_slice(Wake *w, qp_slice_cb cb, void *user, int slice, int kind, const OutPlanes &o);
 
 // A group of batches with possibly different transverse grids, advanced in
 // lockstep with one launch per phase of the slice step over all of them.

@@ -388,6 +388,9 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
     if (w->bunch) QP_TRY(bunch_clear_fields(w->bunch, s));
 
     int delivered_stop = 0;
+    auto planes = [w] {
+        return OutPlanes{{w->psi, w->rho, w->jx, w->jy, w->jz, w->ex, w->ey, w->ez, w->by, w->bz, w->chi, nullptr}};
+    };
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
     for (int i = p.nx - 1; i >= i_end; --i) {
         const double *asq;
@@ -454,17 +457,14 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
                i < p.nx - 1 ? 1 : 0, ctl, 0);
         if (w->bunch) QP_TRY(bunch_slice_gather(w->bunch, w->ex, w->ey, w->ez, w->by, w->bz, ctl, -1, i, s));
         if (cb) {
-            QP_HIP_CHECK(hipStreamSynchronize(s));
             Ctl hc;
-            QP_HIP_CHECK(hipMemcpy(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
+            QP_TRY(stage_slice(w, planes(), ctl, &hc));
             if (hc.stop_acc) {
-                QP_TRY(deliver_slice(w, cb, user, hc.stop_slice, QP_SLICE_STOPPED, w->psi, w->rho, w->jx, w->jy,
-                                     w->jz, w->ex, w->ey, w->ez, w->by, w->bz, w->chi));
+                QP_TRY(call_slice(w, cb, user, hc.stop_slice, QP_SLICE_STOPPED, false));
                 delivered_stop = 1;
                 break;
             }
-            QP_TRY(deliver_slice(w, cb, user, i, QP_SLICE_NORMAL, w->psi, w->rho, w->jx, w->jy, w->jz, w->ex,
-                                 w->ey, w->ez, w->by, w->bz, w->chi));
+            QP_TRY(call_slice(w, cb, user, i, QP_SLICE_NORMAL, false));
         }
         LAUNCH(k_copy, gb, w->jy, w->jyn, nn, ctl);
         LAUNCH(k_copy, gb, w->jz, w->jzn, nn, ctl);
@@ -485,16 +485,12 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
     w->last_ms = ms;
     Ctl hc;
     QP_HIP_CHECK(hipMemcpy(&hc, ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
-    if (hc.stop_acc && cb && !delivered_stop) {
-        QP_TRY(deliver_slice(w, cb, user, hc.stop_slice, QP_SLICE_STOPPED, w->psi, w->rho, w->jx, w->jy, w->jz,
-                             w->ex, w->ey, w->ez, w->by, w->bz, w->chi));
-    }
+    if (hc.stop_acc && cb && !delivered_stop)
+        QP_TRY(deliver_slice(w, cb, user, hc.stop_slice, QP_SLICE_STOPPED, planes()));
     if (cb && i_end == 0) {
-        const double *bz0 = hc.stop_acc ? w->zero2 : w->bz;
-        const double *by0 = hc.stop_acc ? w->zero2 : w->by;
-        const double *chi0 = hc.stop_acc ? w->zero2 : w->chi;
-        QP_TRY(deliver_slice(w, cb, user, 0, QP_SLICE_FINAL, w->psi, w->rho, w->jx, w->jy, w->jz, w->ex, w->ey,
-                             w->ez, by0, bz0, chi0));
+        OutPlanes o = planes();
+        if (hc.stop_acc) o.p[8] = o.p[9] = o.p[10] = w->zero2;
+        QP_TRY(deliver_slice(w, cb, user, 0, QP_SLICE_FINAL, o));
     }
     if (stop_slice) *stop_slice = hc.stop_acc ? hc.stop_slice : -1;
     return hc.stop_acc ? QP_STOPPED : QP_OK;

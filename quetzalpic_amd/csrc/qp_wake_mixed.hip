@@ -1619,13 +1619,15 @@ int resort(MxRun &R, hipStream_t s) {
     return QP_OK;
 }
 
-// Stage the planes of one member (offset go) and call the batch callback.
-int deliver_member(Wake *w, batch_cb cb, void *user, int member, int slice, int kind, const double *psi,
-                   const double *rho, const double *jx, const double *jy, const double *jz, const double *ex,
-                   const double *ey, const double *ez, const double *by, const double *bz, const double *chi,
-                   const double *bx = nullptr) {
-    const size_t go = (size_t)member * w->nn();
-    auto off = [&](const double *a) -> const double * { return a ? a + go : nullptr; };
+// The planes of member mb of a batch's planes.
+OutPlanes member_planes(const Wake *w, int mb, const OutPlanes &o) {
+    OutPlanes r = o;
+    for (const double *&a : r.p)
+        if (a) a += (size_t)mb * w->nn();
+    return r;
+}
+// Hands a member's staged view to the batch callback.
+int call_member(Wake *w, batch_cb cb, void *user, int member, int slice, int kind, bool with_bx) {
     struct Fwd {
         batch_cb cb;
         void *user;
@@ -1635,12 +1637,25 @@ int deliver_member(Wake *w, batch_cb cb, void *user, int member, int slice, int 
         const Fwd *ff = static_cast<const Fwd *>(u);
         return ff->cb(ff->member, v, ff->user);
     };
-    return deliver_slice(w, tramp, &f, slice, kind, off(psi), off(rho), off(jx), off(jy), off(jz), off(ex),
-                         off(ey), off(ez), off(by), off(bz), off(chi), off(bx));
+    return call_slice(w, tramp, &f, slice, kind, with_bx);
+}
+int deliver_member(Wake *w, batch_cb cb, void *user, int member, int slice, int kind, const OutPlanes &o) {
+    QP_TRY(stage_slice(w, member_planes(w, member, o), nullptr, nullptr));
+    return call_member(w, cb, user, member, slice, kind, o.p[kOutPlanes - 1] != nullptr);
+}
+// The planes slice i's step leaves (run in full), and those of a stopped one.
+OutPlanes slice_planes(const Wake *w, const MixedState *m, int i) {
+    const int slot = i & 1;
+    return OutPlanes{{w->psi_b[slot], rho_of(m, i), jx_of(w, m, i), m->jbuf[1 - slot][0], m->jbuf[1 - slot][1], w->ex,
+                      w->ey, w->ez, w->by, w->bz, w->chi, w->p.longitudinal_b ? w->bx : nullptr}};
+}
+OutPlanes stopped_planes(const Wake *w) {
+    return OutPlanes{{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, w->by, w->bz, w->chi,
+                      nullptr}};
 }
 
 constexpr int kHostSlots = 4;   // pinned host slots of the streamed output
-constexpr int kSnapPlanes = 12; // psi, rho, jx, jy, jz, ex, ey, ez, by, bz, chi, bx
+constexpr int kSnapPlanes = kOutPlanes;
 
 // Slot layout: plane f of member m at (f * nw + m) * nn, then the nw control
 // blocks (rounded up to whole doubles).
@@ -1669,17 +1684,8 @@ int ensure_snapshots(Wake *w, MixedState *m) {
 
 // Snapshot of slice i's output planes and control blocks into device slot d.
 int snapshot(Wake *w, MixedState *m, hipStream_t s, int i, int d) {
-    const int slot = i & 1;
-    const size_t nn = w->nn(), nw = (size_t)w->nw, plane = nn * nw;
-    double *dst = m->snap_dev + (size_t)d * m->snap_words;
-    const double *src[kSnapPlanes] = {w->psi_b[slot], rho_of(m, i), jx_of(w, m, i), m->jbuf[1 - slot][0], m->jbuf[1 - slot][1],
-                                      w->ex, w->ey, w->ez, w->by, w->bz, w->chi,
-                                      w->p.longitudinal_b ? w->bx : nullptr};
-    for (int f = 0; f < kSnapPlanes; ++f)
-        if (src[f])
-            QP_HIP_CHECK(hipMemcpyAsync(dst + f * plane, src[f], sizeof(double) * plane, hipMemcpyDeviceToDevice, s));
-    QP_HIP_CHECK(hipMemcpyAsync(dst + kSnapPlanes * plane, w->ctl, sizeof(Ctl) * nw, hipMemcpyDeviceToDevice, s));
-    return QP_OK;
+    return pack_planes(slice_planes(w, m, i), w->nn() * (size_t)w->nw, w->ctl, w->nw, m->snap_dev + (size_t)d * m->snap_words,
+                       s);
 }
 
 // View of member mb in a host slot.
@@ -1841,24 +1847,20 @@ int pass_start(Wake *w, MxRun &R) {
 // slice once.  `running` counts the members still running.
 int deliver_inline(Wake *w, MxRun &R, batch_cb cb, void *user, int i, std::vector<char> &delivered_stop,
                    std::vector<Ctl> &hc, int &running) {
-    const qp_wake_params &p = w->p;
     MixedState *m = R.m;
-    const int nw = R.nw, slot = i & 1;
-    QP_HIP_CHECK(hipStreamSynchronize(w->stream()));
-    QP_HIP_CHECK(copy_wait(hc.data(), w->ctl, sizeof(Ctl) * nw, hipMemcpyDeviceToHost, w->stream()));
+    const OutPlanes o = slice_planes(w, m, i);
     running = 0;
-    for (int mb = 0; mb < nw; ++mb) {
+    for (int mb = 0; mb < R.nw; ++mb) {
         if (delivered_stop[mb]) continue;
+        // the view and the member's control block in one go
+        QP_TRY(stage_slice(w, member_planes(w, mb, o), w->ctl + mb, &hc[mb]));
         if (hc[mb].stop_acc) {
-            QP_TRY(deliver_member(w, cb, user, mb, hc[mb].stop_slice, QP_SLICE_STOPPED, nullptr, nullptr, nullptr,
-                                  nullptr, nullptr, nullptr, nullptr, nullptr, w->by, w->bz, w->chi));
+            QP_TRY(deliver_member(w, cb, user, mb, hc[mb].stop_slice, QP_SLICE_STOPPED, stopped_planes(w)));
             delivered_stop[mb] = 1;
             continue;
         }
         ++running;
-        QP_TRY(deliver_member(w, cb, user, mb, i, QP_SLICE_NORMAL, w->psi_b[slot], rho_of(m, i), jx_of(w, m, i),
-                              m->jbuf[1 - slot][0], m->jbuf[1 - slot][1], w->ex, w->ey, w->ez, w->by, w->bz, w->chi,
-                              p.longitudinal_b ? w->bx : nullptr));
+        QP_TRY(call_member(w, cb, user, mb, i, QP_SLICE_NORMAL, o.p[kOutPlanes - 1] != nullptr));
     }
     return QP_OK;
 }
@@ -1906,25 +1908,24 @@ int pass_finish(Wake *w, MxRun &R, batch_cb cb, void *user, int i_end, std::vect
         w->win_blocks[mb] = launches * (long long)((w->mem[mb].np + R.pt - 1) / R.pt);
         w->win_ovf[mb] = hc[mb].ovf;
         if (stopped && cb && !delivered_stop[mb]) {
-            QP_TRY(deliver_member(w, cb, user, mb, hc[mb].stop_slice, QP_SLICE_STOPPED, nullptr, nullptr, nullptr,
-                                  nullptr, nullptr, nullptr, nullptr, nullptr, w->by, w->bz, w->chi));
+            QP_TRY(deliver_member(w, cb, user, mb, hc[mb].stop_slice, QP_SLICE_STOPPED, stopped_planes(w)));
         }
         if (cb && i_end == 0) {
-            const int cslot = (stopped ? hc[mb].stop_slice : 0) & 1;
-            // a stopped member's B and chi planes hold the stopped slice: zero planes
-            // instead (zero2 has a zero plane for every member)
-            const double *by0 = stopped ? w->zero2 : w->by;
-            const double *bz0 = stopped ? w->zero2 : w->bz;
-            const double *chi0 = stopped ? w->zero2 : w->chi;
-            const double *bx0 = p.longitudinal_b ? (stopped ? w->zero2 : w->bx) : nullptr;
-            // rho and jx of the last step: a stopped one ended in iteration stop_iter, where
-            // jx is that iteration's and rho the step's own only after its last iteration
-            const int it = hc[mb].stop_iter;
-            const double *rho0 = stopped ? m->rho2[it == p.K - 1 ? cslot : 1 - cslot] : rho_of(m, 0);
-            const double *jx0 = stopped ? m->jx2[it & 1] : jx_of(w, m, 0);
-            QP_TRY(deliver_member(w, cb, user, mb, 0, QP_SLICE_FINAL, w->psi_b[cslot], rho0, jx0,
-                                  m->jbuf[1 - cslot][0], m->jbuf[1 - cslot][1], w->ex, w->ey, w->ez, by0, bz0,
-                                  chi0, bx0));
+            // a stopped member's B and chi planes hold the stopped slice: zero planes instead.
+            // rho and jx are those of the last step: a stopped one ended in iteration stop_iter,
+            // where jx is that iteration's and rho the step's own only after its last iteration
+            const int cslot = (stopped ? hc[mb].stop_slice : 0) & 1, it = hc[mb].stop_iter;
+            OutPlanes o = slice_planes(w, m, 0);
+            o.p[0] = w->psi_b[cslot];
+            o.p[3] = m->jbuf[1 - cslot][0];
+            o.p[4] = m->jbuf[1 - cslot][1];
+            if (stopped) {
+                o.p[1] = m->rho2[it == p.K - 1 ? cslot : 1 - cslot];
+                o.p[2] = m->jx2[it & 1];
+                o.p[8] = o.p[9] = o.p[10] = w->zero2;  // a zero plane for every member
+                if (p.longitudinal_b) o.p[11] = w->zero2;
+            }
+            QP_TRY(deliver_member(w, cb, user, mb, 0, QP_SLICE_FINAL, o));
         }
         if (stop_slices) stop_slices[mb] = stopped ? hc[mb].stop_slice : -1;
     }
