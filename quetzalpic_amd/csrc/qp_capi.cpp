@@ -111,8 +111,7 @@ int qp_fourier2d_forward(qp_fourier2d f, const double *in_real, double *out_comp
     hipStream_t s = f->ctx->stream;
     const Solver2d &S = f->S;
     QP_HIP_CHECK(hipMemcpyAsync(f->d_buf, in_real, sizeof(double) * S.n1 * S.n2, hipMemcpyHostToDevice, s));
-    QP_TRY(fourier_rows_fwd(S, f->d_buf, S.spec[0], s));
-    QP_TRY(solve_cols_forward_only(S, s));
+    QP_TRY(fourier_forward(S, f->d_buf, S.spec[0], s));
     QP_HIP_CHECK(hipMemcpyAsync(out_complex, S.spec[0], sizeof(double2) * S.n1 * S.nh, hipMemcpyDeviceToHost, s));
     QP_HIP_CHECK(hipStreamSynchronize(s));
     return QP_OK;
@@ -123,8 +122,7 @@ int qp_fourier2d_backward(qp_fourier2d f, const double *in_complex, double *out_
     hipStream_t s = f->ctx->stream;
     const Solver2d &S = f->S;
     QP_HIP_CHECK(hipMemcpyAsync(S.spec[0], in_complex, sizeof(double2) * S.n1 * S.nh, hipMemcpyHostToDevice, s));
-    QP_TRY(solve_cols_inverse_only(S, s));
-    QP_TRY(fourier_rows_inv(S, S.spec[0], f->d_buf, s));
+    QP_TRY(fourier_backward(S, S.spec[0], f->d_buf, s));
     QP_HIP_CHECK(hipMemcpyAsync(out_real, f->d_buf, sizeof(double) * S.n1 * S.n2, hipMemcpyDeviceToHost, s));
     QP_HIP_CHECK(hipStreamSynchronize(s));
     return QP_OK;
@@ -542,8 +540,7 @@ int qp_wake_describe(qp_wake h, char *buf, size_t len) {
     std::string s = "{\"members\": " + std::to_string(w->nw) +
                     ", \"tile\": [" + std::to_string(w->tile_pt) + ", " + std::to_string(w->tile_cap) + "]" +
                     ", \"tile_tuned\": " + (w->tile_tuned ? "1" : "0") + ", \"tiles\": " + mixed_tiles_json() +
-                    ", \"rows_per_block\": " + std::to_string(w->S.rows_per_block) +
-                    ", \"cols_per_block\": " + std::to_string(w->S.cols_per_block) +
+                    ", \"rows_per_block\": 1, \"cols_per_block\": 1" +  // (generic kernels)
                     ", \"precision\": " + std::to_string(w->p.precision) +
                     ", \"fft\": \"" + (w->S.wave ? "wave" : "generic") + "\"" +
                     ", \"envelope\": " + (w->env ? "1" : "0") + ", \"bunch\": " + (w->bunch ? "1" : "0") + "}";
@@ -590,10 +587,6 @@ int wake_alloc_common(Wake *w) {
     QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * (nn * kOutPlanes + kCtlWords), hipHostMallocDefault));
     QP_HIP_CHECK(hipEventCreate(&w->ev0));
     QP_HIP_CHECK(hipEventCreate(&w->ev1));
-    if (p.precision == QP_PREC_MIXED) {
-        QP_TRY(w->S.autotune(w->stream(), w->src));
-        QP_HIP_CHECK(hipStreamSynchronize(w->stream()));
-    }
     return QP_OK;
 }
 

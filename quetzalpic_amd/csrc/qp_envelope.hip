@@ -103,7 +103,7 @@ struct SrcEnv {
     int nx, n1, n2, use_dcur;
     double idy2, idz2, dt, c2dx;
     int e;
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void row(int, int which, int j, int k0, int dk, double (&v)[E]) const {
         const double *ac = a + (size_t)which * vol + (size_t)e * nn;
         const double *r0 = ac + (size_t)j * n2;
@@ -114,7 +114,7 @@ struct SrcEnv {
         double c[E], cp[E], cm[E], kp[E], km[E], x[E], dp[E], dc[E], mid = 0.0;
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-            const int k = k0 + dk * r;
+            const int k = row_k<TAIL>(k0 + dk * r, n2);
             c[r] = r0[k];
             cp[r] = rp[k];
             cm[r] = rm[k];
@@ -125,12 +125,12 @@ struct SrcEnv {
         }
         if (e != nx - 1) {
 #pragma unroll
-            for (int r = 0; r < E; ++r) dp[r] = ip[k0 + dk * r];
+            for (int r = 0; r < E; ++r) dp[r] = ip[row_k<TAIL>(k0 + dk * r, n2)];
         }
         if (use_dcur) {
             mid = cmid[e];
 #pragma unroll
-            for (int r = 0; r < E; ++r) dc[r] = ic[k0 + dk * r];
+            for (int r = 0; r < E; ++r) dc[r] = ic[row_k<TAIL>(k0 + dk * r, n2)];
         }
 #pragma unroll
         for (int r = 0; r < E; ++r) {
@@ -141,7 +141,7 @@ struct SrcEnv {
             v[r] = u;
         }
     }
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void done(int, int, int, int, int) const {}
 };
 
@@ -214,18 +214,58 @@ __global__ __launch_bounds__(TB) void kw_cols_env(double2 *spec0, double2 *spec1
     }
 }
 
-// Generic path: the multiplier between the forward-only and inverse-only
-// column passes, on the row-major spectra spec[j * nh + l].
-__global__ void k_env_mix(double2 *spec0, double2 *spec1, int n1, int nh, const double *lam1, const double *lam2,
-                          double ar, double ai, double hdt, const double *cmid) {
-    const size_t n = (size_t)n1 * nh;
-    const double c = *cmid;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
-        const int j = (int)(t / nh), l = (int)(t - (size_t)j * nh);
-        double2 X = spec0[t], Y = spec1[t];
-        env_mix(X, Y, lam1[j] + lam2[l] - c, ar, ai, hdt);
-        spec0[t] = X;
-        spec1[t] = Y;
+// The same on the LDS transforms: one block per column l, both spectra.
+template <bool ONE>
+__global__ __launch_bounds__(kGenThreads) void kg_cols_env(double2 *spec0, double2 *spec1, int n1, FftAxisDev ax,
+                                                           const double *lam1, const double *lam2, double ar, double ai,
+                                                           double hdt, const double *cmid) {
+    extern __shared__ double2 lds[];
+    constexpr int E = 4;  // n1 <= E threads
+    const int l = blockIdx.x, T = blockDim.x;
+    double2 *a = lds, *b = lds + 2 * n1, *twl = lds + 4 * n1;
+    LdsTw tw;
+    tw.load(ax);
+    double2 *c0 = spec0 + (size_t)l * n1, *c1 = spec1 + (size_t)l * n1;
+    double2 x[E], y[E];
+    double lm[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int t = min((int)threadIdx.x + r * T, n1 - 1);
+        x[r] = c0[t];
+        y[r] = c1[t];
+        lm[r] = lam1[t];
+    }
+    const double l2 = lam2[l] - *cmid;
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int t = threadIdx.x + r * T;
+        if (t < n1) {
+            a[t] = x[r];
+            a[n1 + t] = y[r];
+        }
+    }
+    tw.store(twl, n1);
+    lds_sync<ONE>();
+    double2 *z = lds_fft<ONE, 2>(a, b, ax, twl);
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int t = threadIdx.x + r * T;
+        if (t < n1) {
+            double2 X = z[t], Y = z[n1 + t];
+            env_mix(X, Y, lm[r] + l2, ar, ai, hdt);
+            z[t] = swap_parts(X);  // forward again for the inverse
+            z[n1 + t] = swap_parts(Y);
+        }
+    }
+    lds_sync<ONE>();
+    const double2 *o = lds_fft<ONE, 2>(z, z == a ? b : a, ax, twl);
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int t = threadIdx.x + r * T;
+        if (t < n1) {
+            c0[t] = swap_parts(o[t]);
+            c1[t] = swap_parts(o[n1 + t]);
+        }
     }
 }
 
@@ -266,16 +306,16 @@ int env_transform(Envelope *e, int i, double dt, bool use_dcur, bool last, hipSt
                                 (const Ctl *)nullptr, 0));
         return QP_OK;
     }
-    ELAUNCH(k_rows_fwd<SrcEnv>, dim3(rows_blocks(S), 2), kSolverThreads, rows_lds(S), src, S.spec[0], S.spec[1],
-            S.n1, S.n2, S.nh, S.ax2.dev, S.rows_per_block, (const Ctl *)nullptr, 0, 2, (size_t)0);
-    QP_TRY(solve_cols_pass(S, 2, 0, s));
-    ELAUNCH(k_env_mix, dim3(eblk((size_t)S.n1 * S.nh)), kET, 0, S.spec[0], S.spec[1], S.n1, S.nh,
-            (const double *)S.d_lam1, (const double *)S.d_lam2, ar, ai, hdt, cmid);
-    QP_TRY(solve_cols_pass(S, 2, 1, s));
-    ELAUNCH(k_rows_inv<SinkEnv>, dim3(rows_blocks(S), 2), kSolverThreads, rows_lds(S), (const double2 *)S.spec[0],
-            (const double2 *)S.spec[1], snk, S.n1, S.n2, S.nh, S.ax2.dev, S.rows_per_block, (const Ctl *)nullptr, 0,
-            2, (size_t)0);
-    return QP_OK;
+    QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, (const Ctl *)nullptr, 0));
+    const int threads = S.ax1.dev.threads;
+    const size_t lds = sizeof(double2) * 5 * (size_t)S.n1;
+    if (threads == 64)
+        ELAUNCH(kg_cols_env<true>, dim3(S.nh), threads, lds, S.spec[0], S.spec[1], S.n1, S.ax1.dev,
+                (const double *)S.d_lam1, (const double *)S.d_lam2, ar, ai, hdt, cmid);
+    else
+        ELAUNCH(kg_cols_env<false>, dim3(S.nh), threads, lds, S.spec[0], S.spec[1], S.n1, S.ax1.dev,
+                (const double *)S.d_lam1, (const double *)S.d_lam2, ar, ai, hdt, cmid);
+    return glaunch_rows_inv(S, (const double2 *)S.spec[0], (const double2 *)S.spec[1], snk, 2, s, (const Ctl *)nullptr, 0);
 }
 
 // One step of the whole envelope (every slice, then <a^2>); m corrections of

@@ -28,7 +28,7 @@ void set_error(const std::string &msg);
     } while (0)
 
 // ------------------------------------------------------------ FFT plan
-constexpr int kMaxStages = 24;
+constexpr int kMaxStages = 12;
 constexpr int kMaxN = 1024;          // longest transform the LDS kernels take
 constexpr int kLdsComplex = 1024;    // complex doubles per LDS data buffer (16 KiB; two buffers)
 
@@ -36,7 +36,13 @@ constexpr int kLdsComplex = 1024;    // complex doubles per LDS data buffer (16 
 struct FftAxisDev {
     int n;
     int nstages;
-    int radix[kMaxStages];
+    int threads;  // per block of the generic kernels
+    // per stage: radix R, n / R, n / (Ns R), division factor (quot) of Ns; one entry more
+    // than stages, so that the next stage's can be loaded ahead
+    struct Stage {
+        int R, nR, tws;
+        unsigned fns;
+    } st[kMaxStages + 1];
     const double2 *tw;  // e^{-2 pi i t / n}, t in [0, n)
 };
 
@@ -57,16 +63,13 @@ struct Solver2d {
     double *d_lam2 = nullptr;  // (2cos(2 pi k/n2) - 2)/d2/d2
     double2 *spec[2] = {nullptr, nullptr};  // n1 x nh half spectra (two for paired solves), nbatch each
     int nbatch = 1;                           // wakes sharing this solver (spectra side by side)
-    int rows_per_block = 1;   // complex row transforms (= 2 real rows) per block
-    int cols_per_block = 1;
-    // 1: both sides 2^p in [16, 1024] -> register-resident FFT kernels with the
-    // column-major spectrum spec[l * n1 + j]; 0: generic kernels, row-major
-    // spec[j * nh + l] (FFTW's r2c layout).  Fourier2d always uses the latter.
+    // 1: both sides of a register-resident length (wf_length); 0: generic kernels.  Both
+    // keep the half spectrum column-major, spec[l * n1 + j]; Fourier2d's transforms use
+    // the generic kernels on FFTW's row-major layout, spec[j * nh + l].
     int wave = 0;
     int init(int n1, int n2, double d1, double d2, int nbatch = 1);
-    void default_shape();  // wave / rows_per_block / cols_per_block from n1, n2
+    void pick_kernels();   // wave from n1, n2
     int set_steps(double d1, double d2);
-    int autotune(hipStream_t s, double *scratch_real);
     void destroy();
 };
 
@@ -208,24 +211,14 @@ __device__ __forceinline__ void wrap_coords(double &y, double &z, double ly, dou
 // All launches go to `s`.  `src_fn` kinds select what the row-forward pass reads.
 int solve_rows_fwd_plain(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);
 int solve_cols(const Solver2d &S, double D, int nspec, hipStream_t s, const Ctl *ctl, int skip_mode);
-// Column pass of nw wakes side by side (spectra at + wake * n1 * nh, control blocks at ctl + wake).
-int solve_cols_batch(const Solver2d &S, double D, int nspec, int nw, hipStream_t s, const Ctl *ctl,
-                     int skip_mode);
 int solve_rows_inv_plain(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
 // Plain-path B solve epilogue: store v/n1/n2 and flag |B| > thr or NaN.
 int solve_rows_inv_bcheck(const Solver2d &S, const double2 *spec, double *dst, double thr, Ctl *ctl,
                           int slice, hipStream_t s);
-size_t rows_lds(const Solver2d &S);
-size_t cols_lds(const Solver2d &S);
-int rows_blocks(const Solver2d &S);
-int solve_cols_forward_only(const Solver2d &S, hipStream_t s);
-int solve_cols_inverse_only(const Solver2d &S, hipStream_t s);
-// Generic kernels only: column transforms of nspec spectra, mode 0 forward, 1 inverse.
-int solve_cols_pass(const Solver2d &S, int nspec, int mode, hipStream_t s);
 int solve_rows_inv_unscaled(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
 // Fourier2d transforms in FFTW's layout (generic kernels whatever S.wave says).
-int fourier_rows_fwd(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);
-int fourier_rows_inv(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
+int fourier_forward(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);
+int fourier_backward(const Solver2d &S, double2 *spec, double *dst, hipStream_t s);
 int solve_rows_fwd_plain_ctl(const Solver2d &S, const double *src, double2 *spec, hipStream_t s,
                              const Ctl *ctl, int skip_mode);
 int solve_rows_inv_plain_ctl(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s,

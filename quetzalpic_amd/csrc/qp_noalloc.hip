@@ -119,7 +119,7 @@ extern "C" int qp_solve2d_device_noalloc(qp_ctx ctx, int n1, int n2, double d1, 
     S.d_lam2 = lam2;
     S.spec[0] = base;
     S.spec[1] = base;   // single solves use spectrum 0 only
-    S.default_shape();
+    S.pick_kernels();
     const int nt = n1 > n2 ? n1 : n2;
     hipLaunchKernelGGL(k_noalloc_tables, dim3((nt + 255) / 256), dim3(256), 0, s, tw1, n1, tw2, n2, lam1, lam2,
                        S.nh, d1, d2);

@@ -554,32 +554,35 @@ struct SrcPsi {
     const Ctl *ctl;
     int slot, n2;
     size_t nn;
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void row(int wk, int, int j, int k0, int dk, double (&x)[E]) const {
-        const size_t t = (size_t)j * n2 + k0, tw = (size_t)wk * nn + t;
+        const size_t t = (size_t)j * n2, tw = (size_t)wk * nn + t;
         double io[E], jb[E], rb[E];
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-            x[r] = acc[tw + dk * r];
-            io[r] = rho_ion[tw + dk * r];
+            const int k = row_k<TAIL>(k0 + dk * r, n2);
+            x[r] = acc[tw + k];
+            io[r] = rho_ion[tw + k];
             jb[r] = rb[r] = 0.0;
         }
         if (jx_b3 || rho_b3) {
             const size_t o = (size_t)ctl[wk].slice_of[slot] * bstride + t;
 #pragma unroll
             for (int r = 0; r < E; ++r) {
-                if (jx_b3) jb[r] = jx_b3[o + dk * r];
-                if (rho_b3) rb[r] = rho_b3[o + dk * r];
+                const int k = row_k<TAIL>(k0 + dk * r, n2);
+                if (jx_b3) jb[r] = jx_b3[o + k];
+                if (rho_b3) rb[r] = rho_b3[o + k];
             }
         }
 #pragma unroll
         for (int r = 0; r < E; ++r) x[r] = (jb[r] - rb[r] - io[r]) + x[r];
     }
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void done(int wk, int, int j, int k0, int dk) const {
-        const size_t tw = (size_t)wk * nn + (size_t)j * n2 + k0;
+        const size_t tw = (size_t)wk * nn + (size_t)j * n2;
 #pragma unroll
-        for (int r = 0; r < E; ++r) acc[tw + dk * r] = 0.0;
+        for (int r = 0; r < E; ++r)
+            if (!TAIL || k0 + dk * r < n2) acc[tw + k0 + dk * r] = 0.0;
     }
 };
 
@@ -588,14 +591,14 @@ struct SrcB {
     const double *by, *bz, *jx, *jy, *jz, *jyn, *jzn;
     int n1, n2;
     double D, inv_dx, inv_dy, inv_dz;  // the differences are scaled by reciprocals (no divisions)
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void row(int wk, int which, int j, int k0, int dk, double (&x)[E]) const {
         const size_t go = (size_t)wk * n1 * n2, rj = go + (size_t)j * n2;
         double b[E], jc[E], jn[E], ja[E], jb[E];
         if (which == 0) {
 #pragma unroll
             for (int r = 0; r < E; ++r) {
-                const int k = k0 + dk * r;
+                const int k = row_k<TAIL>(k0 + dk * r, n2);
                 b[r] = by[rj + k];
                 jc[r] = jx[rj + k];
                 jn[r] = jx[rj + (k < n2 - 1 ? k + 1 : 0)];
@@ -613,7 +616,7 @@ struct SrcB {
         const size_t rn = j < n1 - 1 ? rj + n2 : go, rb = j < n1 - 1 ? rj : go;
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-            const int k = k0 + dk * r;
+            const int k = row_k<TAIL>(k0 + dk * r, n2);
             b[r] = bz[rb + k];
             jc[r] = jx[rj + k];
             jn[r] = jx[rn + k];
@@ -626,7 +629,7 @@ struct SrcB {
             x[r] = -D * b[r] + (jn[r] - jc[r]) * inv_dy - djy;
         }
     }
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void done(int, int, int, int, int) const {}
 };
 
@@ -701,13 +704,13 @@ struct SrcCurl {
     const double *jy, *jz;
     int n1, n2;
     double inv_dy, inv_dz;
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void row(int wk, int, int j, int k0, int dk, double (&x)[E]) const {
         const size_t go = (size_t)wk * n1 * n2, rj = go + (size_t)j * n2, rn = go + (size_t)(j + 1 == n1 ? 0 : j + 1) * n2;
         double yc[E], yn[E], zc[E], zn[E];
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-            const int k = k0 + dk * r;
+            const int k = row_k<TAIL>(k0 + dk * r, n2);
             yc[r] = jy[rj + k];
             yn[r] = jy[rj + (k + 1 == n2 ? 0 : k + 1)];
             zc[r] = jz[rj + k];
@@ -716,7 +719,7 @@ struct SrcCurl {
 #pragma unroll
         for (int r = 0; r < E; ++r) x[r] = (yn[r] - yc[r]) * inv_dz - (zn[r] - zc[r]) * inv_dy;
     }
-    template <int E>
+    template <int E, bool TAIL = false>
     __device__ void done(int, int, int, int, int) const {}
 };
 
@@ -730,69 +733,6 @@ struct SinkMember {
         dst[(size_t)wk * n1 * n2 + (size_t)j * n2 + k] = v * scale;
     }
 };
-
-// Column pass of the psi solves, with the partial sums the border mean needs:
-// after the inverse column transform G[j][l], the c2r row value at k = 0 is
-// sum_l c_l Re G[j][l] (c_0 = c_{n2/2} = 1, else 2) and sum_k x[0][k] = n2 Re G[0][0].
-// blockIdx.y is the member (spectra at + member * sstride, partial sums at +
-// member * bstride).
-__global__ __launch_bounds__(kSolverThreads) void k_cols_psi(double2 *spec, int n1, int nh, int n2, FftAxisDev ax,
-                                                             const double *lam1, const double *lam2, int C,
-                                                             double *bpart, const Ctl *ctl, size_t sstride,
-                                                             size_t bstride) {
-    const int wk = blockIdx.y;
-    if (solver_skip(ctl + wk, 1)) return;
-    spec += wk * sstride;
-    bpart += wk * bstride;
-    extern __shared__ double2 lds2[];
-    double2 *a = lds2, *b = lds2 + (size_t)C * n1, *twl = lds2 + (size_t)2 * C * n1;
-    double *lam1l = reinterpret_cast<double *>(twl + n1);
-    const int l0 = blockIdx.x * C;
-    lds_load_tw(twl, ax);
-    for (int t = threadIdx.x; t < n1; t += blockDim.x) lam1l[t] = lam1[t];
-    for (int t = threadIdx.x; t < C * n1; t += blockDim.x) {
-        const int c = t % C, j = t / C, l = l0 + c;
-        a[c * n1 + j] = l < nh ? spec[(size_t)j * nh + l] : make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-    double2 *r = lds_fft(a, b, C, ax, twl, -1);
-    for (int t = threadIdx.x; t < C * n1; t += blockDim.x) {
-        const int c = t / n1, m = t - c * n1, l = l0 + c;
-        if (l >= nh) continue;
-        double2 v = r[t];
-        if (m == 0 && l == 0) {
-            v = make_double2(0.0, 0.0);
-        } else {
-            const double mult = -0.0 + lam1l[m] + lam2[l];
-            v.x /= mult;
-            v.y /= mult;
-        }
-        r[t] = v;
-    }
-    __syncthreads();
-    double2 *o = lds_fft(r, r == a ? b : a, C, ax, twl, +1);
-    for (int t = threadIdx.x; t < C * n1; t += blockDim.x) {
-        const int c = t % C, j = t / C, l = l0 + c;
-        if (l < nh) spec[(size_t)j * nh + l] = o[c * n1 + j];
-    }
-    // partial sums over the whole block: sum_c w_l sum_j Re G[j][l] and sum_c w_l Re G[0][l]
-    double s1 = 0.0, s2 = 0.0;
-    for (int t = threadIdx.x; t < C * n1; t += blockDim.x) {
-        const int c = t / n1, j = t - c * n1, l = l0 + c;
-        if (l >= nh) continue;
-        const double wl = (l == 0 || 2 * l == n2) ? 1.0 : 2.0;
-        const double v = wl * o[t].x;
-        s1 += v;
-        if (j == 0) s2 += v;
-    }
-    s1 = block_sum(s1);
-    s2 = block_sum(s2);
-    if (threadIdx.x == 0) {
-        bpart[2 * blockIdx.x] = s1;
-        bpart[2 * blockIdx.x + 1] = s2;
-        if (blockIdx.x == 0) bpart[2 * gridDim.x] = o[0].x;
-    }
-}
 
 // ------------------------------------------------------------ re-binning
 // Counting sort of the particles by cell, the cells taken 16x16 tile by tile
@@ -1211,11 +1151,7 @@ static int ensure_state(Wake *w) {
         m = new MixedState();
         w->mixed = m;
         const int ncb = w->S.wave ? wcols_blocks(w->S.n1, w->S.nh)
-                                  : (w->S.nh + w->S.cols_per_block - 1) / w->S.cols_per_block;
-        if (w->S.cols_per_block > 64) {
-            set_error("column block too wide for the border partial sums");
-            return QP_ERR_STATE;
-        }
+                                  : w->S.nh;
         m->ncb = ncb;
         m->bstride = 2 * (size_t)ncb + 2;
         QP_HIP_CHECK(hipMalloc(&m->bpart, sizeof(double) * m->bstride * nw));
@@ -1455,18 +1391,14 @@ int psi_solve(MxRun &R, hipStream_t s, int slot, double *dst) {
         return QP_OK;
     }
     prof_begin(w, "solve");
-    MLAUNCH(k_rows_fwd<SrcPsi>, dim3(rows_blocks(S), nw), kSolverThreads, rows_lds(S), src, S.spec[0], S.spec[0],
-            S.n1, S.n2, S.nh, S.ax2.dev, S.rows_per_block, (const Ctl *)w->ctl, 1, 1, R.sstride);
+    QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[0], 1, s, (const Ctl *)w->ctl, 1, nw));
     prof_end(w, "solve");
     prof_begin(w, "solve");
-    MLAUNCH(k_cols_psi, dim3(m->ncb, nw), kSolverThreads, cols_lds(S), S.spec[0], S.n1, S.nh, S.n2, S.ax1.dev,
-            (const double *)S.d_lam1, (const double *)S.d_lam2, S.cols_per_block, m->bpart, (const Ctl *)w->ctl,
-            R.sstride, m->bstride);
+    QP_TRY(glaunch_cols(S, kColsSolve, 0.0, 1, m->bpart, s, (const Ctl *)w->ctl, 1, nw, m->bstride));
     prof_end(w, "solve");
     prof_begin(w, "solve");
-    MLAUNCH(k_rows_inv<SinkPsiFinal>, dim3(rows_blocks(S), nw), kSolverThreads, rows_lds(S),
-            (const double2 *)S.spec[0], (const double2 *)S.spec[0], snk, S.n1, S.n2, S.nh, S.ax2.dev,
-            S.rows_per_block, (const Ctl *)w->ctl, 1, 1, R.sstride);
+    QP_TRY(glaunch_rows_inv(S, (const double2 *)S.spec[0], (const double2 *)S.spec[0], snk, 1, s, (const Ctl *)w->ctl, 1,
+                            nw));
     prof_end(w, "solve");
     return QP_OK;
 }
@@ -1495,16 +1427,14 @@ int b_solve(MxRun &R, hipStream_t s, int slot, const double *jx) {
         return QP_OK;
     }
     prof_begin(w, "solve");
-    MLAUNCH(k_rows_fwd<SrcB>, dim3(rows_blocks(S), 2 * nw), kSolverThreads, rows_lds(S), src, S.spec[0], S.spec[1],
-            S.n1, S.n2, S.nh, S.ax2.dev, S.rows_per_block, (const Ctl *)w->ctl, 2, 2, R.sstride);
+    QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, (const Ctl *)w->ctl, 2, nw));
     prof_end(w, "solve");
     prof_begin(w, "solve");
-    QP_TRY(solve_cols_batch(S, p.D, 2, nw, s, w->ctl, 2));
+    QP_TRY(glaunch_cols(S, kColsSolve, p.D, 2, nullptr, s, (const Ctl *)w->ctl, 2, nw));
     prof_end(w, "solve");
     prof_begin(w, "solve");
-    MLAUNCH(k_rows_inv<SinkBPair>, dim3(rows_blocks(S), 2 * nw), kSolverThreads, rows_lds(S),
-            (const double2 *)S.spec[0], (const double2 *)S.spec[1], snk, S.n1, S.n2, S.nh, S.ax2.dev,
-            S.rows_per_block, (const Ctl *)w->ctl, 2, 2, R.sstride);
+    QP_TRY(glaunch_rows_inv(S, (const double2 *)S.spec[0], (const double2 *)S.spec[1], snk, 2, s, (const Ctl *)w->ctl, 2,
+                            nw));
     prof_end(w, "solve");
     return QP_OK;
 }
@@ -1525,13 +1455,10 @@ int bx_solve(MxRun &R, hipStream_t s, int slot) {
                                 (const Ctl *)w->ctl, 1, nw));
         return QP_OK;
     }
-    MLAUNCH(k_rows_fwd<SrcCurl>, dim3(rows_blocks(S), nw), kSolverThreads, rows_lds(S), src, S.spec[0], S.spec[0],
-            S.n1, S.n2, S.nh, S.ax2.dev, S.rows_per_block, (const Ctl *)w->ctl, 1, 1, R.sstride);
-    QP_TRY(solve_cols_batch(S, 0.0, 1, nw, s, w->ctl, 1));
-    MLAUNCH(k_rows_inv<SinkMember>, dim3(rows_blocks(S), nw), kSolverThreads, rows_lds(S),
-            (const double2 *)S.spec[0], (const double2 *)S.spec[0], snk, S.n1, S.n2, S.nh, S.ax2.dev,
-            S.rows_per_block, (const Ctl *)w->ctl, 1, 1, R.sstride);
-    return QP_OK;
+    QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[0], 1, s, (const Ctl *)w->ctl, 1, nw));
+    QP_TRY(glaunch_cols(S, kColsSolve, 0.0, 1, nullptr, s, (const Ctl *)w->ctl, 1, nw));
+    return glaunch_rows_inv(S, (const double2 *)S.spec[0], (const double2 *)S.spec[0], snk, 1, s, (const Ctl *)w->ctl, 1,
+                            nw);
 }
 
 // Enqueue the work of slice i (everything between two output steps) for every member.

@@ -94,6 +94,18 @@ constexpr double cos12(int m) {
 }
 constexpr double sin12(int m) { return cos12(m - 3); }
 
+// cos / sin of 2 pi m / R, m in [0, R/2], R = 5 and 7.
+constexpr double cos_odd(int R, int m) {
+    if (m == 0) return 1.0;
+    if (R == 5) return m == 1 ? 0.30901699437494742410 : -0.80901699437494742410;
+    return m == 1 ? 0.62348980185873353053 : m == 2 ? -0.22252093395631440429 : -0.90096886790241912624;
+}
+constexpr double sin_odd(int R, int m) {
+    if (m == 0) return 0.0;
+    if (R == 5) return m == 1 ? 0.95105651629515357212 : 0.58778525229247312917;
+    return m == 1 ? 0.78183148246802980871 : m == 2 ? 0.97492791218182360702 : 0.43388373911755812048;
+}
+
 // (S i) * a
 template <int S>
 __device__ __forceinline__ double2 mul_si(double2 a) {
@@ -160,7 +172,40 @@ __device__ __forceinline__ void dft4(double2 &v0, double2 &v1, double2 &v2, doub
     v3 = csub(t1, t3);
 }
 
-// In-register DFT of length R in {1, 2, 3, 4, 6, 8, 12, 16}: u[q] <- sum_r u[r] e^{S 2 pi i r q / R}.
+// Length R = 5 or 7: with p_r = u_r + u_{R-r}, m_r = u_r - u_{R-r} the outputs q and
+// R - q are u_0 + sum_r cos(2 pi r q / R) p_r +- S i sum_r sin(2 pi r q / R) m_r.
+template <int R, int S>
+__device__ __forceinline__ void dft_odd(double2 (&u)[R]) {
+    constexpr int H = (R - 1) / 2;
+    double2 p[H], m[H], o[R];
+    o[0] = u[0];
+#pragma unroll
+    for (int r = 1; r <= H; ++r) {
+        p[r - 1] = cadd(u[r], u[R - r]);
+        m[r - 1] = csub(u[r], u[R - r]);
+        o[0] = cadd(o[0], p[r - 1]);
+    }
+#pragma unroll
+    for (int q = 1; q <= H; ++q) {
+        double2 c = u[0], d = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+            const int e = (r * q) % R;
+            const double cs = cos_odd(R, e <= H ? e : R - e), sn = e <= H ? sin_odd(R, e) : -sin_odd(R, R - e);
+            c.x += cs * p[r - 1].x;
+            c.y += cs * p[r - 1].y;
+            d.x += sn * m[r - 1].x;
+            d.y += sn * m[r - 1].y;
+        }
+        d = mul_si<S>(d);
+        o[q] = cadd(c, d);
+        o[R - q] = csub(c, d);
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) u[q] = o[q];
+}
+
+// In-register DFT of length R in {1, ..., 8, 12, 16}: u[q] <- sum_r u[r] e^{S 2 pi i r q / R}.
 // Radix 8 and 16 split as r = r1 + (R/4 or 4) r2 with internal twiddles; radix
 // 12 as r = r1 + 4 r2, q = q2 + 3 q1: length-3 DFTs over r2, twiddles
 // e^{S 2 pi i r1 q2 / 12}, length-4 DFTs over r1; radix 6 the same way with
@@ -169,6 +214,8 @@ template <int R, int S>
 __device__ __forceinline__ void dft(double2 (&u)[R]) {
     if constexpr (R == 3) {
         dft3<S>(u[0], u[1], u[2]);
+    } else if constexpr (R == 5 || R == 7) {
+        dft_odd<R, S>(u);
     } else if constexpr (R == 6) {
         double2 a0 = u[0], a1 = u[2], a2 = u[4], b0 = u[1], b1 = u[3], b2 = u[5];
         dft3<S>(a0, a1, a2);
