@@ -576,7 +576,7 @@ int wake_alloc_common(Wake *w) {
     QP_HIP_CHECK(hipMalloc(&w->g_base, sizeof(double) * nn * nw * ngrids));
     QP_HIP_CHECK(hipMemset(w->g_base, 0, sizeof(double) * nn * nw * ngrids));
     double **grids[] = {&w->src, &w->psi, &w->psi_prev, &w->psim, &w->rho, &w->jx, &w->jy, &w->jz, &w->jyn,
-                        &w->jzn, &w->djy, &w->djz, &w->rho_ion, &w->by, &w->bz, &w->chi, &w->ex, &w->ey,
+                        &w->jzn, &w->rho_ion, &w->by, &w->bz, &w->chi, &w->ex, &w->ey,
                         &w->ez, &w->src2, &w->asq2, &w->psi_b[0], &w->psi_b[1], &w->zero2, &w->bx};
     int gi = 0;
     for (double **g : grids) *g = w->g_base + nn * nw * (gi++);
@@ -592,7 +592,7 @@ int wake_alloc_common(Wake *w) {
 
 void wake_free_particles(Wake *w) {
     PartFP64 &P = w->pf;
-    double *arrs[] = {P.y, P.z, P.py, P.pz, P.n, P.gamma, P.px, P.ym, P.zm, P.pyn, P.pzn};
+    double *arrs[] = {P.y, P.z, P.py, P.pz, P.n, P.gamma, P.ym, P.zm, P.pyn, P.pzn};
     for (double *a : arrs)
         if (a) (void)hipFree(a);
     w->pf = PartFP64{};

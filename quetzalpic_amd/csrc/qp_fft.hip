@@ -177,9 +177,4 @@ int solve_rows_inv_plain(const Solver2d &S, const double2 *spec, double *dst, hi
     return solve_rows_inv_plain_ctl(S, spec, dst, s, nullptr);
 }
 
-int solve_rows_inv_bcheck(const Solver2d &S, const double2 *spec, double *dst, double thr, Ctl *ctl, int slice,
-                          hipStream_t s) {
-    return rows_inv(S, spec, SinkBCheck{dst, S.n1, S.n2, thr, ctl, slice}, s, (const Ctl *)ctl, 2);
-}
-
 }  // namespace qp

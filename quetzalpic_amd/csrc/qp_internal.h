@@ -88,7 +88,6 @@ struct Ctl {
     unsigned ovf;      // mixed path: particle blocks whose deposit window exceeded the LDS capacity
     int iter;          // mixed path: predictor-corrector iteration of the slice step (k_mx_B)
     int stop_iter;     // mixed path: the iteration whose B solve tripped the stop rule
-    double border[4];  // plain path: border mean of the last psi solve
 };
 
 __device__ __forceinline__ bool ctl_skip(const Ctl *c) { return c->stop_acc != 0; }
@@ -212,9 +211,6 @@ __device__ __forceinline__ void wrap_coords(double &y, double &z, double ly, dou
 int solve_rows_fwd_plain(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);
 int solve_cols(const Solver2d &S, double D, int nspec, hipStream_t s, const Ctl *ctl, int skip_mode);
 int solve_rows_inv_plain(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
-// Plain-path B solve epilogue: store v/n1/n2 and flag |B| > thr or NaN.
-int solve_rows_inv_bcheck(const Solver2d &S, const double2 *spec, double *dst, double thr, Ctl *ctl,
-                          int slice, hipStream_t s);
 int solve_rows_inv_unscaled(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
 // Fourier2d transforms in FFTW's layout (generic kernels whatever S.wave says).
 int fourier_forward(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);

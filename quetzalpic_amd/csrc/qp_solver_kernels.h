@@ -104,25 +104,6 @@ struct SinkRaw {
     __device__ void operator()(int, int, int j, int k, double v) const { dst[(size_t)j * n2 + k] = v; }
 };
 
-// B store with the stop rule (src/System_3d.cpp:541-552, 569-580).
-struct SinkBCheck {
-    double *dst;
-    int n1, n2;
-    double thr;
-    Ctl *ctl;
-    int slice;
-    __device__ void prep(int) {}
-    __device__ void begin(int) {}
-    __device__ void operator()(int wk, int, int j, int k, double v) const {
-        const double b = v / n1 / n2;
-        dst[(size_t)j * n2 + k] = b;
-        if (fabs(b) > thr || isnan(b)) {
-            ctl[wk].stop_acc = 1;
-            ctl[wk].stop_slice = slice;
-        }
-    }
-};
-
 // ------------------------------------------------ generic kernels (any side up to 1024)
 // Spectrum element (row j, frequency l) at j * sj + l * sl: column-major (sj = 1,
 // sl = n1) for the solves, so that column transforms read and write contiguous

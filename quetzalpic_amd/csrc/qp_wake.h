@@ -19,7 +19,7 @@ struct LaserGauss {
 // (src/containers.h:31-43) as separate device arrays.
 struct PartFP64 {
     double *y = nullptr, *z = nullptr, *py = nullptr, *pz = nullptr, *n = nullptr, *gamma = nullptr,
-           *px = nullptr, *ym = nullptr, *zm = nullptr, *pyn = nullptr, *pzn = nullptr;
+           *ym = nullptr, *zm = nullptr, *pyn = nullptr, *pzn = nullptr;
 };
 
 // Host data of one member of a batch of wakes (a single wake is a batch of
@@ -47,8 +47,8 @@ struct Wake {
     // grids: nw planes of ny*nz FP64 side by side each (member m at + m*ny*nz)
     double *g_base = nullptr;
     double *src = nullptr, *psi = nullptr, *psi_prev = nullptr, *psim = nullptr, *rho = nullptr,
-           *jx = nullptr, *jy = nullptr, *jz = nullptr, *jyn = nullptr, *jzn = nullptr, *djy = nullptr,
-           *djz = nullptr, *rho_ion = nullptr, *by = nullptr, *bz = nullptr, *chi = nullptr, *ex = nullptr,
+           *jx = nullptr, *jy = nullptr, *jz = nullptr, *jyn = nullptr, *jzn = nullptr,
+           *rho_ion = nullptr, *by = nullptr, *bz = nullptr, *chi = nullptr, *ex = nullptr,
            *ey = nullptr, *ez = nullptr, *src2 = nullptr, *asq2 = nullptr, *psi_b[2] = {nullptr, nullptr},
            *zero2 = nullptr, *bx = nullptr;
     // driver inputs (the 3D arrays only for a single wake)
