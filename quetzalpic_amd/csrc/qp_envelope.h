@@ -24,10 +24,13 @@ struct Envelope {
     double *chi3 = nullptr;  // nx * nn: chi of every slice
     double *asq3 = nullptr;  // nx * nn: <a^2> = |a|^2 / 2
     double *cmid = nullptr;  // nx: midrange of chi per slice (set at each advance)
+    int pipe = 0;                    // steps in flight the two buffers below hold (0: none)
+    double *pipe_inc = nullptr;      // as inc, per step
+    double2 *pipe_spec = nullptr;    // spectra of the real parts per step, then of the imaginary parts
     int attached = 0;        // wakes reading this envelope
-    hipGraphExec_t gexec = nullptr;  // one sweep, captured for dtau = g_dtau, g_iter chi corrections
+    hipGraphExec_t gexec = nullptr;  // g_steps steps, captured for dtau = g_dtau, g_iter chi corrections
     double g_dtau = 0.0;
-    int g_iter = 0;
+    int g_iter = 0, g_steps = 0;
     hipStream_t g_stream = nullptr;  // stream the graph was captured on
 
     size_t nn() const { return (size_t)ny * nz; }

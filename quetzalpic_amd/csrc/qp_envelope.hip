@@ -24,6 +24,13 @@
 // spectra), and the last row pass stores d_i (and, after the last transform
 // of the slice, adds it to a_i).  |alpha + (lambda - c_i) dt/2| > 2/dx for
 // every mode, so the sweep over the slices is stable for any dt.
+//
+// Several steps run as one pipeline: step s may take slice i as soon as step s - 1 has
+// left it and step s has left slice i + 1, so at time t the steps s = 0 .. ns - 1 work
+// on the slices nx - 1 - (t - s), each in its own spectra and increments, in one set of
+// launches.  ns steps then take nx + ns - 1 turns of 3 (m + 1) launches instead of
+// ns nx: a lone transform of a 256^2 grid is a chain of latency-bound launches (64-129
+// blocks).  Twelve steps of 256^2 x 100 slices: 35 -> 7.5 ms of launches.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -97,20 +104,21 @@ __global__ __launch_bounds__(kET) void k_env_cmid(const double *chi3, double *cm
 struct SrcEnv {
     const double *a;      // real parts of all slices (imaginary parts at + vol)
     const double *chi;    // chi of all slices
-    const double *inc;    // 2 slots x (re, im) x nn increments
+    const double *inc;    // per step: 2 slots x (re, im) x nn increments
     const double *cmid;   // c of all slices
     size_t vol, nn;
     int nx, n1, n2, use_dcur;
     double idy2, idz2, dt, c2dx;
-    int e;
+    int e0, s0;  // the launch's member wk is step s0 + wk at slice e0 + wk
     template <int E, bool TAIL = false>
-    __device__ void row(int, int which, int j, int k0, int dk, double (&v)[E]) const {
+    __device__ void row(int wk, int which, int j, int k0, int dk, double (&v)[E]) const {
+        const int e = e0 + wk;
         const double *ac = a + (size_t)which * vol + (size_t)e * nn;
         const double *r0 = ac + (size_t)j * n2;
         const double *rm = ac + (size_t)(j == 0 ? n1 - 1 : j - 1) * n2, *rp = ac + (size_t)(j + 1 == n1 ? 0 : j + 1) * n2;
         const double *xr = chi + (size_t)e * nn + (size_t)j * n2;
-        const double *ip = inc + (size_t)((e + 1) & 1) * 2 * nn + (size_t)which * nn + (size_t)j * n2;
-        const double *ic = inc + (size_t)(e & 1) * 2 * nn + (size_t)which * nn + (size_t)j * n2;
+        const double *is = inc + (size_t)(s0 + wk) * 4 * nn + (size_t)which * nn + (size_t)j * n2;
+        const double *ip = is + (size_t)((e + 1) & 1) * 2 * nn, *ic = is + (size_t)(e & 1) * 2 * nn;
         double c[E], cp[E], cm[E], kp[E], km[E], x[E], dp[E], dc[E], mid = 0.0;
 #pragma unroll
         for (int r = 0; r < E; ++r) {
@@ -151,13 +159,14 @@ struct SinkEnv {
     double *a;     // all slices (imaginary parts at + vol); null: store d_e only
     double *inc;
     size_t vol, nn;
-    int n1, n2, e;
+    int n1, n2, e0, s0;
     __device__ void prep(int) {}
     __device__ void begin(int) {}
-    __device__ void operator()(int, int which, int j, int k, double v) const {
+    __device__ void operator()(int wk, int which, int j, int k, double v) const {
+        const int e = e0 + wk;
         const size_t t = (size_t)j * n2 + k;
         const double d = v / n1 / n2;
-        inc[(size_t)(e & 1) * 2 * nn + (size_t)which * nn + t] = d;
+        inc[(size_t)(s0 + wk) * 4 * nn + (size_t)(e & 1) * 2 * nn + (size_t)which * nn + t] = d;
         if (a) a[(size_t)which * vol + (size_t)e * nn + t] += d;
     }
 };
@@ -180,6 +189,10 @@ template <int N1, int E, int TB>
 __global__ __launch_bounds__(TB) void kw_cols_env(double2 *spec0, double2 *spec1, int nh, const double2 *tw1,
                                                   const double *lam1, const double *lam2, double ar, double ai,
                                                   double hdt, const double *cmid) {
+    const int wk = blockIdx.y;  // step of the pipeline
+    cmid += wk;
+    spec0 += (size_t)wk * N1 * nh;
+    spec1 += (size_t)wk * N1 * nh;
     using W = WfShape<N1, E, TB>;
     __shared__ double2 sb0[W::LDS], sb1[W::LDS], twl[WfTw<N1, E, TB>::NL];
     const int tid = threadIdx.x;
@@ -221,7 +234,10 @@ __global__ __launch_bounds__(kGenThreads) void kg_cols_env(double2 *spec0, doubl
                                                            double hdt, const double *cmid) {
     extern __shared__ double2 lds[];
     constexpr int E = 4;  // n1 <= E threads
-    const int l = blockIdx.x, T = blockDim.x;
+    const int l = blockIdx.x, T = blockDim.x, wk = blockIdx.y;
+    cmid += wk;
+    spec0 += (size_t)wk * n1 * gridDim.x;
+    spec1 += (size_t)wk * n1 * gridDim.x;
     double2 *a = lds, *b = lds + 2 * n1, *twl = lds + 4 * n1;
     LdsTw tw;
     tw.load(ax);
@@ -275,13 +291,19 @@ __global__ __launch_bounds__(kGenThreads) void kg_cols_env(double2 *spec0, doubl
         QP_HIP_CHECK(hipGetLastError());                                      \
     } while (0)
 
+void drop_graph(Envelope *e) {
+    if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
+    e->gexec = nullptr;
+}
+
 // One transform per block, as the wake solves' column pass: 256^2 x 1000 slices
 // 36.50 -> 35.3 ms per envelope step, 512^2 x 2000 slices 120.5 -> 114.0 ms.
-int wlaunch_cols_env(const Solver2d &S, double ar, double ai, double hdt, const double *cmid, hipStream_t s) {
+int wlaunch_cols_env(const Solver2d &S, double2 *spec0, double2 *spec1, double ar, double ai, double hdt,
+                     const double *cmid, int ns, hipStream_t s) {
     wf_dispatch(S.n1, [&](auto NC) {
         constexpr int N = decltype(NC)::value, E = WfCfg<N>::E, TB = WfCfg<N>::TBC;
-        const dim3 grid(wcols_blocks_t(S.nh, WfShape<N, E, TB>::T));
-        hipLaunchKernelGGL((kw_cols_env<N, E, TB>), grid, dim3(TB), 0, s, S.spec[0], S.spec[1], S.nh,
+        const dim3 grid(wcols_blocks_t(S.nh, WfShape<N, E, TB>::T), ns);
+        hipLaunchKernelGGL((kw_cols_env<N, E, TB>), grid, dim3(TB), 0, s, spec0, spec1, S.nh,
                            (const double2 *)S.ax1.dev.tw, (const double *)S.d_lam1, (const double *)S.d_lam2, ar,
                            ai, hdt, cmid);
     });
@@ -289,64 +311,86 @@ int wlaunch_cols_env(const Solver2d &S, double ar, double ai, double hdt, const 
     return QP_OK;
 }
 
-// One transform of slice i: d_i from the bracket with the previous iterate
-// (use_dcur) or without it, onto a_i when `last`.
-int env_transform(Envelope *e, int i, double dt, bool use_dcur, bool last, hipStream_t s) {
+// One transform of the steps s0 .. s0 + ns - 1 at the slices e0 .. e0 + ns - 1: each d
+// from the bracket with the previous iterate (use_dcur) or without it, onto a when `last`.
+int env_transform(Envelope *e, int e0, int s0, int ns, double dt, bool use_dcur, bool last, hipStream_t s) {
     const Solver2d &S = e->S;
     const size_t nn = e->nn(), vol = e->vol();
     const double ar = -2.0 / e->dx, ai = 2.0 * e->k0, hdt = 0.5 * dt;
-    SrcEnv src{e->a, e->chi3, e->inc, e->cmid, vol, nn, e->nx, S.n1, S.n2, use_dcur ? 1 : 0,
-               1.0 / (e->dy * e->dy), 1.0 / (e->dz * e->dz), dt, 2.0 / e->dx, i};
-    SinkEnv snk{last ? e->a : nullptr, e->inc, vol, nn, S.n1, S.n2, i};
-    const double *cmid = e->cmid + i;
+    double *inc = e->pipe_inc ? e->pipe_inc : e->inc;
+    double2 *sp0 = e->pipe_spec ? e->pipe_spec : S.spec[0];
+    double2 *sp1 = e->pipe_spec ? e->pipe_spec + (size_t)e->pipe * S.n1 * S.nh : S.spec[1];
+    SrcEnv src{e->a, e->chi3, inc, e->cmid, vol, nn, e->nx, S.n1, S.n2, use_dcur ? 1 : 0,
+               1.0 / (e->dy * e->dy), 1.0 / (e->dz * e->dz), dt, 2.0 / e->dx, e0, s0};
+    SinkEnv snk{last ? e->a : nullptr, inc, vol, nn, S.n1, S.n2, e0, s0};
+    const double *cmid = e->cmid + e0;
+    const Ctl *none = nullptr;
     if (S.wave) {
-        QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, (const Ctl *)nullptr, 0));
-        QP_TRY(wlaunch_cols_env(S, ar, ai, hdt, cmid, s));
-        QP_TRY(wlaunch_rows_inv(S, (const double2 *)S.spec[0], (const double2 *)S.spec[1], snk, 2, s,
-                                (const Ctl *)nullptr, 0));
-        return QP_OK;
+        QP_TRY(wlaunch_rows_fwd(S, src, sp0, sp1, 2, s, none, 0, ns));
+        QP_TRY(wlaunch_cols_env(S, sp0, sp1, ar, ai, hdt, cmid, ns, s));
+        return wlaunch_rows_inv(S, (const double2 *)sp0, (const double2 *)sp1, snk, 2, s, none, 0, ns);
     }
-    QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, (const Ctl *)nullptr, 0));
+    QP_TRY(glaunch_rows_fwd(S, src, sp0, sp1, 2, s, none, 0, ns));
     const int threads = S.ax1.dev.threads;
     const size_t lds = sizeof(double2) * 5 * (size_t)S.n1;
     if (threads == 64)
-        ELAUNCH(kg_cols_env<true>, dim3(S.nh), threads, lds, S.spec[0], S.spec[1], S.n1, S.ax1.dev,
-                (const double *)S.d_lam1, (const double *)S.d_lam2, ar, ai, hdt, cmid);
+        ELAUNCH(kg_cols_env<true>, dim3(S.nh, ns), threads, lds, sp0, sp1, S.n1, S.ax1.dev, (const double *)S.d_lam1,
+                (const double *)S.d_lam2, ar, ai, hdt, cmid);
     else
-        ELAUNCH(kg_cols_env<false>, dim3(S.nh), threads, lds, S.spec[0], S.spec[1], S.n1, S.ax1.dev,
-                (const double *)S.d_lam1, (const double *)S.d_lam2, ar, ai, hdt, cmid);
-    return glaunch_rows_inv(S, (const double2 *)S.spec[0], (const double2 *)S.spec[1], snk, 2, s, (const Ctl *)nullptr, 0);
+        ELAUNCH(kg_cols_env<false>, dim3(S.nh, ns), threads, lds, sp0, sp1, S.n1, S.ax1.dev, (const double *)S.d_lam1,
+                (const double *)S.d_lam2, ar, ai, hdt, cmid);
+    return glaunch_rows_inv(S, (const double2 *)sp0, (const double2 *)sp1, snk, 2, s, none, 0, ns);
 }
 
-// One step of the whole envelope (every slice, then <a^2>); m corrections of
-// the (chi - c) d term per slice.  c_i are set before the first step.
-int env_sweep(Envelope *e, double dt, int m, hipStream_t s) {
+// Steps in flight at once: enough to fill the chip (2^20 nodes), at most 16; 256^2 takes
+// 16, 512^2 four, 1024^2 (whose launches fill it alone) one.
+int pipe_depth(const Envelope *e) {
+    return (int)std::max<size_t>(1, std::min<size_t>(16, ((size_t)1 << 20) / e->nn()));
+}
+
+// Spectra and increments of `depth` steps in flight (kept: 2^20 nodes take 50 MB).
+int ensure_pipe(Envelope *e, int depth) {
+    if (depth <= std::max(1, e->pipe)) return QP_OK;
+    drop_graph(e);
+    QP_HIP_CHECK(hipStreamSynchronize(e->stream()));
+    if (e->pipe_inc) (void)hipFree(e->pipe_inc);
+    if (e->pipe_spec) (void)hipFree(e->pipe_spec);
+    e->pipe_inc = nullptr;
+    e->pipe_spec = nullptr;
+    e->pipe = 0;
+    QP_HIP_CHECK(hipMalloc(&e->pipe_inc, sizeof(double) * 4 * e->nn() * depth));
+    if (hipMalloc(&e->pipe_spec, sizeof(double2) * 2 * (size_t)e->S.n1 * e->S.nh * depth) != hipSuccess) {
+        (void)hipFree(e->pipe_inc);
+        e->pipe_inc = nullptr;
+        set_error("envelope: device allocation failed");
+        return QP_ERR_ALLOC;
+    }
+    e->pipe = depth;
+    return QP_OK;
+}
+
+// ns steps of the whole envelope as one pipeline (every slice, then <a^2>); m corrections
+// of the (chi - c) d term per slice.  c_i are set before the first step.
+int env_sweep(Envelope *e, double dt, int m, int ns, hipStream_t s) {
     const size_t vol = e->vol();
-    for (int i = e->nx - 1; i >= 0; --i)
-        for (int it = 0; it <= m; ++it) QP_TRY(env_transform(e, i, dt, it > 0, it == m, s));
+    const int nx = e->nx;
+    for (int t = 0; t < nx + ns - 1; ++t) {
+        const int s0 = std::max(0, t - nx + 1), s1 = std::min(ns - 1, t);
+        for (int it = 0; it <= m; ++it)
+            QP_TRY(env_transform(e, nx - 1 - t + s0, s0, s1 - s0 + 1, dt, it > 0, it == m, s));
+    }
     ELAUNCH(k_env_asq, dim3(eblk(vol)), kET, 0, (const double *)e->a, e->asq3, vol);
     return QP_OK;
 }
 
-void drop_graph(Envelope *e) {
-    if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
-    e->gexec = nullptr;
-}
-
-}  // namespace
-
-// ------------------------------------------------------- wake-side step
-// One step of the whole envelope after a wake pass, enqueued on s: midranges
-// of chi, then the sweep, replayed from the captured graph of this (dt, m)
-// when use_graph, else launched directly.
-int envelope_step(Envelope *e, double dt, int m, int use_graph, hipStream_t s) {
-    ELAUNCH(k_env_cmid, dim3(e->nx), kET, 0, (const double *)e->chi3, e->cmid, e->nn());
-    if (!use_graph) return env_sweep(e, dt, m, s);
-    if (!e->gexec || e->g_dtau != dt || e->g_iter != m || e->g_stream != s) {
+// The same as a captured graph of this (dt, m, ns, stream), replayed, when use_graph.
+int env_run(Envelope *e, double dt, int m, int ns, int use_graph, hipStream_t s) {
+    if (!use_graph) return env_sweep(e, dt, m, ns, s);
+    if (!e->gexec || e->g_dtau != dt || e->g_iter != m || e->g_steps != ns || e->g_stream != s) {
         drop_graph(e);
         hipGraph_t gr;
         QP_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        const int st = env_sweep(e, dt, m, s);
+        const int st = env_sweep(e, dt, m, ns, s);
         const hipError_t ce = hipStreamEndCapture(s, &gr);
         if (st < 0) {
             if (ce == hipSuccess) (void)hipGraphDestroy(gr);
@@ -365,10 +409,22 @@ int envelope_step(Envelope *e, double dt, int m, int use_graph, hipStream_t s) {
         }
         e->g_dtau = dt;
         e->g_iter = m;
+        e->g_steps = ns;
         e->g_stream = s;
     }
     QP_HIP_CHECK(hipGraphLaunch(e->gexec, s));
     return QP_OK;
+}
+
+}  // namespace
+
+// ------------------------------------------------------- wake-side step
+// One step of the whole envelope after a wake pass, enqueued on s: midranges
+// of chi, then the sweep, replayed from the captured graph of this (dt, m)
+// when use_graph, else launched directly.
+int envelope_step(Envelope *e, double dt, int m, int use_graph, hipStream_t s) {
+    ELAUNCH(k_env_cmid, dim3(e->nx), kET, 0, (const double *)e->chi3, e->cmid, e->nn());
+    return env_run(e, dt, m, 1, use_graph, s);
 }
 
 }  // namespace qp
@@ -439,8 +495,9 @@ int qp_envelope_destroy(qp_envelope h) {
     if (e->ctx) (void)hipStreamSynchronize(e->stream());
     drop_graph(e);
     e->S.destroy();
-    for (double *p : {e->a, e->inc, e->chi3, e->asq3, e->cmid})
+    for (double *p : {e->a, e->inc, e->chi3, e->asq3, e->cmid, e->pipe_inc})
         if (p) (void)hipFree(p);
+    if (e->pipe_spec) (void)hipFree(e->pipe_spec);
 
     delete h;
     return QP_OK;
@@ -537,35 +594,15 @@ int qp_envelope_advance(qp_envelope h, double dtau, int steps, int chi_iteration
         QP_HIP_CHECK(hipEventRecord(ev.a, s));
     }
     if (steps > 0) ELAUNCH(k_env_cmid, dim3(e->nx), kET, 0, (const double *)e->chi3, e->cmid, e->nn());
-    if (use_graph && steps > 0) {
-        if (!e->gexec || e->g_dtau != dtau || e->g_iter != chi_iterations || e->g_stream != s) {
-            drop_graph(e);
-            hipGraph_t gr;
-            QP_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            const int st = env_sweep(e, dtau, chi_iterations, s);
-            const hipError_t ce = hipStreamEndCapture(s, &gr);
-            if (st < 0) {
-                if (ce == hipSuccess) (void)hipGraphDestroy(gr);
-                return st;
-            }
-            if (ce != hipSuccess) {
-                set_error(std::string("hipStreamEndCapture: ") + hipGetErrorString(ce));
-                return QP_ERR_HIP;
-            }
-            const hipError_t ie = hipGraphInstantiate(&e->gexec, gr, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(gr);
-            if (ie != hipSuccess) {
-                e->gexec = nullptr;
-                set_error(std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
-                return QP_ERR_HIP;
-            }
-            e->g_dtau = dtau;
-            e->g_iter = chi_iterations;
-            e->g_stream = s;
-        }
-        for (int n = 0; n < steps; ++n) QP_HIP_CHECK(hipGraphLaunch(e->gexec, s));
-    } else {
-        for (int n = 0; n < steps; ++n) QP_TRY(env_sweep(e, dtau, chi_iterations, s));
+    // pipelines of nearly equal depth; a graph for the deeper ones, the shallower (one
+    // step less, at most) launched directly
+    const int groups = steps > 0 ? (steps + pipe_depth(e) - 1) / pipe_depth(e) : 0;
+    const int deep = groups ? (steps + groups - 1) / groups : 0;
+    QP_TRY(ensure_pipe(e, deep));
+    for (int g = 0, left = steps; g < groups; ++g) {
+        const int ns = (left + groups - g - 1) / (groups - g);
+        QP_TRY(env_run(e, dtau, chi_iterations, ns, use_graph && ns == deep, s));
+        left -= ns;
     }
     if (ms) {
         QP_HIP_CHECK(hipEventRecord(ev.b, s));

@@ -243,3 +243,32 @@ def test_mixed_graphs_follow_driver_changes(qp_ctx, oracle):
         assert same(wk.get_particles(), want)
     wk.close()
     e.close()
+
+
+@pytest.mark.parametrize("ny,nz", [(16, 16), (24, 20), (64, 96)])
+@pytest.mark.parametrize("nx,steps,m,use_graph", [(1, 3, 1, 1), (2, 5, 0, 0), (6, 2, 2, 1), (5, 16, 1, 1), (4, 19, 1, 1),
+                                                  (3, 33, 0, 1)])
+def test_steps_in_flight(qp_ctx, ny, nz, nx, steps, m, use_graph):
+    """Several steps of one call run as a pipeline over the slices (fewer slices than
+    steps, more steps than the pipeline holds, uneven groups of steps): the same as one
+    call per step."""
+    from quetzalpic_amd import capi
+    rng = np.random.default_rng(nx * 100 + steps)
+    a = rng.standard_normal((nx, ny, nz)) + 1j * rng.standard_normal((nx, ny, nz))
+    chi = 1.0 + 0.5 * rng.random((nx, ny, nz))
+    got = []
+    for calls, per in ((1, steps), (steps, 1)):
+        e = capi.Envelope(qp_ctx, nx, ny, nz, 0.1, 20.0 / ny, 20.0 / nz, 10.0)
+        e.set(a)
+        e.set_chi(chi)
+        for _ in range(calls):
+            e.advance(0.5, steps=per, chi_iterations=m, use_graph=use_graph)
+        if calls == 1:   # replay of the captured pipeline against direct launches
+            first = e.get()
+            e.set(a)
+            e.advance(0.5, steps=per, chi_iterations=m, use_graph=use_graph)
+            assert np.array_equal(e.get(), first)
+        got.append((e.get(), e.get_a_sqr()))
+        e.close()
+    for x, y in zip(*got):
+        assert np.array_equal(x, y)
