@@ -144,10 +144,7 @@ int qp_solve2d_device(qp_fourier2d f, double d1, double d2, double D, const doub
     QP_TRY(ensure_steps(f, d1, d2));
     hipStream_t s = f->ctx->stream;
     const Solver2d &S = f->S;
-    QP_TRY(solve_rows_fwd_plain(S, src_dev, S.spec[0], s));
-    QP_TRY(solve_cols(S, D, 1, s, nullptr, 0));
-    QP_TRY(solve_rows_inv_unscaled(S, S.spec[0], dst_dev, s));
-    return QP_OK;
+    return solve_plain(S, D, src_dev, dst_dev, s);
 }
 
 int qp_solve2d(qp_fourier2d f, double d1, double d2, double D, const double *src, double *dst) {

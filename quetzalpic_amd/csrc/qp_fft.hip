@@ -17,8 +17,7 @@
 #include <utility>
 #include <vector>
 
-#include "qp_fft_lds.h"
-#include "qp_solver_kernels.h"
+#include "qp_solver_small.h"
 #include "qp_wave_solver.h"
 
 namespace qp {
@@ -130,17 +129,6 @@ void Solver2d::destroy() {
 }
 
 // ------------------------------------------------------------ launches
-int solve_rows_fwd_plain_ctl(const Solver2d &S, const double *src, double2 *spec, hipStream_t s,
-                             const Ctl *ctl, int skip_mode) {
-    const SrcPlain f{src, S.n2};
-    if (S.wave) return wlaunch_rows_fwd(S, f, spec, spec, 1, s, ctl, skip_mode);
-    return glaunch_rows_fwd(S, f, spec, spec, 1, s, ctl, skip_mode);
-}
-
-int solve_rows_fwd_plain(const Solver2d &S, const double *src, double2 *spec, hipStream_t s) {
-    return solve_rows_fwd_plain_ctl(S, src, spec, s, nullptr, 0);
-}
-
 int solve_cols(const Solver2d &S, double D, int nspec, hipStream_t s, const Ctl *ctl, int skip_mode) {
     if (S.wave) return wlaunch_cols(S, D, nspec, nullptr, s, ctl, skip_mode);
     return glaunch_cols(S, kColsSolve, D, nspec, nullptr, s, ctl, skip_mode);
@@ -157,24 +145,20 @@ int fourier_backward(const Solver2d &S, double2 *spec, double *dst, hipStream_t 
                             (const Ctl *)nullptr, 0, 1, true);
 }
 
-template <class Sink>
-static int rows_inv(const Solver2d &S, const double2 *spec, const Sink &f, hipStream_t s, const Ctl *ctl,
-                    int skip_mode) {
-    if (S.wave) return wlaunch_rows_inv(S, spec, spec, f, 1, s, ctl, skip_mode);
-    return glaunch_rows_inv(S, spec, spec, f, 1, s, ctl, skip_mode);
-}
-
-int solve_rows_inv_unscaled(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s) {
-    return rows_inv(S, spec, SinkRaw{dst, S.n2}, s, (const Ctl *)nullptr, 0);
-}
-
-int solve_rows_inv_plain_ctl(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s,
-                             const Ctl *ctl) {
-    return rows_inv(S, spec, SinkScaled{dst, S.n1, S.n2}, s, ctl, ctl ? 1 : 0);
-}
-
-int solve_rows_inv_plain(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s) {
-    return solve_rows_inv_plain_ctl(S, spec, dst, s, nullptr);
+int solve_plain(const Solver2d &S, double D, const double *src, double *dst, hipStream_t s) {
+    const SrcPlain f{src, S.n2};
+    const SinkRaw o{dst, S.n2};
+    const Ctl *none = nullptr;
+    const double2 *spec = S.spec[0];
+    if (small_solve(S)) return slaunch(S, f, o, D, 1, s, none, 0);
+    if (S.wave) {
+        QP_TRY(wlaunch_rows_fwd(S, f, S.spec[0], S.spec[0], 1, s, none, 0));
+        QP_TRY(solve_cols(S, D, 1, s, none, 0));
+        return wlaunch_rows_inv(S, spec, spec, o, 1, s, none, 0);
+    }
+    QP_TRY(glaunch_rows_fwd(S, f, S.spec[0], S.spec[0], 1, s, none, 0));
+    QP_TRY(solve_cols(S, D, 1, s, none, 0));
+    return glaunch_rows_inv(S, spec, spec, o, 1, s, none, 0);
 }
 
 }  // namespace qp

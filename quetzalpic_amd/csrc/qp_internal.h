@@ -207,18 +207,13 @@ __device__ __forceinline__ void wrap_coords(double &y, double &z, double ly, dou
 }
 
 // ----------------------------------------------------- solver launches
-// All launches go to `s`.  `src_fn` kinds select what the row-forward pass reads.
-int solve_rows_fwd_plain(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);
+// All launches go to `s`.
 int solve_cols(const Solver2d &S, double D, int nspec, hipStream_t s, const Ctl *ctl, int skip_mode);
-int solve_rows_inv_plain(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
-int solve_rows_inv_unscaled(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s);
+// dst = n1 n2 times the solution of (lap_perp - D) dst = src (mean mode dropped).
+int solve_plain(const Solver2d &S, double D, const double *src, double *dst, hipStream_t s);
 // Fourier2d transforms in FFTW's layout (generic kernels whatever S.wave says).
 int fourier_forward(const Solver2d &S, const double *src, double2 *spec, hipStream_t s);
 int fourier_backward(const Solver2d &S, double2 *spec, double *dst, hipStream_t s);
-int solve_rows_fwd_plain_ctl(const Solver2d &S, const double *src, double2 *spec, hipStream_t s,
-                             const Ctl *ctl, int skip_mode);
-int solve_rows_inv_plain_ctl(const Solver2d &S, const double2 *spec, double *dst, hipStream_t s,
-                             const Ctl *ctl);
 
 }  // namespace qp
 

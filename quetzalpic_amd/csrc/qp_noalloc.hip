@@ -124,8 +124,5 @@ extern "C" int qp_solve2d_device_noalloc(qp_ctx ctx, int n1, int n2, double d1, 
     hipLaunchKernelGGL(k_noalloc_tables, dim3((nt + 255) / 256), dim3(256), 0, s, tw1, n1, tw2, n2, lam1, lam2,
                        S.nh, d1, d2);
     QP_HIP_CHECK(hipGetLastError());
-    QP_TRY(solve_rows_fwd_plain(S, src_dev, S.spec[0], s));
-    QP_TRY(solve_cols(S, D, 1, s, nullptr, 0));
-    QP_TRY(solve_rows_inv_unscaled(S, S.spec[0], dst_dev, s));
-    return QP_OK;
+    return solve_plain(S, D, src_dev, dst_dev, s);
 }

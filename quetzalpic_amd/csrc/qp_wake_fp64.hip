@@ -12,7 +12,7 @@
 // iterations.  200^2 x 60 slices with inline output, K = 5: 57.1 -> 29.4 ms.
 #include <cstring>
 
-#include "qp_solver_kernels.h"
+#include "qp_solver_small.h"
 #include "qp_wake.h"
 #include "qp_wave_solver.h"
 
@@ -397,10 +397,22 @@ int wake_download_fp64(Wake *w, double *y, double *z, double *py, double *pz) {
 static int solve_psi(Wake *w, double *psi) {
     const Solver2d &S = w->S;
     hipStream_t s = w->stream();
+    const SrcPlain src{w->src, S.n2};
+    const SinkScaled snk{w->src, S.n1, S.n2};
+    const Ctl *ctl = w->ctl;
+    const double2 *s0 = S.spec[0];
     prof_begin(w, "solve");
-    QP_TRY(solve_rows_fwd_plain_ctl(S, w->src, S.spec[0], s, w->ctl, 1));
-    QP_TRY(solve_cols(S, 0.0, 1, s, w->ctl, 1));
-    QP_TRY(solve_rows_inv_plain_ctl(S, S.spec[0], w->src, s, w->ctl));
+    if (small_solve(S)) {
+        QP_TRY(slaunch(S, src, snk, 0.0, 1, s, ctl, 1));
+    } else if (S.wave) {
+        QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[0], 1, s, ctl, 1));
+        QP_TRY(solve_cols(S, 0.0, 1, s, ctl, 1));
+        QP_TRY(wlaunch_rows_inv(S, s0, s0, snk, 1, s, ctl, 1));
+    } else {
+        QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[0], 1, s, ctl, 1));
+        QP_TRY(solve_cols(S, 0.0, 1, s, ctl, 1));
+        QP_TRY(glaunch_rows_inv(S, s0, s0, snk, 1, s, ctl, 1));
+    }
     prof_end(w, "solve");
     const int per = kT * kNormPer;
     LAUNCH(k_norm_clamp, (int)((w->nn() + per - 1) / per), psi, w->src, S.n1, S.n2, w->p.psi_threshold - 1, w->ctl);
@@ -418,11 +430,17 @@ static int solve_b(Wake *w, int slice) {
     const SinkB64 snk{w->by, w->bz, S.n1, S.n2, p.b_threshold, w->ctl, slice};
     const double2 *s0 = S.spec[0], *s1 = S.spec[1];
     prof_begin(w, "solve");
-    if (S.wave) QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, ctl, 2));
-    else QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, ctl, 2));
-    QP_TRY(solve_cols(S, p.D, 2, s, ctl, 2));
-    if (S.wave) QP_TRY(wlaunch_rows_inv(S, s0, s1, snk, 2, s, ctl, 2));
-    else QP_TRY(glaunch_rows_inv(S, s0, s1, snk, 2, s, ctl, 2));
+    if (small_solve(S)) {
+        QP_TRY(slaunch(S, src, snk, p.D, 2, s, ctl, 2));
+    } else if (S.wave) {
+        QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, ctl, 2));
+        QP_TRY(solve_cols(S, p.D, 2, s, ctl, 2));
+        QP_TRY(wlaunch_rows_inv(S, s0, s1, snk, 2, s, ctl, 2));
+    } else {
+        QP_TRY(glaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, ctl, 2));
+        QP_TRY(solve_cols(S, p.D, 2, s, ctl, 2));
+        QP_TRY(glaunch_rows_inv(S, s0, s1, snk, 2, s, ctl, 2));
+    }
     prof_end(w, "solve");
     return QP_OK;
 }

@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "qp_mixed_kernels.h"
+#include "qp_solver_small.h"
 #include "qp_wave_solver.h"
 
 namespace qp {
@@ -663,7 +664,10 @@ struct SinkPsiFinal {
         g00 = bp[ncb].x;
     }
     __device__ void begin(int) {
-        const double sraw = wave_sum(s1) + (double)n2 * g00 - wave_sum(s2);
+        set_sums(wave_sum(s1), wave_sum(s2), g00);
+    }
+    __device__ void set_sums(double t1, double t2, double g) {
+        const double sraw = t1 + (double)n2 * g - t2;
         b = sraw / n1 / n2 / (n1 + n2 - 1);
     }
     __device__ void operator()(int wk, int, int j, int k, double v) const {
@@ -1377,6 +1381,12 @@ int psi_solve(MxRun &R, hipStream_t s, int slot, double *dst) {
     SrcPsi src{w->src, w->rho_ion, w->rho_b_src(), w->jx_b_src(), w->bsrc_stride(), w->ctl, slot, S.n2, R.nn};
     SinkPsiFinal snk{dst, m->bpart, m->ncb, S.n1, S.n2, w->p.psi_threshold - 1, 0.0, m->bstride,
                      1.0 / ((double)S.n1 * S.n2)};
+    if (small_solve(S)) {
+        prof_begin(w, "solve");
+        QP_TRY(slaunch(S, src, snk, 0.0, 1, s, (const Ctl *)w->ctl, 1, nw));
+        prof_end(w, "solve");
+        return QP_OK;
+    }
     if (S.wave) {
         prof_begin(w, "solve");
         QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[0], 1, s, (const Ctl *)w->ctl, 1, nw));
@@ -1413,6 +1423,12 @@ int b_solve(MxRun &R, hipStream_t s, int slot, const double *jx) {
     double *jyn = m->jbuf[slot][0], *jzn = m->jbuf[slot][1];
     SrcB src{w->by, w->bz, jx, jy, jz, jyn, jzn, S.n1, S.n2, p.D, 1.0 / p.dx, 1.0 / p.dy, 1.0 / p.dz};
     SinkBPair snk{w->by, w->bz, S.n1, S.n2, p.b_threshold, w->ctl, slot, 1.0 / ((double)S.n1 * S.n2)};
+    if (small_solve(S)) {
+        prof_begin(w, "solve");
+        QP_TRY(slaunch(S, src, snk, p.D, 2, s, (const Ctl *)w->ctl, 2, nw));
+        prof_end(w, "solve");
+        return QP_OK;
+    }
     if (S.wave) {
         prof_begin(w, "solve");
         QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[1], 2, s, (const Ctl *)w->ctl, 2, nw));
@@ -1448,6 +1464,7 @@ int bx_solve(MxRun &R, hipStream_t s, int slot) {
     const int nw = R.nw;
     SrcCurl src{m->jbuf[1 - slot][0], m->jbuf[1 - slot][1], S.n1, S.n2, 1.0 / p.dy, 1.0 / p.dz};
     SinkMember snk{w->bx, S.n1, S.n2, 1.0 / ((double)S.n1 * S.n2)};
+    if (small_solve(S)) return slaunch(S, src, snk, 0.0, 1, s, (const Ctl *)w->ctl, 1, nw);
     if (S.wave) {
         QP_TRY(wlaunch_rows_fwd(S, src, S.spec[0], S.spec[0], 1, s, (const Ctl *)w->ctl, 1, nw));
         QP_TRY(wlaunch_cols(S, 0.0, 1, nullptr, s, (const Ctl *)w->ctl, 1, nw));
