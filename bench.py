@@ -538,7 +538,6 @@ class C4Job:
                 log(f"[bench] C4 class {n}x{n}: {len(ms)} members, {self.batches[n][2]} particles")
             if len(chain) > 1:
                 g = capi.WakeGroup(ctx, [self.batches[n][1] for n in chain])
-                g.set_fork(chains == 1)   # a second stream per group only pays when the group runs alone
                 self.groups.append(g)
             else:
                 self.groups.append(self.batches[chain[0]][1])

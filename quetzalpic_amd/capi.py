@@ -677,8 +677,7 @@ class WakeGroup:
         _check(load().qp_group_set_tile(self.h, threads_per_block, window_nodes), "qp_group_set_tile")
 
     def set_fork(self, fork_families):
-        """Run the two transform families' solver launches on two streams (True, the
-        default) or in sequence on the context's stream (False)."""
+        """Accepted and without effect: both transform families share each solver launch."""
         _check(load().qp_group_set_fork(self.h, 1 if fork_families else 0), "qp_group_set_fork")
 
     def close(self):

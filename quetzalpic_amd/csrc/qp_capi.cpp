@@ -527,7 +527,7 @@ int qp_group_set_tile(qp_group h, int threads_per_block, int window_nodes) {
 
 int qp_group_set_fork(qp_group h, int fork_families) {
     ARG_CHECK(h, "null group");
-    h->g.fork_families = fork_families != 0;
+    (void)fork_families;  // both families share a launch
     return QP_OK;
 }
 

@@ -832,12 +832,18 @@ __global__ void k_sort_copyback(MxPart P, MxPart Q, int *perm, const int *perm2)
 // (a uniform switch) with one launch shape for all sides, 64 threads per
 // block, so the LDS buffers are one dynamic allocation sized for the largest
 // transform group (sides 3 * 2^p: eight 96-point or four 192-point transforms).
+// A kernel holds the lengths of one transform family (2^p: 0, 3 * 2^p: 1) or of both
+// (2), whichever the group's sides need: with both, every block has the registers and
+// LDS of the 3 * 2^p transforms (12 blocks to a CU instead of 18), but these launches have
+// few blocks (2500 at 32 wakes of five grids, two wavefronts to a SIMD) and wait on
+// latencies, so one launch takes little more than its slower half did: B-source rows 17 us
+// against 12.3 and 11.4, columns 10.8 against 8.5 and 9.7.  (Before, the halves ran on two
+// streams, whose fork and join cost each solver launch about 10 us more.)  That group, 160
+// slices, 206 -> 175 ms; one wake of each grid 42 -> 28, twice the group 175 -> 162 ms (60 slices).
 constexpr int kGroupMax = 16;
 constexpr int kGrpTB = 64;
-// LDS of the two transform families per 64-thread block: T * PADN = 64 E / N *
-// 17 N / 16 = 68 E complex values per exchange buffer (E = 4 for sides 2^p,
-// kWfE3 for 3 * 2^p).  The families launch separately: one kernel holding both
-// would give every block the registers and LDS of the 3 * 2^p transforms.
+// LDS per 64-thread block: T * PADN = 64 E / N * 17 N / 16 = 68 E complex values per
+// exchange buffer (E = 4 for sides 2^p, kWfE3 for 3 * 2^p).
 constexpr int grp_lds(int fam) { return 68 * (fam ? kWfE3 : 4); }
 
 struct GrpMap {
@@ -997,8 +1003,10 @@ __global__ __launch_bounds__(kGrpTB) void kg_rows_fwd(GrpMap m, const GArgsRowsF
         break;
     if constexpr (FAM == 0) {
         switch (a.n2) { QP_GRP_SIDES_P2(QP_CASE) default: break; }
-    } else {
+    } else if constexpr (FAM == 1) {
         switch (a.n2) { QP_GRP_SIDES_P3(QP_CASE) default: break; }
+    } else {
+        switch (a.n2) { QP_GRP_SIDES_P2(QP_CASE) QP_GRP_SIDES_P3(QP_CASE) default: break; }
     }
 #undef QP_CASE
 }
@@ -1010,7 +1018,7 @@ __global__ __launch_bounds__(kGrpTB) void kg_cols(GrpMap m, const GArgsCols *__r
     int b, bx, by;
     grp_locate(m, b, bx, by);
     const GArgsCols &a = t[b];
-    const int tpb = kGrpTB * (FAM ? kWfE3 : 4) / a.n1;   // transforms per block
+    const int tpb = kGrpTB * (a.n1 % 3 == 0 ? kWfE3 : 4) / a.n1;   // transforms per block
     const int gx = (a.nh + tpb - 1) / tpb;
     double2 *sb0 = gl2, *sb1 = gl2 + grp_lds(FAM);
 #define QP_CASE(N)                                                                                                  \
@@ -1020,8 +1028,10 @@ __global__ __launch_bounds__(kGrpTB) void kg_cols(GrpMap m, const GArgsCols *__r
         break;
     if constexpr (FAM == 0) {
         switch (a.n1) { QP_GRP_SIDES_P2(QP_CASE) default: break; }
-    } else {
+    } else if constexpr (FAM == 1) {
         switch (a.n1) { QP_GRP_SIDES_P3(QP_CASE) default: break; }
+    } else {
+        switch (a.n1) { QP_GRP_SIDES_P2(QP_CASE) QP_GRP_SIDES_P3(QP_CASE) default: break; }
     }
 #undef QP_CASE
 }
@@ -1040,8 +1050,10 @@ __global__ __launch_bounds__(kGrpTB) void kg_rows_inv(GrpMap m, const GArgsRowsI
         break;
     if constexpr (FAM == 0) {
         switch (a.n2) { QP_GRP_SIDES_P2(QP_CASE) default: break; }
-    } else {
+    } else if constexpr (FAM == 1) {
         switch (a.n2) { QP_GRP_SIDES_P3(QP_CASE) default: break; }
+    } else {
+        switch (a.n2) { QP_GRP_SIDES_P2(QP_CASE) QP_GRP_SIDES_P3(QP_CASE) default: break; }
     }
 #undef QP_CASE
 }
@@ -2123,15 +2135,11 @@ struct GroupTabs {
 
 struct GroupMaps {
     GrpMap part, out;
-    GrpMap rows1[2], rows2[2], cols1[2], cols2[2];   // per transform family (sides 2^p, 3 * 2^p)
+    GrpMap rows1, rows2, cols1, cols2;
+    int rfam, cfam;   // transform families of the rows / the columns: 0 2^p, 1 3 * 2^p, 2 both
 };
 
 struct GroupState {
-    // the second transform family's launches run on this stream, forked from and
-    // joined back into the group's (a parallel branch of the captured step)
-    hipStream_t side = nullptr;
-    std::vector<hipEvent_t> ev;   // fork / join pairs of one slice step
-    size_t ev_next = 0;
     GroupTabs *d_tabs = nullptr;
     GroupTabs h_tabs;
     GroupMaps maps{}, graph_maps{};
@@ -2199,11 +2207,13 @@ void group_tables(Group *G, std::vector<MxRun> &R, GroupTabs &T, GroupMaps &M) {
         // block maps: the launch grids of the single-batch path with 64-thread solver blocks
         const int T2 = kGrpTB * grp_elems(S.n2) / S.n2, T1 = kGrpTB * grp_elems(S.n1) / S.n1;
         const int f2 = S.n2 % 3 == 0 ? 1 : 0, f1 = S.n1 % 3 == 0 ? 1 : 0;   // transform families
+        M.rfam = bi == 0 || M.rfam == f2 ? f2 : 2;
+        M.cfam = bi == 0 || M.cfam == f1 ? f1 : 2;
         map_add(M.part, b, R[b].pb, nw);
-        map_add(M.rows1[f2], b, wrows_blocks_t(S.n1, T2), nw);
-        map_add(M.rows2[f2], b, wrows_blocks_t(S.n1, T2), 2 * nw);
-        map_add(M.cols1[f1], b, wcols_blocks_t(S.nh, T1), nw);
-        map_add(M.cols2[f1], b, wcols_blocks_t(S.nh, T1), 2 * nw);
+        map_add(M.rows1, b, wrows_blocks_t(S.n1, T2), nw);
+        map_add(M.rows2, b, wrows_blocks_t(S.n1, T2), 2 * nw);
+        map_add(M.cols1, b, wcols_blocks_t(S.nh, T1), nw);
+        map_add(M.cols2, b, wcols_blocks_t(S.nh, T1), 2 * nw);
         map_add(M.out, b, R[b].gb, nw);
     }
 }
@@ -2215,56 +2225,21 @@ void group_tables(Group *G, std::vector<MxRun> &R, GroupTabs &T, GroupMaps &M) {
             QP_HIP_CHECK(hipGetLastError());                                                   \
         }                                                                                      \
     } while (0)
-// One solver pass of every batch: one launch per transform family present
-// (GSOLVE_T for the kernels templated on their source / sink type).
-// The two transform families of one solver pass are independent launches with
-// few blocks each (latency-bound): with both present and Group::fork_families
-// set, the 3 * 2^p family's runs on the side stream beside the 2^p family's.
-// The 64-wake group of five grid sizes: 2.50 -> 2.40 ms per slice.  With the
-// same wakes in three chains on their own streams (one chain a group of three
-// batches) the extra stream was slower (1.99 -> 2.32 ms per slice), so callers
-// running several groups or batches at once switch it off.
-template <class L0, class L1>
-int fam_pair(GroupState *st, hipStream_t s, bool both, L0 &&l0, L1 &&l1) {
-    if (!both) {
-        QP_TRY(l0(s));
-        return l1(s);
-    }
-    if (st->ev_next + 2 > st->ev.size()) {
-        set_error("group: fork events exhausted");
-        return QP_ERR_HIP;
-    }
-    hipEvent_t ef = st->ev[st->ev_next++], ej = st->ev[st->ev_next++];
-    QP_HIP_CHECK(hipEventRecord(ef, s));
-    QP_HIP_CHECK(hipStreamWaitEvent(st->side, ef, 0));
-    QP_TRY(l1(st->side));
-    QP_HIP_CHECK(hipEventRecord(ej, st->side));
-    QP_TRY(l0(s));
-    QP_HIP_CHECK(hipStreamWaitEvent(s, ej, 0));
-    return QP_OK;
-}
-#define GSOLVE(kern, maps, nspec, tab)                                                                     \
-    QP_TRY(fam_pair(                                                                                       \
-        st, s, G->fork_families && (maps)[0].nb > 0 && (maps)[1].nb > 0,                                   \
-        [&](hipStream_t s) {                                                                               \
-            GLAUNCH((kern<0>), maps[0], kGrpTB, sizeof(double2) * 2 * grp_lds(0), tab, nspec, nspec);      \
-            return QP_OK;                                                                                  \
-        },                                                                                                 \
-        [&](hipStream_t s) {                                                                               \
-            GLAUNCH((kern<1>), maps[1], kGrpTB, sizeof(double2) * 2 * grp_lds(1), tab, nspec, nspec);      \
-            return QP_OK;                                                                                  \
-        }))
-#define GSOLVE_T(kern, T, maps, nspec, tab)                                                                \
-    QP_TRY(fam_pair(                                                                                       \
-        st, s, G->fork_families && (maps)[0].nb > 0 && (maps)[1].nb > 0,                                   \
-        [&](hipStream_t s) {                                                                               \
-            GLAUNCH((kern<T, 0>), maps[0], kGrpTB, sizeof(double2) * 2 * grp_lds(0), tab, nspec, nspec);   \
-            return QP_OK;                                                                                  \
-        },                                                                                                 \
-        [&](hipStream_t s) {                                                                               \
-            GLAUNCH((kern<T, 1>), maps[1], kGrpTB, sizeof(double2) * 2 * grp_lds(1), tab, nspec, nspec);   \
-            return QP_OK;                                                                                  \
-        }))
+// One solver pass of every batch, by the kernel of the transform families present.
+#define GSOLVE_F(kern, fam, map, nspec, ...) \
+    GLAUNCH((kern), map, kGrpTB, sizeof(double2) * 2 * grp_lds(fam), __VA_ARGS__, nspec, nspec)
+#define GROWS(kern, T, map, nspec, tab)                                                  \
+    do {                                                                                 \
+        if (M.rfam == 0) GSOLVE_F((kern<T, 0>), 0, map, nspec, tab);                     \
+        else if (M.rfam == 1) GSOLVE_F((kern<T, 1>), 1, map, nspec, tab);                \
+        else GSOLVE_F((kern<T, 2>), 2, map, nspec, tab);                                 \
+    } while (0)
+#define GCOLS(map, nspec, tab)                                                           \
+    do {                                                                                 \
+        if (M.cfam == 0) GSOLVE_F(kg_cols<0>, 0, map, nspec, tab);                       \
+        else if (M.cfam == 1) GSOLVE_F(kg_cols<1>, 1, map, nspec, tab);                  \
+        else GSOLVE_F(kg_cols<2>, 2, map, nspec, tab);                                   \
+    } while (0)
 
 // One slice step of every batch: enqueue_slice with one launch per phase.
 template <int PT, int CAP>
@@ -2272,14 +2247,13 @@ int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
     const qp_wake_params &p = G->b[0]->p;
     const GroupMaps &M = st->maps;
     GroupTabs *T = st->d_tabs;
-    st->ev_next = 0;
     const int slot = i & 1;
     const bool first = (i == p.nx - 1);
     const bool s_phase = (i == 0) || (p.K == 0);
     GLAUNCH((kg_mx_A<PT, CAP>), M.part, PT, 0, T->A[slot], first ? 0 : (p.K == 0 ? 2 : 1));
-    GSOLVE_T(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
-    GSOLVE(kg_cols, M.cols1, 1, T->PC);
-    GSOLVE_T(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->PI[slot]);
+    GROWS(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
+    GCOLS(M.cols1, 1, T->PC);
+    GROWS(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->PI[slot]);
     if (s_phase) {
         GLAUNCH((kg_mx_S<PT, CAP>), M.part, PT, sizeof(double) * 3 * CAP, T->S[slot]);
         if (i == 0) return QP_OK;
@@ -2291,13 +2265,13 @@ int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
                         it);
                 return QP_OK;
             }));
-            GSOLVE_T(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
-            GSOLVE(kg_cols, M.cols1, 1, T->PC);
-            GSOLVE_T(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->MI);
+            GROWS(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
+            GCOLS(M.cols1, 1, T->PC);
+            GROWS(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->MI);
             GLAUNCH((kg_mx_C<PT, CAP>), M.part, PT, 0, T->C[slot]);
-            GSOLVE_T(kg_rows_fwd, SrcB, M.rows2, 2, T->BF[slot][it & 1]);
-            GSOLVE(kg_cols, M.cols2, 2, T->BC);
-            GSOLVE_T(kg_rows_inv, SinkBPair, M.rows2, 2, T->BI[slot]);
+            GROWS(kg_rows_fwd, SrcB, M.rows2, 2, T->BF[slot][it & 1]);
+            GCOLS(M.cols2, 2, T->BC);
+            GROWS(kg_rows_inv, SinkBPair, M.rows2, 2, T->BI[slot]);
         }
     }
     GLAUNCH(kg_mx_out, M.out, 256, 0, T->O, first ? 0 : 1, slot, 0);
@@ -2365,9 +2339,6 @@ void group_destroy_mixed(Group *G) {
     for (auto &g : st->gexec)
         if (g) (void)hipGraphExecDestroy(g);
     if (st->d_tabs) (void)hipFree(st->d_tabs);
-    for (hipEvent_t e : st->ev)
-        if (e) (void)hipEventDestroy(e);
-    if (st->side) (void)hipStreamDestroy(st->side);
     delete st;
     G->dev = nullptr;
 }
@@ -2413,13 +2384,6 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
         st = new GroupState();
         G->dev = st;
         QP_HIP_CHECK(hipMalloc(&st->d_tabs, sizeof(GroupTabs)));
-        QP_HIP_CHECK(hipStreamCreateWithFlags(&st->side, hipStreamNonBlocking));
-    }
-    // fork / join events: two per solver pass of one slice step (3 + 6 K passes)
-    while (st->ev.size() < (size_t)(2 * (3 + 6 * G->b[0]->p.K))) {
-        hipEvent_t e = nullptr;
-        QP_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        st->ev.push_back(e);
     }
     std::vector<MxRun> R(nb);
     for (int b = 0; b < nb; ++b) QP_TRY(pass_setup(G->b[b], R[b]));
@@ -2429,7 +2393,6 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
     std::vector<unsigned> epochs(nb);
     for (int b = 0; b < nb; ++b) epochs[b] = G->b[b]->inputs_epoch;
     epochs.push_back((unsigned)G->tile_cap);   // the maps carry the block counts of the tile, not its capacity
-    epochs.push_back(G->fork_families ? 1u : 0u);
     if (std::memcmp(&st->maps, &st->graph_maps, sizeof(GroupMaps)) != 0 || epochs != st->graph_epochs) {
         for (auto &g : st->gexec)
             if (g) (void)hipGraphExecDestroy(g);

@@ -223,3 +223,28 @@ def test_c4_as_one_group(qp_ctx, oracle):
             assert e[0] < 1e-6, (n, f, e)
     for b in batches:
         b.close()
+
+
+@pytest.mark.parametrize("layout", [[(16, 256)], [(48, 192), (96, 96)], [(64, 48), (32, 32)], [(48, 64), (96, 16)],
+                                    [(256, 192), (16, 16), (192, 32)]])
+def test_solver_launch_per_families_present(qp_ctx, oracle, layout):
+    """Rows and columns choose their kernel by the transform families of their own sides: 2^p
+    only, 3 * 2^p only, both, and different choices for rows and columns; the shortest and
+    longest sides together.  Same bar as the members above, 1e-9."""
+    from quetzalpic_amd import capi
+    fields = ("psi", "ez", "by", "bz")
+    batches = []
+    for bi, (ny, nz) in enumerate(layout):
+        g = oracle.grid_from_box(1.0, L, L, DX, L / ny, L / nz, K=2)
+        batches.append(make_batch(qp_ctx, g, [inputs(oracle, g, 10 * bi + m) for m in range(2)]))
+    grp = capi.WakeGroup(qp_ctx, batches)
+    outs, st, _ = grp.run(fields=fields)
+    grp.close()
+    assert st == 0
+    for got, b in zip(outs, batches):
+        alone, s1, _ = b.run(fields=fields)
+        assert s1 == 0
+        for m in range(2):
+            for f in fields:
+                assert rel_err(got[m][f], alone[m][f])[0] < 1e-9, (m, f)
+        b.close()
