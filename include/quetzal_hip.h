@@ -256,6 +256,8 @@ int qp_envelope_set(qp_envelope e, const double *re, const double *im);
 int qp_envelope_set_gaussian(qp_envelope e, double a0, double xsigma, double ysigma, double zsigma,
                              double x0, double y0, double z0);
 int qp_envelope_get(qp_envelope e, double *re, double *im);
+/* The same as complex values: re, im of each node side by side (2 nx ny nz doubles). */
+int qp_envelope_get_complex(qp_envelope e, double *a);
 /* chi of every slice, nx*ny*nz (NULL = zero). */
 int qp_envelope_set_chi(qp_envelope e, const double *chi);
 int qp_envelope_get_chi(qp_envelope e, double *chi);

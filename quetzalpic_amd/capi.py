@@ -104,6 +104,7 @@ def load():
         "qp_envelope_set": ([vp, _dp, _dp], ctypes.c_int),
         "qp_envelope_set_gaussian": ([vp] + [ctypes.c_double] * 7, ctypes.c_int),
         "qp_envelope_get": ([vp, _dp, _dp], ctypes.c_int),
+        "qp_envelope_get_complex": ([vp, _dp], ctypes.c_int),
         "qp_envelope_set_chi": ([vp, _dp], ctypes.c_int),
         "qp_envelope_get_chi": ([vp, _dp], ctypes.c_int),
         "qp_envelope_get_a_sqr": ([vp, _dp], ctypes.c_int),
@@ -409,9 +410,9 @@ class Envelope:
                "qp_envelope_set_gaussian")
 
     def get(self):
-        re, im = np.zeros(self.shape), np.zeros(self.shape)
-        _check(load().qp_envelope_get(self.h, _ptr(re), _ptr(im)), "qp_envelope_get")
-        return re + 1j * im
+        a = np.empty(self.shape, dtype=np.complex128)
+        _check(load().qp_envelope_get_complex(self.h, _ptr(a.view(np.float64))), "qp_envelope_get_complex")
+        return a
 
     def set_chi(self, chi):
         c = _f64(chi, self.shape, "Envelope.set_chi")

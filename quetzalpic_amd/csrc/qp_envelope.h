@@ -10,6 +10,8 @@
 // The scheme is stated in qp_envelope.hip.
 #pragma once
 
+#include <mutex>
+
 #include "qp_internal.h"
 
 namespace qp {
@@ -27,6 +29,9 @@ struct Envelope {
     int pipe = 0;                    // steps in flight the two buffers below hold (0: none)
     double *pipe_inc = nullptr;      // as inc, per step
     double2 *pipe_spec = nullptr;    // spectra of the real parts per step, then of the imaginary parts
+    double2 *join = nullptr;         // complex values on their way to the host (njoin of them; join_lock's holder)
+    size_t njoin = 0;
+    std::mutex join_lock;
     int attached = 0;        // wakes reading this envelope
     hipGraphExec_t gexec = nullptr;  // g_steps steps, captured for dtau = g_dtau, g_iter chi corrections
     double g_dtau = 0.0;

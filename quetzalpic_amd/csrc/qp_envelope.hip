@@ -63,6 +63,12 @@ __global__ void k_env_gauss(double *a, double *asq, size_t vol, size_t nn, int n
     }
 }
 
+// Real and imaginary parts side by side, for the copy to the host.
+__global__ void k_env_join(const double *re, const double *im, double2 *out, size_t n) {
+    const size_t t = (size_t)blockIdx.x * kET + threadIdx.x;
+    if (t < n) out[t] = make_double2(re[t], im[t]);
+}
+
 __global__ void k_env_asq(const double *a, double *asq, size_t vol) {
     for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < vol; t += (size_t)gridDim.x * blockDim.x) {
         const double re = a[t], im = a[vol + t];
@@ -498,7 +504,7 @@ int qp_envelope_destroy(qp_envelope h) {
     for (double *p : {e->a, e->inc, e->chi3, e->asq3, e->cmid, e->pipe_inc})
         if (p) (void)hipFree(p);
     if (e->pipe_spec) (void)hipFree(e->pipe_spec);
-
+    if (e->join) (void)hipFree(e->join);
     delete h;
     return QP_OK;
 }
@@ -542,6 +548,40 @@ int qp_envelope_get(qp_envelope h, double *re, double *im) {
     const size_t vol = e->vol();
     if (re) QP_HIP_CHECK(hipMemcpy(re, e->a, sizeof(double) * vol, hipMemcpyDeviceToHost));
     if (im) QP_HIP_CHECK(hipMemcpy(im, e->a + vol, sizeof(double) * vol, hipMemcpyDeviceToHost));
+    return QP_OK;
+}
+
+// Through at most 32 MB of device memory at a time (one copy to pageable memory runs at
+// 18 GB/s, a chunk's launch is lost in it).  105 MB: 25.3 ms as two parts that the caller
+// joined (three passes over fresh host memory), 9.8 ms so, 3.9 of them page faults.
+int qp_envelope_get_complex(qp_envelope h, double *a) {
+    EARG_CHECK(h && a, "qp_envelope_get_complex: null argument");
+    Envelope *e = &h->e;
+    hipStream_t s = e->stream();
+    const size_t vol = e->vol();
+    QP_HIP_CHECK(hipSetDevice(e->ctx->device));
+    std::lock_guard<std::mutex> lock(e->join_lock);
+    if (!e->join) {
+        size_t n = std::min(vol, (size_t)1 << 21);
+        while (hipMalloc(&e->join, sizeof(double2) * n) != hipSuccess) {
+            (void)hipGetLastError();
+            e->join = nullptr;
+            if (n <= 4096) {
+                set_error("qp_envelope_get_complex: device allocation failed");
+                return QP_ERR_ALLOC;
+            }
+            n /= 2;
+        }
+        e->njoin = n;
+    }
+    for (size_t o = 0; o < vol; o += e->njoin) {
+        const size_t n = std::min(e->njoin, vol - o);
+        hipLaunchKernelGGL(k_env_join, dim3(eblk(n)), dim3(kET), 0, s, (const double *)e->a + o,
+                           (const double *)e->a + vol + o, e->join, n);
+        QP_HIP_CHECK(hipGetLastError());
+        QP_HIP_CHECK(hipMemcpyAsync(a + 2 * o, e->join, sizeof(double2) * n, hipMemcpyDeviceToHost, s));
+    }
+    QP_HIP_CHECK(hipStreamSynchronize(s));
     return QP_OK;
 }
 

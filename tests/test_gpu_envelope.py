@@ -272,3 +272,24 @@ def test_steps_in_flight(qp_ctx, ny, nz, nx, steps, m, use_graph):
         e.close()
     for x, y in zip(*got):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(2, 16, 16), (2, 1024, 1024), (3, 1000, 701), (7, 640, 480)])
+def test_complex_values_are_the_parts(qp_ctx, nx, ny, nz):
+    """Below, at and beyond the chunk of the copy (2^21 values): every bit of both parts."""
+    import ctypes
+    from quetzalpic_amd import capi
+    rng = np.random.default_rng(nx * ny)
+    a = rng.standard_normal((nx, ny, nz)) + 1j * rng.standard_normal((nx, ny, nz))
+    a.real[0, 0, :3] = (np.inf, -0.0, np.nan)
+    a.imag[-1, -1, -3:] = (np.nan, -np.inf, -0.0)
+    e = capi.Envelope(qp_ctx, nx, ny, nz, 0.1, 0.1, 0.1, 10.0)
+    e.set(a)
+    got = e.get()
+    re, im = np.empty(a.shape), np.empty(a.shape)
+    dp = ctypes.POINTER(ctypes.c_double)
+    assert capi.load().qp_envelope_get(e.h, re.ctypes.data_as(dp), im.ctypes.data_as(dp)) == 0
+    e.close()
+    assert np.array_equal(got.real.copy().view(np.int64), re.view(np.int64))
+    assert np.array_equal(got.imag.copy().view(np.int64), im.view(np.int64))
+    assert np.array_equal(re.view(np.int64), a.real.copy().view(np.int64))
