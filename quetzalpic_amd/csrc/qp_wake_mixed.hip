@@ -634,6 +634,9 @@ struct SrcB {
     __device__ void done(int, int, int, int, int) const {}
 };
 
+template <>
+inline constexpr bool eight_per_lane<SrcB> = true;
+
 // psi finalisation: v/n1/n2, minus the border mean (normalize_potential,
 // :30-47) computed from the column pass's partial sums, then the clamp.
 struct SinkPsiFinal {

@@ -360,11 +360,12 @@ __device__ __forceinline__ void wf_tw_load(double2 (&t)[NT], const double2 *__re
 // Twiddle source of wave_fft.  Every lane loads the twiddles it applies into
 // registers at kernel start, next to its data loads: no LDS table and no
 // barrier to publish it.  That holds 3 per pass with 4 elements per lane, and
-// up to 15 in all for lengths 3 * 2^p <= 192 with 6 per lane (18 with 12); for
+// up to 15 in all for lengths 3 * 2^p <= 192 with 6 per lane (18 with 12) and 18 for
+// 1024 with 8; for
 // 384 the block stages the N-entry table in LDS instead.
 template <int N, int E, int TB>
 struct WfTw {
-    static constexpr bool kRegs = E == 4 || N <= 192;
+    static constexpr bool kRegs = E == 4 || E == 8 || N <= 192;
     static constexpr int NT = kRegs ? wf_ntw(N, E, E) : 1;
     static constexpr int NL = kRegs ? 1 : N;  // entries of the LDS table
     double2 reg[NT > 0 ? NT : 1];

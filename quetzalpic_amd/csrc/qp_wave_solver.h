@@ -41,6 +41,15 @@ struct WfCfg {
     static constexpr int TBC = N == 256 ? 64 : (N == 512 ? 128 : (N == 1024 ? 256 : TB));
 };
 
+// Sources whose rows of 1024 run with eight elements to a lane (four passes instead of
+// five, half the wavefronts): a plain 1024^2 solve 26.4 -> 26.1 us, the B sources' launch 20.15 ->
+// 19.8.  The psi source's launch was slower with eight (12.7 -> 13.2 us), as were the column
+// pass (a solve 26.3 -> 26.5) and the inverse rows of both sinks (13.8 -> 14.2, 10.1 -> 10.3).
+template <class Src>
+constexpr bool eight_per_lane = false;
+template <>
+inline constexpr bool eight_per_lane<SrcPlain> = true;
+
 // Sum of three values over a block of TB threads (every thread gets the sums).
 template <int TB>
 __device__ __forceinline__ void block_sum3(double &a, double &b, double &c) {
@@ -352,7 +361,9 @@ int wlaunch_rows_fwd(const Solver2d &S, const Src &src, double2 *spec0, double2 
                      const Ctl *ctl, int skip_mode, int nw = 1) {
     const size_t sstride = (size_t)S.n1 * S.nh;
     wf_dispatch(S.n2, [&](auto NC) {
-        constexpr int N = decltype(NC)::value, E = WfCfg<N>::E, TB = WfCfg<N>::TB;
+        constexpr int N = decltype(NC)::value;
+        constexpr bool eight = N == 1024 && eight_per_lane<Src>;
+        constexpr int E = eight ? 8 : WfCfg<N>::E, TB = eight ? WfCfg<N>::TB / 2 : WfCfg<N>::TB;
         const dim3 grid(wrows_blocks_t(S.n1, WfShape<N, E, TB>::T), nspec * nw);
         hipLaunchKernelGGL((kw_rows_fwd<N, E, TB, Src>), grid, dim3(TB), 0, s, src, spec0, spec1, S.n1,
                            (const double2 *)S.ax2.dev.tw, ctl, skip_mode, nspec, sstride);
