@@ -39,16 +39,17 @@ def bytes_per_particle(cls, K):
     offsets, 2 x f64 momenta, f64 weight; scratch T = 16 B: 2 x f64 predicted
     momenta p*):
       A: read cell, offsets, weight, p* (36), write cell, offsets, momenta (28) = 64
-      B: read S (+ T after the first iteration), write T                      = 52 | 68
-      C: read S + T                                                           = 52
+      B: read S (+ T after the first iteration), write T, in the first
+         iteration 1/(1 + psi) too (8)                                        = 60 | 68
+      C: read cell, offsets, weight, p*, 1/(1 + psi)                          = 44
       S: read S                                                               = 36
-    648 B per particle-slice at K = 5."""
+    616 B per particle-slice at K = 5."""
     if cls == "push_A":
         return 64.0
     if cls == "push_B":
-        return (52.0 + 68.0 * (K - 1)) / K if K > 0 else 52.0
+        return (60.0 + 68.0 * (K - 1)) / K if K > 0 else 60.0
     if cls == "push_C":
-        return 52.0
+        return 44.0
     if cls == "push_S":
         return 36.0
     raise KeyError(cls)
