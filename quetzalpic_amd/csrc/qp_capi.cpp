@@ -581,7 +581,7 @@ int wake_alloc_common(Wake *w) {
     QP_HIP_CHECK(hipMemset(w->ctl, 0, sizeof(Ctl) * nw));
     QP_HIP_CHECK(hipMalloc(&w->d_laser, sizeof(LaserGauss) * nw));
     QP_HIP_CHECK(hipMemset(w->d_laser, 0, sizeof(LaserGauss) * nw));
-    QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * (nn * kOutPlanes + kCtlWords), hipHostMallocDefault));
+    QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * (nn * kOutPlanes + kCtlWords + 1), hipHostMallocDefault));
     QP_HIP_CHECK(hipEventCreate(&w->ev0));
     QP_HIP_CHECK(hipEventCreate(&w->ev1));
     return QP_OK;

@@ -1,5 +1,6 @@
-// qp_output.hip -- per-slice output: the planes of a view leave the device in one
-// launch (output_step, src/System_3d.cpp:629-666, writes them slice by slice).
+// qp_output.hip -- what a pass hands to the host while it runs: per-slice output, where the
+// planes of a view leave the device in one launch (output_step, src/System_3d.cpp:629-666,
+// writes them slice by slice), and the number of members that have not stopped.
 #include <string>
 
 #include "qp_wake.h"
@@ -26,7 +27,32 @@ __global__ __launch_bounds__(kPackT) void k_pack(OutPlanes o, size_t plane, cons
         d[t] = src ? src[t] : 0.0;
 }
 
+// Members of the batches that have not stopped.
+__global__ __launch_bounds__(64) void k_running(CtlSets c, int *count) {
+    int n = 0;
+    for (int b = 0; b < c.nb; ++b)
+        for (int m = threadIdx.x; m < c.nw[b]; m += 64) n += c.ctl[b][m].stop_acc == 0;
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+    if (threadIdx.x == 0) *count = n;
+}
+
 }  // namespace
+
+int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t ev, hipStream_t s, bool &over) {
+    over = false;
+    if (done == 0 || done % kWatchSlices != 0) return QP_OK;
+    if (done > kWatchSlices) {  // the mark before this one
+        QP_HIP_CHECK(hipEventSynchronize(ev));
+        over = *count == 0;
+        if (over) return QP_OK;
+    }
+    hipLaunchKernelGGL(k_running, dim3(1), dim3(64), 0, s, c, count);
+    QP_HIP_CHECK(hipGetLastError());
+    QP_HIP_CHECK(hipEventRecord(ev, s));
+    return QP_OK;
+}
+
+int *Wake::h_running() const { return reinterpret_cast<int *>(h_out + kOutPlanes * nn() + kCtlWords); }
 
 int pack_planes(const OutPlanes &o, size_t plane, const Ctl *ctl, int nctl, double *dst, hipStream_t s) {
     const size_t blocks = (plane + kPackT - 1) / kPackT;

@@ -475,7 +475,13 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
         return OutPlanes{{w->psi, w->rho, w->jx, w->jy, w->jz, w->ex, w->ey, w->ez, w->by, w->bz, w->chi, nullptr}};
     };
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
+    const CtlSets cs = w->ctl_set();
     for (int i = p.nx - 1; i >= i_end; --i) {
+        if (!cb) {
+            bool over = false;
+            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev1, s, over));
+            if (over) break;
+        }
         const double *asq;
         QP_TRY(wake_asq_slice(w, i, &asq));
         if (w->bunch) QP_TRY(bunch_slice_sources(w->bunch, ctl, -1, i, s));

@@ -869,7 +869,6 @@ __global__ void k_sort_copyback(MxPart P, MxPart Q, int *perm, const int *perm2)
 // against 12.3 and 11.4, columns 10.8 against 8.5 and 9.7.  (Before, the halves ran on two
 // streams, whose fork and join cost each solver launch about 10 us more.)  That group, 160
 // slices, 206 -> 175 ms; one wake of each grid 42 -> 28, twice the group 175 -> 162 ms (60 slices).
-constexpr int kGroupMax = 16;
 constexpr int kGrpTB = 64;
 // LDS per 64-thread block: T * PADN = 64 E / N * 17 N / 16 = 68 E complex values per
 // exchange buffer (E = 4 for sides 2^p, kWfE3 for 3 * 2^p).
@@ -2055,8 +2054,14 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
         }
     } join{q, writer};
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
+    const CtlSets cs = w->ctl_set();
     for (int i = p.nx - 1; i >= i_end; --i) {
         const int slot = i & 1;
+        if (!cb) {
+            bool over = false;
+            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev1, s, over));
+            if (over) break;
+        }
         if (p.resort_every > 0 && i < p.nx - 1 && ((p.nx - 1 - i) % p.resort_every) == 0 && m->P.np)
             QP_TRY(resort(R, s));
         const bool generic = (i < p.nx - 1) && (i > 0) && (p.K > 0);
@@ -2443,8 +2448,18 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
         cctx[b] = GroupCbCtx{cb, user, b};
     }
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
+    CtlSets cs{};
+    for (Wake *w : G->b) {
+        cs.ctl[cs.nb] = w->ctl;
+        cs.nw[cs.nb++] = w->nw;
+    }
     for (int i = p.nx - 1; i >= i_end; --i) {
         const int slot = i & 1;
+        if (!cb) {
+            bool over = false;
+            QP_TRY(watch_stops(cs, p.nx - 1 - i, G->b[0]->h_running(), G->ev1, s, over));
+            if (over) break;
+        }
         const bool generic = (i < p.nx - 1) && (i > 0) && (p.K > 0);
         if (graph_ok && generic) {
             if (!st->gexec[slot]) {
