@@ -216,6 +216,7 @@ int qp_wake_destroy(qp_wake h) {
     if (w->h_out) (void)hipHostFree(w->h_out);
     if (w->ev0) (void)hipEventDestroy(w->ev0);
     if (w->ev1) (void)hipEventDestroy(w->ev1);
+    if (w->ev_mark) (void)hipEventDestroy(w->ev_mark);
     for (hipEvent_t e : w->prof_ev) (void)hipEventDestroy(e);
     delete h;
     return QP_OK;

@@ -38,13 +38,13 @@ __global__ __launch_bounds__(64) void k_running(CtlSets c, int *count) {
 
 }  // namespace
 
-int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t ev, hipStream_t s, bool &over) {
-    over = false;
+int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t &ev, hipStream_t s, int &running) {
     if (done == 0 || done % kWatchSlices != 0) return QP_OK;
+    if (!ev) QP_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     if (done > kWatchSlices) {  // the mark before this one
         QP_HIP_CHECK(hipEventSynchronize(ev));
-        over = *count == 0;
-        if (over) return QP_OK;
+        running = *count;
+        if (!running) return QP_OK;
     }
     hipLaunchKernelGGL(k_running, dim3(1), dim3(64), 0, s, c, count);
     QP_HIP_CHECK(hipGetLastError());

@@ -37,9 +37,10 @@ struct CtlSets {               // the control blocks of a launch's batches
     int nw[kGroupMax];
     int nb;
 };
-// Before slice number `done` (from 0) of a pass: over = every member had stopped at the last
-// mark.  `count` is pinned; `ev` may be recorded anew after the pass.
-int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t ev, hipStream_t s, bool &over);
+// Before slice number `done` (from 0) of a pass: sets `running` to the members that ran at
+// the last mark, where a mark is due.  `count` is pinned; `ev` is made at the first mark
+// (45 us; without time stamps: with them each mark took 14 us, not 3).
+int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t &ev, hipStream_t s, int &running);
 
 // Host data of one member of a batch of wakes (a single wake is a batch of
 // one): the initial particles (FP64, re-uploaded every pass) and the laser.
@@ -78,6 +79,7 @@ struct Wake {
     Ctl *ctl = nullptr;                  // nw control blocks
     double *h_out = nullptr;             // pinned host staging, 12 planes, a control block, a count of members
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipEvent_t ev_mark = nullptr;        // watch_stops
     double last_ms = 0.0;
     // mixed path: particle tile (threads per block, LDS window nodes per grid),
     // from the tile autotuner on the first pass unless set by QP_TILE

@@ -478,9 +478,9 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
     const CtlSets cs = w->ctl_set();
     for (int i = p.nx - 1; i >= i_end; --i) {
         if (!cb) {
-            bool over = false;
-            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev1, s, over));
-            if (over) break;
+            int running = 1;
+            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev_mark, s, running));
+            if (!running) break;
         }
         const double *asq;
         QP_TRY(wake_asq_slice(w, i, &asq));

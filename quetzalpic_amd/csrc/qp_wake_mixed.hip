@@ -47,6 +47,19 @@ namespace qp {
         return;                   \
     }
 
+// The push launches load particles beside the stop flag.  Once some members of a batch or
+// group have stopped while others run (the host learns it at a mark or from the output),
+// instances that test the flag first (FF) take their place, so that a stopped member costs
+// no reads.  A template parameter: as an argument the test cost passes without a stopped
+// member 0.4-0.7 % (beam step of 1024^2 166.5 -> 167.8 ms), as the only form 1.0-2.4 %.
+#define MX_FLAG_FIRST(FF, ctl)                  \
+    if constexpr (FF) {                         \
+        if (ctl_skip(ctl)) {                    \
+            ctl_latch(ctl);                     \
+            return;                             \
+        }                                       \
+    }
+
 // ------------------------------------------------------------------ A phase
 // Commit and advance (src/System_3d.cpp:593-608), then deposit -n at the new
 // position into the psi source accumulator (:349-353).  The grid part
@@ -54,10 +67,11 @@ namespace qp {
 // first jx (:381-388).  The block's cell window is kept for the B phase.
 // Batches: blockIdx.y is the member; its grids sit at + member * nn, its
 // particles at + member * pstride, its control block at ctl + member.
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 __device__ __forceinline__ void mx_A(MxPart P, MxGeom g, MxSliceIn si, const double *psim, double *src_acc,
                                               double *asq2, const LaserGauss *Ls, int laser, double *rho, double *jx,
                                               double *chi, int advance, Ctl *ctl, int bx, int wk, int gx) {
+    MX_FLAG_FIRST(FF, ctl + wk);
     // The particle's state is loaded before the control block is checked: the
     // index stays inside the member's allocation (pstride is a whole number of
     // blocks), so these loads share a round trip with the control block's.
@@ -151,11 +165,11 @@ __device__ __forceinline__ void mx_A(MxPart P, MxGeom g, MxSliceIn si, const dou
         chi[t] = 0.0;
     }
 }
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 __global__ __launch_bounds__(PT) void k_mx_A(MxPart P, MxGeom g, MxSliceIn si, const double *psim, double *src_acc,
                                               double *asq2, const LaserGauss *Ls, int laser, double *rho, double *jx,
                                               double *chi, int advance, Ctl *ctl) {
-    mx_A<PT, CAP>(P, g, si, psim, src_acc, asq2, Ls, laser, rho, jx, chi, advance, ctl, blockIdx.x, blockIdx.y,
+    mx_A<PT, CAP, FF>(P, g, si, psim, src_acc, asq2, Ls, laser, rho, jx, chi, advance, ctl, blockIdx.x, blockIdx.y,
          gridDim.x);
 }
 
@@ -187,7 +201,7 @@ constexpr int b_waves(int PT, int CAP, bool RHO, bool CHI) {
 // leaves its cell by more than one (such a particle deposits with global atomics).  So
 // the launch starts with the window's grid loads beside the particle loads, and finds
 // no window of its own: no reductions over the block, two barriers fewer, one flush.
-template <int PT, int CAP, bool RHO, bool CHI>
+template <int PT, int CAP, bool RHO, bool CHI, bool FF>
 __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const double *psi, const double *by,
                                               const double *bz, double *src_acc, double *rho, double *jx,
                                               double *jx_next, double *chi, double *jyn, double *jzn, int it,
@@ -195,6 +209,7 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
     constexpr int G = 1 + (RHO ? 1 : 0) + (CHI ? 1 : 0);  // node grids
     __shared__ double lds[b_lds(CAP, RHO, CHI)];  // the staged grids, then (behind a barrier) the deposit windows
     ctl += wk;
+    MX_FLAG_FIRST(FF, ctl);
     const int stop = ctl->stop_acc;
     const int n1 = g.n1, n2 = g.n2;
     const size_t nn = (size_t)n1 * n2, go = (size_t)wk * nn;
@@ -330,12 +345,12 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
     }
     if (bx == 0 && threadIdx.x == 0) ctl->iter = it;
 }
-template <int PT, int CAP, bool RHO, bool CHI>
+template <int PT, int CAP, bool RHO, bool CHI, bool FF>
 __global__ __launch_bounds__(PT, b_waves(PT, CAP, RHO, CHI)) void k_mx_B(MxPart P, MxGeom g, MxSliceIn si, const double *psi, const double *by,
                                               const double *bz, double *src_acc, double *rho, double *jx,
                                               double *jx_next, double *chi, double *jyn, double *jzn, int it,
                                               Ctl *ctl) {
-    mx_B<PT, CAP, RHO, CHI>(P, g, si, psi, by, bz, src_acc, rho, jx, jx_next, chi, jyn, jzn, it, ctl, blockIdx.x,
+    mx_B<PT, CAP, RHO, CHI, FF>(P, g, si, psi, by, bz, src_acc, rho, jx, jx_next, chi, jyn, jzn, it, ctl, blockIdx.x,
          blockIdx.y, gridDim.x);
 }
 
@@ -343,11 +358,12 @@ __global__ __launch_bounds__(PT, b_waves(PT, CAP, RHO, CHI)) void k_mx_B(MxPart 
 // jy*, jz* at the half-step positions.  The deposit window is the block's cell window
 // with the row and column each side that a half step reaches, and one more ahead (the
 // half-cell stencils start at cell or cell - 1).
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 __device__ __forceinline__ void mx_C(MxPart P, MxGeom g, const double *psim, double *jyn, double *jzn, Ctl *ctl, int bx,
                                      int wk) {
     __shared__ double lds[2 * CAP];
     ctl += wk;
+    MX_FLAG_FIRST(FF, ctl);
     const int stop = ctl->stop_acc;
     const int n1 = g.n1, n2 = g.n2;
     const size_t go = (size_t)wk * n1 * n2;
@@ -400,9 +416,9 @@ __device__ __forceinline__ void mx_C(MxPart P, MxGeom g, const double *psim, dou
     double *gl[2] = {jyn, jzn};
     win_flush<CAP>(lds, gl, 2, win, n1, n2);
 }
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 __global__ __launch_bounds__(PT) void k_mx_C(MxPart P, MxGeom g, const double *psim, double *jyn, double *jzn, Ctl *ctl) {
-    mx_C<PT, CAP>(P, g, psim, jyn, jzn, ctl, blockIdx.x, blockIdx.y);
+    mx_C<PT, CAP, FF>(P, g, psim, jyn, jzn, ctl, blockIdx.x, blockIdx.y);
 }
 
 // -------------------------------------------------- S phase (slice 0, K = 0)
@@ -964,28 +980,28 @@ struct GArgsRowsI {
 // argument segment): left alone the compiler holds more of them in vector
 // registers than the single-batch kernels do (A 68 against 50).  The bounds keep
 // 7 or 8 waves at 256 threads without scratch (B as k_mx_B, A 64 VGPRs).
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 __global__ __launch_bounds__(PT, 8) void kg_mx_A(GrpMap m, const GArgsA *__restrict__ t, int advance) {
     int b, bx, wk;
     grp_locate(m, b, bx, wk);
     const GArgsA &a = t[b];
-    mx_A<PT, CAP>(a.P, a.g, a.si, a.psim, a.src_acc, a.asq2, a.Ls, a.laser, a.rho, a.jx, a.chi, advance, a.ctl, bx, wk,
+    mx_A<PT, CAP, FF>(a.P, a.g, a.si, a.psim, a.src_acc, a.asq2, a.Ls, a.laser, a.rho, a.jx, a.chi, advance, a.ctl, bx, wk,
          m.gx[b]);
 }
-template <int PT, int CAP, bool RHO, bool CHI>
+template <int PT, int CAP, bool RHO, bool CHI, bool FF>
 __global__ __launch_bounds__(PT, b_waves(PT, CAP, RHO, CHI)) void kg_mx_B(GrpMap m, const GArgsB *__restrict__ t, int it) {
     int b, bx, wk;
     grp_locate(m, b, bx, wk);
     const GArgsB &a = t[b];
-    mx_B<PT, CAP, RHO, CHI>(a.P, a.g, a.si, a.psi, a.by, a.bz, a.src_acc, a.rho, a.jx, RHO ? nullptr : a.jx_next, a.chi,
-                            a.jyn, a.jzn, it, a.ctl, bx, wk, m.gx[b]);
+    mx_B<PT, CAP, RHO, CHI, FF>(a.P, a.g, a.si, a.psi, a.by, a.bz, a.src_acc, a.rho, a.jx, RHO ? nullptr : a.jx_next, a.chi,
+                                a.jyn, a.jzn, it, a.ctl, bx, wk, m.gx[b]);
 }
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 __global__ __launch_bounds__(PT, 8) void kg_mx_C(GrpMap m, const GArgsC *__restrict__ t) {
     int b, bx, wk;
     grp_locate(m, b, bx, wk);
     const GArgsC &a = t[b];
-    mx_C<PT, CAP>(a.P, a.g, a.psim, a.jyn, a.jzn, a.ctl, bx, wk);
+    mx_C<PT, CAP, FF>(a.P, a.g, a.psim, a.jyn, a.jzn, a.ctl, bx, wk);
 }
 template <int PT, int CAP>
 __global__ __launch_bounds__(PT) void kg_mx_S(GrpMap m, const GArgsS *__restrict__ t) {
@@ -1105,7 +1121,7 @@ struct MixedState {
     // the step it stopped in.  [0] are the wake's own, [1] belong to this state.
     double *rho2[2] = {nullptr, nullptr}, *jx2[2] = {nullptr, nullptr};
     std::vector<int> h_perm;
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    hipGraphExec_t gexec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [flag_first][slice parity]
     unsigned graph_epoch = 0;  // Wake::inputs_epoch the graphs were captured at
     int graph_pt = 0, graph_cap = 0;  // particle tile the graphs were captured with
     // streamed output (async_output): per-slice snapshots of the output planes
@@ -1131,6 +1147,14 @@ static MixedState *mstate(Wake *w) { return static_cast<MixedState *>(w->mixed);
 static hipError_t copy_wait(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
     hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
+static void drop_graphs(hipGraphExec_t (&gexec)[2][2]) {
+    for (auto &v : gexec)
+        for (hipGraphExec_t &g : v) {
+            if (g) (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
 }
 
 static void free_part(MxPart &P) {
@@ -1167,8 +1191,7 @@ void wake_destroy_mixed(Wake *w) {
                     m->totals,     m->bpart,      m->rho2[1],    m->jx2[1],     m->jbuf[0][0], m->jbuf[0][1], m->jbuf[1][0], m->jbuf[1][1]};
     for (void *a : arrs)
         if (a) (void)hipFree(a);
-    for (auto &g : m->gexec)
-        if (g) (void)hipGraphExecDestroy(g);
+    drop_graphs(m->gexec);
     if (m->snap_dev) (void)hipFree(m->snap_dev);
     if (m->snap_host) (void)hipHostFree(m->snap_host);
     for (hipEvent_t e : {m->ev_done[0], m->ev_done[1], m->ev_copied[0], m->ev_copied[1]})
@@ -1230,9 +1253,7 @@ static int ensure_state(Wake *w) {
         QP_HIP_CHECK(hipMalloc(&m->perm0, sizeof(int) * need));
         m->cap = need;
         m->init_valid = false;
-        for (auto &g : m->gexec)
-            if (g) (void)hipGraphExecDestroy(g);
-        m->gexec[0] = m->gexec[1] = nullptr;
+        drop_graphs(m->gexec);
     }
     m->pstride = pstride;
     std::vector<int> hn(nw);
@@ -1369,6 +1390,7 @@ struct MxRun {
     size_t sstride;
     size_t ldsS;
     int pt, cap;   // particle tile: threads per block, LDS window nodes per grid
+    int flag_first = 0;   // some member has stopped (MX_FLAG_FIRST)
 };
 
 // The instantiated particle tiles (threads per block, window nodes per grid).
@@ -1519,7 +1541,7 @@ int bx_solve(MxRun &R, hipStream_t s, int slot) {
 }
 
 // Enqueue the work of slice i (everything between two output steps) for every member.
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
     Wake *w = R.w;
     MixedState *m = R.m;
@@ -1533,7 +1555,7 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
     const dim3 pg(R.pb, R.nw);
     if (w->bunch) QP_TRY(bunch_slice_sources(w->bunch, (const Ctl *)w->ctl, slot, 0, s));
     prof_begin(w, "push_A");
-    MLAUNCH((k_mx_A<PT, CAP>), pg, PT, 0, m->P, R.g, si, (const double *)w->psim, w->src, w->asq2,
+    MLAUNCH((k_mx_A<PT, CAP, FF>), pg, PT, 0, m->P, R.g, si, (const double *)w->psim, w->src, w->asq2,
             (const LaserGauss *)w->d_laser, laser, m->rho2[slot], m->jx2[0], w->chi,
             first ? 0 : (p.K == 0 ? 2 : 1), w->ctl);
     prof_end(w, "push_A");
@@ -1553,7 +1575,7 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
             double *jx = m->jx2[it & 1], *jx_next = last_it ? nullptr : m->jx2[(it + 1) & 1];
             prof_begin(w, "push_B");
             QP_TRY(with_flags(last_it, first_it, [&](auto RH, auto CH) {
-                MLAUNCH((k_mx_B<PT, CAP, decltype(RH)::value, decltype(CH)::value>), pg, PT, 0, m->P, R.g, si,
+                MLAUNCH((k_mx_B<PT, CAP, decltype(RH)::value, decltype(CH)::value, FF>), pg, PT, 0, m->P, R.g, si,
                         (const double *)psi, (const double *)w->by, (const double *)w->bz, w->src, m->rho2[slot], jx,
                         jx_next, w->chi, m->jbuf[slot][0], m->jbuf[slot][1], it, w->ctl);
                 return QP_OK;
@@ -1561,7 +1583,7 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
             prof_end(w, "push_B");
             QP_TRY(psi_solve(R, s, slot, w->psim));
             prof_begin(w, "push_C");
-            MLAUNCH((k_mx_C<PT, CAP>), pg, PT, 0, m->P, R.g, (const double *)w->psim, m->jbuf[slot][0],
+            MLAUNCH((k_mx_C<PT, CAP, FF>), pg, PT, 0, m->P, R.g, (const double *)w->psim, m->jbuf[slot][0],
                     m->jbuf[slot][1], w->ctl);
             prof_end(w, "push_C");
             QP_TRY(b_solve(R, s, slot, jx));
@@ -1579,7 +1601,10 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
 }
 
 int enqueue_slice(MxRun &R, hipStream_t s, int i) {
-    return with_tile(R.pt, R.cap, [&](auto P, auto C) { return enqueue_slice_t<decltype(P)::value, decltype(C)::value>(R, s, i); });
+    return with_tile(R.pt, R.cap, [&](auto P, auto C) {
+        constexpr int PT = decltype(P)::value, CAP = decltype(C)::value;
+        return R.flag_first ? enqueue_slice_t<PT, CAP, true>(R, s, i) : enqueue_slice_t<PT, CAP, false>(R, s, i);
+    });
 }
 
 int resort(MxRun &R, hipStream_t s) {
@@ -1702,7 +1727,7 @@ struct OutQueue {
     std::deque<std::pair<int, int>> jobs;  // (slice, host slot)
     std::vector<char> slot_free;
     bool closed = false;
-    std::atomic<bool> all_stopped{false};
+    std::atomic<int> running{0};  // members that had not stopped at the last job
     std::atomic<bool> failed{false};
     std::string error;
 };
@@ -1748,7 +1773,7 @@ void writer_loop(Wake *w, MixedState *m, OutQueue *q, batch_cb cb, void *user, s
                     q->failed = true;
                 }
             }
-            if (!running) q->all_stopped = true;
+            q->running = running;
         }
         {
             std::lock_guard<std::mutex> lk(q->mu);
@@ -1786,9 +1811,7 @@ int pass_setup(Wake *w, MxRun &R) {
         R.si[sl] = MxSliceIn{w->asq3(), w->asq2, w->rho_b_src(), w->jx_b_src(), w->bsrc_stride(), sl};
     // captured slice steps hold the driver pointers and flags of their inputs
     if (m->graph_epoch != w->inputs_epoch || m->graph_pt != R.pt || m->graph_cap != R.cap) {
-        for (auto &g : m->gexec)
-            if (g) (void)hipGraphExecDestroy(g);
-        m->gexec[0] = m->gexec[1] = nullptr;
+        drop_graphs(m->gexec);
         m->graph_epoch = w->inputs_epoch;
         m->graph_pt = R.pt;
         m->graph_cap = R.cap;
@@ -2037,6 +2060,7 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
     if (async) {
         QP_TRY(ensure_snapshots(w, m));
         q.slot_free.assign(kHostSlots, 1);
+        q.running = nw;
         writer = std::thread(writer_loop, w, m, &q, cb, user, &delivered_stop);
     }
     // ends the writer (after the jobs queued so far) on every exit path
@@ -2055,18 +2079,20 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
     } join{q, writer};
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
     const CtlSets cs = w->ctl_set();
+    int running = nw;
     for (int i = p.nx - 1; i >= i_end; --i) {
         const int slot = i & 1;
         if (!cb) {
-            bool over = false;
-            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev1, s, over));
-            if (over) break;
+            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev_mark, s, running));
+            if (!running) break;
         }
+        R.flag_first = running < nw;
         if (p.resort_every > 0 && i < p.nx - 1 && ((p.nx - 1 - i) % p.resort_every) == 0 && m->P.np)
             QP_TRY(resort(R, s));
         const bool generic = (i < p.nx - 1) && (i > 0) && (p.K > 0);
         if (graph_ok && generic) {
-            if (!m->gexec[slot]) {
+            hipGraphExec_t &gexec = m->gexec[R.flag_first][slot];
+            if (!gexec) {
                 hipGraph_t gr;
                 QP_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
                 int st = enqueue_slice(R, s, i);
@@ -2079,14 +2105,14 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
                     set_error(std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
                     return QP_ERR_HIP;
                 }
-                e = hipGraphInstantiate(&m->gexec[slot], gr, nullptr, nullptr, 0);
+                e = hipGraphInstantiate(&gexec, gr, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(gr);
                 if (e != hipSuccess) {
                     set_error(std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
                     return QP_ERR_HIP;
                 }
             }
-            QP_HIP_CHECK(hipGraphLaunch(m->gexec[slot], s));
+            QP_HIP_CHECK(hipGraphLaunch(gexec, s));
         } else {
             QP_TRY(enqueue_slice(R, s, i));
         }
@@ -2114,9 +2140,9 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
                 q.jobs.emplace_back(i, h);
             }
             q.cv.notify_all();
-            if (q.failed || q.all_stopped) break;
+            running = q.running;
+            if (q.failed || !running) break;
         } else if (cb && i > 0) {
-            int running = 0;
             QP_TRY(deliver_inline(w, R, cb, user, i, delivered_stop, hc, running));
             if (!running) break;
         }
@@ -2177,7 +2203,7 @@ struct GroupState {
     GroupTabs *d_tabs = nullptr;
     GroupTabs h_tabs;
     GroupMaps maps{}, graph_maps{};
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
+    hipGraphExec_t gexec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // [flag_first][slice parity]
     std::vector<unsigned> graph_epochs;
 };
 
@@ -2276,7 +2302,7 @@ void group_tables(Group *G, std::vector<MxRun> &R, GroupTabs &T, GroupMaps &M) {
     } while (0)
 
 // One slice step of every batch: enqueue_slice with one launch per phase.
-template <int PT, int CAP>
+template <int PT, int CAP, bool FF>
 int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
     const qp_wake_params &p = G->b[0]->p;
     const GroupMaps &M = st->maps;
@@ -2284,7 +2310,7 @@ int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
     const int slot = i & 1;
     const bool first = (i == p.nx - 1);
     const bool s_phase = (i == 0) || (p.K == 0);
-    GLAUNCH((kg_mx_A<PT, CAP>), M.part, PT, 0, T->A[slot], first ? 0 : (p.K == 0 ? 2 : 1));
+    GLAUNCH((kg_mx_A<PT, CAP, FF>), M.part, PT, 0, T->A[slot], first ? 0 : (p.K == 0 ? 2 : 1));
     GROWS(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
     GCOLS(M.cols1, 1, T->PC);
     GROWS(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->PI[slot]);
@@ -2295,14 +2321,14 @@ int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
         for (int it = 0; it < p.K; ++it) {
             const bool first_it = it == 0, last_it = it == p.K - 1;
             QP_TRY(with_flags(last_it, first_it, [&](auto RH, auto CH) {
-                GLAUNCH((kg_mx_B<PT, CAP, decltype(RH)::value, decltype(CH)::value>), M.part, PT, 0, T->B[slot][it & 1],
-                        it);
+                GLAUNCH((kg_mx_B<PT, CAP, decltype(RH)::value, decltype(CH)::value, FF>), M.part, PT, 0,
+                        T->B[slot][it & 1], it);
                 return QP_OK;
             }));
             GROWS(kg_rows_fwd, SrcPsi, M.rows1, 1, T->PF[slot]);
             GCOLS(M.cols1, 1, T->PC);
             GROWS(kg_rows_inv, SinkPsiFinal, M.rows1, 1, T->MI);
-            GLAUNCH((kg_mx_C<PT, CAP>), M.part, PT, 0, T->C[slot]);
+            GLAUNCH((kg_mx_C<PT, CAP, FF>), M.part, PT, 0, T->C[slot]);
             GROWS(kg_rows_fwd, SrcB, M.rows2, 2, T->BF[slot][it & 1]);
             GCOLS(M.cols2, 2, T->BC);
             GROWS(kg_rows_inv, SinkBPair, M.rows2, 2, T->BI[slot]);
@@ -2312,9 +2338,10 @@ int enqueue_group_t(Group *G, GroupState *st, hipStream_t s, int i) {
     return QP_OK;
 }
 
-int enqueue_group(Group *G, GroupState *st, hipStream_t s, int i) {
+int enqueue_group(Group *G, GroupState *st, hipStream_t s, int i, int flag_first) {
     return with_tile(G->b[0]->tile_pt, G->b[0]->tile_cap, [&](auto P, auto C) {
-        return enqueue_group_t<decltype(P)::value, decltype(C)::value>(G, st, s, i);
+        constexpr int PT = decltype(P)::value, CAP = decltype(C)::value;
+        return flag_first ? enqueue_group_t<PT, CAP, true>(G, st, s, i) : enqueue_group_t<PT, CAP, false>(G, st, s, i);
     });
 }
 
@@ -2370,8 +2397,7 @@ int group_member_cb(int member, const qp_slice_view *v, void *u) {
 void group_destroy_mixed(Group *G) {
     GroupState *st = static_cast<GroupState *>(G->dev);
     if (!st) return;
-    for (auto &g : st->gexec)
-        if (g) (void)hipGraphExecDestroy(g);
+    drop_graphs(st->gexec);
     if (st->d_tabs) (void)hipFree(st->d_tabs);
     delete st;
     G->dev = nullptr;
@@ -2428,9 +2454,7 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
     for (int b = 0; b < nb; ++b) epochs[b] = G->b[b]->inputs_epoch;
     epochs.push_back((unsigned)G->tile_cap);   // the maps carry the block counts of the tile, not its capacity
     if (std::memcmp(&st->maps, &st->graph_maps, sizeof(GroupMaps)) != 0 || epochs != st->graph_epochs) {
-        for (auto &g : st->gexec)
-            if (g) (void)hipGraphExecDestroy(g);
-        st->gexec[0] = st->gexec[1] = nullptr;
+        drop_graphs(st->gexec);
         st->graph_maps = st->maps;
         st->graph_epochs = epochs;
     }
@@ -2449,23 +2473,27 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
     }
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
     CtlSets cs{};
+    int members = 0;
     for (Wake *w : G->b) {
         cs.ctl[cs.nb] = w->ctl;
         cs.nw[cs.nb++] = w->nw;
+        members += w->nw;
     }
+    int running = members;
     for (int i = p.nx - 1; i >= i_end; --i) {
         const int slot = i & 1;
         if (!cb) {
-            bool over = false;
-            QP_TRY(watch_stops(cs, p.nx - 1 - i, G->b[0]->h_running(), G->ev1, s, over));
-            if (over) break;
+            QP_TRY(watch_stops(cs, p.nx - 1 - i, G->b[0]->h_running(), G->b[0]->ev_mark, s, running));
+            if (!running) break;
         }
+        const int flag_first = running < members;
         const bool generic = (i < p.nx - 1) && (i > 0) && (p.K > 0);
         if (graph_ok && generic) {
-            if (!st->gexec[slot]) {
+            hipGraphExec_t &gexec = st->gexec[flag_first][slot];
+            if (!gexec) {
                 hipGraph_t gr;
                 QP_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                int rc = enqueue_group(G, st, s, i);
+                int rc = enqueue_group(G, st, s, i, flag_first);
                 hipError_t e = hipStreamEndCapture(s, &gr);
                 if (rc < 0) {
                     if (e == hipSuccess) (void)hipGraphDestroy(gr);
@@ -2475,19 +2503,19 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
                     set_error(std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
                     return QP_ERR_HIP;
                 }
-                e = hipGraphInstantiate(&st->gexec[slot], gr, nullptr, nullptr, 0);
+                e = hipGraphInstantiate(&gexec, gr, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(gr);
                 if (e != hipSuccess) {
                     set_error(std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
                     return QP_ERR_HIP;
                 }
             }
-            QP_HIP_CHECK(hipGraphLaunch(st->gexec[slot], s));
+            QP_HIP_CHECK(hipGraphLaunch(gexec, s));
         } else {
-            QP_TRY(enqueue_group(G, st, s, i));
+            QP_TRY(enqueue_group(G, st, s, i, flag_first));
         }
         if (cb && i > 0) {
-            int running = 0;
+            running = 0;
             for (int b = 0; b < nb; ++b) {
                 int rb = 0;
                 QP_TRY(deliver_inline(G->b[b], R[b], group_member_cb, &cctx[b], i, delivered_stop[b], hc[b], rb));
