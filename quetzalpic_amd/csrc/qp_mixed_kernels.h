@@ -386,24 +386,35 @@ __device__ inline Win block_window(int rmin, int rmax, int cmin, int cmax, int j
 }
 
 // A window kept for a later launch of the same block, with `lo` rows and columns
-// more ahead of it and `hi` more behind it (each below the grid's sides).
+// more ahead of it and `hi` more behind it (each below the grid's sides): padded.  Where
+// that does not fit the sides or the capacity, the kept window itself, if it does: it
+// holds the deposits at the cells and most of those a half step away (the others, at its
+// rim, take global atomics).  So blocks that straddle two tiles, as after a re-binning
+// (17 x 33 nodes, padded 19 x 35 or 20 x 36), keep their window: of a 1024^2 x 120-slice
+// wake re-binned every 20 slices 3.2 % of the blocks had none, now 0.09 % (152.5 -> 138.8 ms).
 template <int CAP>
-__device__ __forceinline__ Win win_load(const int4 *t, int blk, int lo, int hi, int n1, int n2) {
+__device__ __forceinline__ Win win_load(const int4 *t, int blk, int lo, int hi, int n1, int n2, bool &padded) {
     const int4 d = t[blk];
     Win w;
-    w.j0 = __builtin_amdgcn_readfirstlane(d.x) - lo;
-    w.k0 = __builtin_amdgcn_readfirstlane(d.y) - lo;
+    w.j0 = __builtin_amdgcn_readfirstlane(d.x);
+    w.k0 = __builtin_amdgcn_readfirstlane(d.y);
     w.wj = __builtin_amdgcn_readfirstlane(d.z);
     w.wk = __builtin_amdgcn_readfirstlane(d.w);
     if (w.wj == 0) {  // a block without particles
         w.j0 = w.k0 = 0;
-        w.lds = true;
+        w.lds = padded = true;
         return w;
     }
-    if (w.j0 < 0) w.j0 += n1;
-    if (w.k0 < 0) w.k0 += n2;
-    w.wj += lo + hi;
-    w.wk += lo + hi;
+    const int pj = w.wj + lo + hi, pk = w.wk + lo + hi;
+    padded = pj <= n1 && pk <= n2 && pj * pk <= CAP;
+    if (padded) {
+        w.j0 -= lo;
+        w.k0 -= lo;
+        if (w.j0 < 0) w.j0 += n1;
+        if (w.k0 < 0) w.k0 += n2;
+        w.wj = pj;
+        w.wk = pk;
+    }
     w.lds = (w.wj <= n1 && w.wk <= n2 && w.wj * w.wk <= CAP);
     return w;
 }

@@ -198,7 +198,8 @@ constexpr int b_waves(int PT, int CAP, bool RHO, bool CHI) {
 // One window serves the launch: rows and columns -1 .. +2 around the block's cells,
 // from the cell window that the A phase kept.  It holds every node of the gathers and
 // of the deposits at the cells, and those of the half-step deposit unless the half step
-// leaves its cell by more than one (such a particle deposits with global atomics).  So
+// leaves its cell by more than one (such a particle deposits with global atomics; so do
+// more of them where the window is not padded, which is not staged either).  So
 // the launch starts with the window's grid loads beside the particle loads, and finds
 // no window of its own: no reductions over the block, two barriers fewer, one flush.
 template <int PT, int CAP, bool RHO, bool CHI, bool FF>
@@ -233,13 +234,14 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
     const double2 pp = P.p[p];
     double2 pst = make_double2(0.0, 0.0);
     if (!CHI) pst = P.ps[p];  // P6 of the previous iteration (:503-505)
-    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 1, 1, n1, n2);
+    bool padded;
+    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 1, 1, n1, n2, padded);
     if (stop) {
         ctl_latch(ctl);
         return;
     }
     const double *asq = mx_asq(ctl, si, nn, go);
-    const bool staged = win.lds && win.wj * win.wk <= kGwCap;
+    const bool staged = padded && win.wj * win.wk <= kGwCap;
     if (staged) {
         const double *src[4] = {psi, asq, by, bz};
         gwin_load<4>(lds, kGwCap, src, win, n1, n2);
@@ -379,7 +381,8 @@ __device__ __forceinline__ void mx_C(MxPart P, MxGeom g, const double *psim, dou
     double vjy = 0, vjz = 0;
     const double w = P.w[p], iv = P.iv[p];
     const double2 pst = P.ps[p];
-    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 2, 1, n1, n2);
+    bool padded;
+    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 2, 1, n1, n2, padded);
     if (stop) {
         ctl_latch(ctl);
         return;
