@@ -354,22 +354,24 @@ int pipe_depth(const Envelope *e) {
     return (int)std::max<size_t>(1, std::min<size_t>(16, ((size_t)1 << 20) / e->nn()));
 }
 
-// Spectra and increments of `depth` steps in flight (kept: 2^20 nodes take 50 MB).
-int ensure_pipe(Envelope *e, int depth) {
+// Spectra and increments of `depth` steps in flight (kept: 2^20 nodes take 50 MB).  Where
+// the device has no room for them, of half as many, down to one step, which needs neither;
+// depth: what the envelope can run.
+int ensure_pipe(Envelope *e, int &depth) {
     if (depth <= std::max(1, e->pipe)) return QP_OK;
-    drop_graph(e);
     QP_HIP_CHECK(hipStreamSynchronize(e->stream()));
-    if (e->pipe_inc) (void)hipFree(e->pipe_inc);
-    if (e->pipe_spec) (void)hipFree(e->pipe_spec);
-    e->pipe_inc = nullptr;
-    e->pipe_spec = nullptr;
-    e->pipe = 0;
-    QP_HIP_CHECK(hipMalloc(&e->pipe_inc, sizeof(double) * 4 * e->nn() * depth));
-    if (hipMalloc(&e->pipe_spec, sizeof(double2) * 2 * (size_t)e->S.n1 * e->S.nh * depth) != hipSuccess) {
-        (void)hipFree(e->pipe_inc);
+    drop_graph(e);
+    for (;; depth /= 2) {
+        if (e->pipe_inc) (void)hipFree(e->pipe_inc);
+        if (e->pipe_spec) (void)hipFree(e->pipe_spec);
         e->pipe_inc = nullptr;
-        set_error("envelope: device allocation failed");
-        return QP_ERR_ALLOC;
+        e->pipe_spec = nullptr;
+        e->pipe = 0;
+        if (depth <= 1) return QP_OK;
+        if (hipMalloc(&e->pipe_inc, sizeof(double) * 4 * e->nn() * depth) == hipSuccess &&
+            hipMalloc(&e->pipe_spec, sizeof(double2) * 2 * (size_t)e->S.n1 * e->S.nh * depth) == hipSuccess)
+            break;
+        (void)hipGetLastError();
     }
     e->pipe = depth;
     return QP_OK;
@@ -621,6 +623,7 @@ int qp_envelope_advance(qp_envelope h, double dtau, int steps, int chi_iteration
     EARG_CHECK(chi_iterations >= 0 && chi_iterations <= 16, "qp_envelope_advance: chi_iterations in [0, 16]");
     Envelope *e = &h->e;
     hipStream_t s = e->stream();
+    QP_HIP_CHECK(hipSetDevice(e->ctx->device));  // (it may allocate)
     struct Events {
         hipEvent_t a = nullptr, b = nullptr;
         ~Events() {
@@ -636,9 +639,11 @@ int qp_envelope_advance(qp_envelope h, double dtau, int steps, int chi_iteration
     if (steps > 0) ELAUNCH(k_env_cmid, dim3(e->nx), kET, 0, (const double *)e->chi3, e->cmid, e->nn());
     // pipelines of nearly equal depth; a graph for the deeper ones, the shallower (one
     // step less, at most) launched directly
-    const int groups = steps > 0 ? (steps + pipe_depth(e) - 1) / pipe_depth(e) : 0;
+    auto split = [steps](int depth) { return steps > 0 ? (steps + depth - 1) / depth : 0; };
+    int groups = split(pipe_depth(e)), depth = groups ? (steps + groups - 1) / groups : 1;
+    QP_TRY(ensure_pipe(e, depth));
+    groups = split(depth);
     const int deep = groups ? (steps + groups - 1) / groups : 0;
-    QP_TRY(ensure_pipe(e, deep));
     for (int g = 0, left = steps; g < groups; ++g) {
         const int ns = (left + groups - g - 1) / (groups - g);
         QP_TRY(env_run(e, dtau, chi_iterations, ns, use_graph && ns == deep, s));
