@@ -16,6 +16,8 @@
 
 namespace qp {
 
+constexpr int kEnvPipeMax = 16;  // steps in flight
+
 struct Envelope {
     qp_ctx_s *ctx = nullptr;
     int nx = 0, ny = 0, nz = 0;
@@ -33,10 +35,13 @@ struct Envelope {
     size_t njoin = 0;
     std::mutex join_lock;
     int attached = 0;        // wakes reading this envelope
-    hipGraphExec_t gexec = nullptr;  // g_steps steps, captured for dtau = g_dtau, g_iter chi corrections
+    // Captured pipelines by their number of steps, all for dtau = g_dtau, g_iter chi
+    // corrections and stream g_stream; g_seen: a pipeline of that many steps has run.
+    hipGraphExec_t gexec[kEnvPipeMax + 1] = {};
+    bool g_seen[kEnvPipeMax + 1] = {};
     double g_dtau = 0.0;
-    int g_iter = 0, g_steps = 0;
-    hipStream_t g_stream = nullptr;  // stream the graph was captured on
+    int g_iter = 0;
+    hipStream_t g_stream = nullptr;
 
     size_t nn() const { return (size_t)ny * nz; }
     size_t vol() const { return (size_t)nx * nn(); }

@@ -297,9 +297,12 @@ __global__ __launch_bounds__(kGenThreads) void kg_cols_env(double2 *spec0, doubl
         QP_HIP_CHECK(hipGetLastError());                                      \
     } while (0)
 
-void drop_graph(Envelope *e) {
-    if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
-    e->gexec = nullptr;
+void drop_graphs(Envelope *e) {
+    for (int n = 0; n <= kEnvPipeMax; ++n) {
+        if (e->gexec[n]) (void)hipGraphExecDestroy(e->gexec[n]);
+        e->gexec[n] = nullptr;
+        e->g_seen[n] = false;
+    }
 }
 
 // One transform per block, as the wake solves' column pass: 256^2 x 1000 slices
@@ -348,10 +351,10 @@ int env_transform(Envelope *e, int e0, int s0, int ns, double dt, bool use_dcur,
     return glaunch_rows_inv(S, (const double2 *)sp0, (const double2 *)sp1, snk, 2, s, none, 0, ns);
 }
 
-// Steps in flight at once: enough to fill the chip (2^20 nodes), at most 16; 256^2 takes
+// Steps in flight at once: enough to fill the chip (2^20 nodes), at most kEnvPipeMax; 256^2 takes
 // 16, 512^2 four, 1024^2 (whose launches fill it alone) one.
 int pipe_depth(const Envelope *e) {
-    return (int)std::max<size_t>(1, std::min<size_t>(16, ((size_t)1 << 20) / e->nn()));
+    return (int)std::max<size_t>(1, std::min<size_t>(kEnvPipeMax, ((size_t)1 << 20) / e->nn()));
 }
 
 // Spectra and increments of `depth` steps in flight (kept: 2^20 nodes take 50 MB).  Where
@@ -360,7 +363,7 @@ int pipe_depth(const Envelope *e) {
 int ensure_pipe(Envelope *e, int &depth) {
     if (depth <= std::max(1, e->pipe)) return QP_OK;
     QP_HIP_CHECK(hipStreamSynchronize(e->stream()));
-    drop_graph(e);
+    drop_graphs(e);
     for (;; depth /= 2) {
         if (e->pipe_inc) (void)hipFree(e->pipe_inc);
         if (e->pipe_spec) (void)hipFree(e->pipe_spec);
@@ -391,11 +394,29 @@ int env_sweep(Envelope *e, double dt, int m, int ns, hipStream_t s) {
     return QP_OK;
 }
 
-// The same as a captured graph of this (dt, m, ns, stream), replayed, when use_graph.
+// The same, when use_graph, as a captured graph of this (dt, m, ns, stream): launched
+// directly the first time (a capture costs more than the launches it replaces once),
+// captured the second, replayed after.  Graphs of several ns stay side by side, for callers
+// who vary the steps of a call, whose steps split unevenly or who step the envelope in a
+// wake's passes too (one, then twelve steps of 128^2 x 60 slices: 8.3-12.7 ms with one graph
+// captured anew each time, 5.7 so); beyond kEnvGraphs of them the launches are direct.
+constexpr int kEnvGraphs = 4;
 int env_run(Envelope *e, double dt, int m, int ns, int use_graph, hipStream_t s) {
     if (!use_graph) return env_sweep(e, dt, m, ns, s);
-    if (!e->gexec || e->g_dtau != dt || e->g_iter != m || e->g_steps != ns || e->g_stream != s) {
-        drop_graph(e);
+    if (e->g_dtau != dt || e->g_iter != m || e->g_stream != s) {
+        drop_graphs(e);
+        e->g_dtau = dt;
+        e->g_iter = m;
+        e->g_stream = s;
+    }
+    hipGraphExec_t &gexec = e->gexec[ns];
+    if (!gexec) {
+        int held = 0;
+        for (hipGraphExec_t g : e->gexec) held += g != nullptr;
+        if (!e->g_seen[ns] || held >= kEnvGraphs) {
+            e->g_seen[ns] = true;
+            return env_sweep(e, dt, m, ns, s);
+        }
         hipGraph_t gr;
         QP_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         const int st = env_sweep(e, dt, m, ns, s);
@@ -408,19 +429,15 @@ int env_run(Envelope *e, double dt, int m, int ns, int use_graph, hipStream_t s)
             set_error(std::string("hipStreamEndCapture: ") + hipGetErrorString(ce));
             return QP_ERR_HIP;
         }
-        const hipError_t ie = hipGraphInstantiate(&e->gexec, gr, nullptr, nullptr, 0);
+        const hipError_t ie = hipGraphInstantiate(&gexec, gr, nullptr, nullptr, 0);
         (void)hipGraphDestroy(gr);
         if (ie != hipSuccess) {
-            e->gexec = nullptr;
+            gexec = nullptr;
             set_error(std::string("hipGraphInstantiate: ") + hipGetErrorString(ie));
             return QP_ERR_HIP;
         }
-        e->g_dtau = dt;
-        e->g_iter = m;
-        e->g_steps = ns;
-        e->g_stream = s;
     }
-    QP_HIP_CHECK(hipGraphLaunch(e->gexec, s));
+    QP_HIP_CHECK(hipGraphLaunch(gexec, s));
     return QP_OK;
 }
 
@@ -501,7 +518,7 @@ int qp_envelope_destroy(qp_envelope h) {
         return QP_ERR_STATE;
     }
     if (e->ctx) (void)hipStreamSynchronize(e->stream());
-    drop_graph(e);
+    drop_graphs(e);
     e->S.destroy();
     for (double *p : {e->a, e->inc, e->chi3, e->asq3, e->cmid, e->pipe_inc})
         if (p) (void)hipFree(p);
@@ -637,16 +654,14 @@ int qp_envelope_advance(qp_envelope h, double dtau, int steps, int chi_iteration
         QP_HIP_CHECK(hipEventRecord(ev.a, s));
     }
     if (steps > 0) ELAUNCH(k_env_cmid, dim3(e->nx), kET, 0, (const double *)e->chi3, e->cmid, e->nn());
-    // pipelines of nearly equal depth; a graph for the deeper ones, the shallower (one
-    // step less, at most) launched directly
+    // pipelines of nearly equal depth
     auto split = [steps](int depth) { return steps > 0 ? (steps + depth - 1) / depth : 0; };
     int groups = split(pipe_depth(e)), depth = groups ? (steps + groups - 1) / groups : 1;
     QP_TRY(ensure_pipe(e, depth));
     groups = split(depth);
-    const int deep = groups ? (steps + groups - 1) / groups : 0;
     for (int g = 0, left = steps; g < groups; ++g) {
         const int ns = (left + groups - g - 1) / (groups - g);
-        QP_TRY(env_run(e, dtau, chi_iterations, ns, use_graph && ns == deep, s));
+        QP_TRY(env_run(e, dtau, chi_iterations, ns, use_graph, s));
         left -= ns;
     }
     if (ms) {
