@@ -335,9 +335,9 @@ int env_transform(Envelope *e, int e0, int s0, int ns, double dt, bool use_dcur,
     const double *cmid = e->cmid + e0;
     const Ctl *none = nullptr;
     if (S.wave) {
-        QP_TRY(wlaunch_rows_fwd(S, src, sp0, sp1, 2, s, none, 0, ns));
+        QP_TRY(wlaunch_rows_fwd(S, src, sp0, sp1, 2, s, NoCtl{}, 0, ns));
         QP_TRY(wlaunch_cols_env(S, sp0, sp1, ar, ai, hdt, cmid, ns, s));
-        return wlaunch_rows_inv(S, (const double2 *)sp0, (const double2 *)sp1, snk, 2, s, none, 0, ns);
+        return wlaunch_rows_inv(S, (const double2 *)sp0, (const double2 *)sp1, snk, 2, s, NoCtl{}, 0, ns);
     }
     QP_TRY(glaunch_rows_fwd(S, src, sp0, sp1, 2, s, none, 0, ns));
     const int threads = S.ax1.dev.threads;

@@ -152,9 +152,9 @@ int solve_plain(const Solver2d &S, double D, const double *src, double *dst, hip
     const double2 *spec = S.spec[0];
     if (small_solve(S)) return slaunch(S, f, o, D, 1, s, none, 0);
     if (S.wave) {
-        QP_TRY(wlaunch_rows_fwd(S, f, S.spec[0], S.spec[0], 1, s, none, 0));
-        QP_TRY(solve_cols(S, D, 1, s, none, 0));
-        return wlaunch_rows_inv(S, spec, spec, o, 1, s, none, 0);
+        QP_TRY(wlaunch_rows_fwd(S, f, S.spec[0], S.spec[0], 1, s, NoCtl{}, 0));
+        QP_TRY(wlaunch_cols(S, D, 1, nullptr, s, NoCtl{}, 0));
+        return wlaunch_rows_inv(S, spec, spec, o, 1, s, NoCtl{}, 0);
     }
     QP_TRY(glaunch_rows_fwd(S, f, S.spec[0], S.spec[0], 1, s, none, 0));
     QP_TRY(solve_cols(S, D, 1, s, none, 0));

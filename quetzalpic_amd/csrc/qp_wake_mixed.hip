@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(kGrpTB) void kg_rows_fwd(GrpMap m, const GArgsRowsF
     double2 *sb0 = gl2, *sb1 = gl2 + grp_lds(FAM);
 #define QP_CASE(N)                                                                                                 \
     case N:                                                                                                        \
-        wrows_fwd_body<N, WfCfg<N>::E, kGrpTB, Src>(a.src, a.spec0, a.spec1, a.n1, a.tw2, a.ctl, skip_mode, nspec, \
+        wrows_fwd_body<N, WfCfg<N>::E, kGrpTB>(a.src, a.spec0, a.spec1, a.n1, a.tw2, a.ctl, skip_mode, nspec, \
                                                     a.sstride, bx, by, sb0, sb1, nullptr);                         \
         break;
     if constexpr (FAM == 0) {

@@ -42,9 +42,11 @@ struct WfCfg {
 };
 
 // Sources whose rows of 1024 run with eight elements to a lane (four passes instead of
-// five, half the wavefronts): a plain 1024^2 solve 26.4 -> 26.1 us, the B sources' launch 20.15 ->
-// 19.8.  The psi source's launch was slower with eight (12.7 -> 13.2 us), as were the column
-// pass (a solve 26.3 -> 26.5) and the inverse rows of both sinks (13.8 -> 14.2, 10.1 -> 10.3).
+// five, half the wavefronts): a plain 1024^2 solve 26.03 -> 25.82 us, the B sources' launch
+// 20.15 -> 19.8.  The psi source's launch was slower with eight (12.7 -> 13.2 us), as were the
+// column pass (a solve 26.3 -> 26.5) and the inverse rows of both sinks (13.8 -> 14.2, 10.1 ->
+// 10.3).  Rows of 512 (three passes instead of five) have four: with eight a plain 512^2 solve
+// takes 15.9 us for 16.4, which has not been weighed for the B sources.
 template <class Src>
 constexpr bool eight_per_lane = false;
 template <>
@@ -81,14 +83,14 @@ __device__ __forceinline__ void block_sum3(double &a, double &b, double &c) {
 // by) and LDS buffers as arguments: the plain kernels pass blockIdx and their
 // own static LDS, the group launch (several batches of different grid sizes
 // in one launch) the coordinates inside one batch and a shared dynamic buffer.
-template <int N2, int E, int TB, class Src>
+template <int N2, int E, int TB, class Src, class C>
 __device__ __forceinline__ void wrows_fwd_body(const Src &src, double2 *spec0, double2 *spec1, int n1,
-                                               const double2 *tw2, const Ctl *ctl, int skip_mode, int nspec,
+                                               const double2 *tw2, C ctls, int skip_mode, int nspec,
                                                size_t sstride, int bx, int by, double2 *sb0, double2 *sb1,
                                                double2 *twl) {
     using W = WfShape<N2, E, TB>;
     const int which = by % nspec, wk = by / nspec;
-    if (ctl) ctl += wk;
+    const C ctl = ctl_of(ctls, wk);
     const int skip = solver_skip_flag(ctl, skip_mode);
     double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
     const int tid = threadIdx.x;
@@ -113,7 +115,7 @@ __device__ __forceinline__ void wrows_fwd_body(const Src &src, double2 *spec0, d
     double2 v[E];
 #pragma unroll
     for (int r = 0; r < E; ++r) v[r] = make_double2(xa[r], xb[r]);
-    keep_here(v);
+    keep_for_skip(ctl, v);
     if (solver_skip_act(ctl, skip_mode, skip)) return;
     if (ra < n1) src.template done<E>(wk, which, ra, j, W::L);
     if (rb < n1) src.template done<E>(wk, which, rb, j, W::L);
@@ -141,13 +143,13 @@ __device__ __forceinline__ void wrows_fwd_body(const Src &src, double2 *spec0, d
     }
 }
 
-template <int N2, int E, int TB, class Src>
+template <int N2, int E, int TB, class Src, class C>
 __global__ __launch_bounds__(TB) void kw_rows_fwd(Src src, double2 *spec0, double2 *spec1, int n1,
-                                                  const double2 *tw2, const Ctl *ctl, int skip_mode, int nspec,
+                                                  const double2 *tw2, C ctl, int skip_mode, int nspec,
                                                   size_t sstride) {
     using W = WfShape<N2, E, TB>;
     __shared__ double2 sb0[W::LDS], sb1[W::LDS], twl[WfTw<N2, E, TB>::NL];
-    wrows_fwd_body<N2, E, TB, Src>(src, spec0, spec1, n1, tw2, ctl, skip_mode, nspec, sstride, blockIdx.x,
+    wrows_fwd_body<N2, E, TB>(src, spec0, spec1, n1, tw2, ctl, skip_mode, nspec, sstride, blockIdx.x,
                                    blockIdx.y, sb0, sb1, twl);
 }
 
@@ -161,15 +163,15 @@ __global__ __launch_bounds__(TB) void kw_rows_fwd(Src src, double2 *spec0, doubl
 // and l = n2/2, else 2); per block: bpart[2b] = first sum, bpart[2b+1] =
 // second, and block 0 writes Re G[0][0] to bpart[2 gridDim.x] (each wake of
 // a batch at its own offset bstride).
-template <int N1, int E, int TB>
+template <int N1, int E, int TB, class C>
 __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int nh, int n2, const double2 *tw1,
                                            const double *lam1, const double *lam2, double D, double *bpart,
-                                           const Ctl *ctl, int skip_mode, int nspec, size_t sstride,
+                                           C ctls, int skip_mode, int nspec, size_t sstride,
                                            size_t bstride, int bx, int by, int gx, double2 *sb0, double2 *sb1,
                                            double2 *twl) {
     using W = WfShape<N1, E, TB>;
     const int which = by % nspec, wk = by / nspec;
-    if (ctl) ctl += wk;
+    const C ctl = ctl_of(ctls, wk);
     const int skip = solver_skip_flag(ctl, skip_mode);
     double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
     if (bpart) bpart += wk * bstride;
@@ -188,7 +190,7 @@ __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int n
         lm[r] = lam1[j + W::L * r];
     }
     const double l2 = valid ? lam2[l] : 0.0;
-    keep_here(v);
+    keep_for_skip(ctl, v);
     if (solver_skip_act(ctl, skip_mode, skip)) return;
     double2 *b0 = sb0 + tt * W::PADN, *b1 = sb1 + tt * W::PADN;
     wave_fft<N1, E, -1>(v, b0, b1, tw, j);
@@ -229,10 +231,10 @@ __device__ __forceinline__ void wcols_body(double2 *spec0, double2 *spec1, int n
     }
 }
 
-template <int N1, int E, int TB>
+template <int N1, int E, int TB, class C>
 __global__ __launch_bounds__(TB) void kw_cols(double2 *spec0, double2 *spec1, int nh, int n2, const double2 *tw1,
                                               const double *lam1, const double *lam2, double D, double *bpart,
-                                              const Ctl *ctl, int skip_mode, int nspec, size_t sstride,
+                                              C ctl, int skip_mode, int nspec, size_t sstride,
                                               size_t bstride) {
     using W = WfShape<N1, E, TB>;
     __shared__ double2 sb0[W::LDS], sb1[W::LDS], twl[WfTw<N1, E, TB>::NL];
@@ -243,14 +245,14 @@ __global__ __launch_bounds__(TB) void kw_cols(double2 *spec0, double2 *spec1, in
 // Rows inverse (c2r): Z[k] = X[k] + i Y[k] with X[-k] = conj X[k]; the
 // imaginary parts of the k = 0 and k = n2/2 terms are ignored (FFTW c2r
 // semantics).  Re z -> row 2p, Im z -> row 2p+1, handed to the sink.
-template <int N2, int E, int TB, class Sink, bool STAGE>
+template <int N2, int E, int TB, class Sink, bool STAGE, class C>
 __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const double2 *spec1, Sink sink, int n1,
-                                               const double2 *tw2, const Ctl *ctl, int skip_mode, int nspec,
+                                               const double2 *tw2, C ctls, int skip_mode, int nspec,
                                                size_t sstride, int bx, int by, double2 *sb0, double2 *sb1,
                                                double2 *twl) {
     using W = WfShape<N2, E, TB>;
     const int which = by % nspec, wk = by / nspec;
-    if (ctl) ctl += wk;
+    const C ctl = ctl_of(ctls, wk);
     const int skip = solver_skip_flag(ctl, skip_mode);
     const double2 *spec = (which == 0 ? spec0 : spec1) + wk * sstride;
     const int tid = threadIdx.x;
@@ -283,23 +285,18 @@ __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const doubl
     }
     const double2 *st = sb1 + tt * W::PADN;
     double2 v[E], u[E];
+    if constexpr (!staged) {
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const int k = j + W::L * r;
-        const int kk = k > N2 / 2 ? N2 - k : k;
-        if constexpr (staged) {
-            v[r] = st[kk];
-            u[r] = st[NHF + kk];
-        } else {
+        for (int r = 0; r < E; ++r) {
+            const int k = j + W::L * r;
+            const int kk = k > N2 / 2 ? N2 - k : k;
             // rows beyond n1 read row n1 - 1 and go nowhere
             v[r] = spec[(size_t)kk * n1 + (ra < n1 ? ra : n1 - 1)];
             u[r] = spec[(size_t)kk * n1 + (rb < n1 ? rb : n1 - 1)];
         }
-    }
-    if constexpr (!staged) {
         sink.prep(wk);
-        keep_here(v);
-        keep_here(u);
+        keep_for_skip(ctl, v);
+        keep_for_skip(ctl, u);
         if (solver_skip_act(ctl, skip_mode, skip)) return;
     }
 #pragma unroll
@@ -307,8 +304,14 @@ __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const doubl
         const int k = j + W::L * r;
         const bool cj = k > N2 / 2;
         const int kk = cj ? N2 - k : k;
-        double2 X = v[r], Y = u[r];
-        if (rb >= n1) Y = make_double2(0.0, 0.0);
+        double2 X, Y;
+        if constexpr (staged) {
+            X = st[kk];
+            Y = st[NHF + kk];
+        } else {
+            X = v[r];
+            Y = rb < n1 ? u[r] : make_double2(0.0, 0.0);
+        }
         if (cj) {
             X.y = -X.y;
             Y.y = -Y.y;
@@ -330,9 +333,9 @@ __device__ __forceinline__ void wrows_inv_body(const double2 *spec0, const doubl
     }
 }
 
-template <int N2, int E, int TB, class Sink, bool STAGE>
+template <int N2, int E, int TB, class Sink, bool STAGE, class C>
 __global__ __launch_bounds__(TB) void kw_rows_inv(const double2 *spec0, const double2 *spec1, Sink sink, int n1,
-                                                  const double2 *tw2, const Ctl *ctl, int skip_mode, int nspec,
+                                                  const double2 *tw2, C ctl, int skip_mode, int nspec,
                                                   size_t sstride) {
     using W = WfShape<N2, E, TB>;
     __shared__ double2 sb0[W::LDS], sb1[W::LDS], twl[WfTw<N2, E, TB>::NL];
@@ -356,29 +359,30 @@ inline int wcols_blocks(int n1, int nh) {
 
 // nw wakes of one batch: spectra of wake w at spec0/spec1 + w * n1 * nh, control
 // blocks at ctl + w.
-template <class Src>
+template <class Src, class C>
 int wlaunch_rows_fwd(const Solver2d &S, const Src &src, double2 *spec0, double2 *spec1, int nspec, hipStream_t s,
-                     const Ctl *ctl, int skip_mode, int nw = 1) {
+                     C ctl, int skip_mode, int nw = 1) {
     const size_t sstride = (size_t)S.n1 * S.nh;
     wf_dispatch(S.n2, [&](auto NC) {
         constexpr int N = decltype(NC)::value;
         constexpr bool eight = N == 1024 && eight_per_lane<Src>;
         constexpr int E = eight ? 8 : WfCfg<N>::E, TB = eight ? WfCfg<N>::TB / 2 : WfCfg<N>::TB;
         const dim3 grid(wrows_blocks_t(S.n1, WfShape<N, E, TB>::T), nspec * nw);
-        hipLaunchKernelGGL((kw_rows_fwd<N, E, TB, Src>), grid, dim3(TB), 0, s, src, spec0, spec1, S.n1,
+        hipLaunchKernelGGL((kw_rows_fwd<N, E, TB, Src, C>), grid, dim3(TB), 0, s, src, spec0, spec1, S.n1,
                            (const double2 *)S.ax2.dev.tw, ctl, skip_mode, nspec, sstride);
     });
     QP_HIP_CHECK(hipGetLastError());
     return QP_OK;
 }
 
-inline int wlaunch_cols(const Solver2d &S, double D, int nspec, double *bpart, hipStream_t s, const Ctl *ctl,
-                        int skip_mode, int nw = 1, size_t bstride = 0) {
+template <class C>
+int wlaunch_cols(const Solver2d &S, double D, int nspec, double *bpart, hipStream_t s, C ctl, int skip_mode,
+                 int nw = 1, size_t bstride = 0) {
     const size_t sstride = (size_t)S.n1 * S.nh;
     wf_dispatch(S.n1, [&](auto NC) {
         constexpr int N = decltype(NC)::value, E = WfCfg<N>::E, TB = WfCfg<N>::TBC;
         const dim3 grid(wcols_blocks_t(S.nh, WfShape<N, E, TB>::T), nspec * nw);
-        hipLaunchKernelGGL((kw_cols<N, E, TB>), grid, dim3(TB), 0, s, S.spec[0], S.spec[1], S.nh, S.n2,
+        hipLaunchKernelGGL((kw_cols<N, E, TB, C>), grid, dim3(TB), 0, s, S.spec[0], S.spec[1], S.nh, S.n2,
                            (const double2 *)S.ax1.dev.tw, (const double *)S.d_lam1, (const double *)S.d_lam2, D,
                            bpart, ctl, skip_mode, nspec, sstride, bstride);
     });
@@ -386,9 +390,9 @@ inline int wlaunch_cols(const Solver2d &S, double D, int nspec, double *bpart, h
     return QP_OK;
 }
 
-template <class Sink>
+template <class Sink, class C>
 int wlaunch_rows_inv(const Solver2d &S, const double2 *spec0, const double2 *spec1, const Sink &sink, int nspec,
-                     hipStream_t s, const Ctl *ctl, int skip_mode, int nw = 1) {
+                     hipStream_t s, C ctl, int skip_mode, int nw = 1) {
     const size_t sstride = (size_t)S.n1 * S.nh;
     wf_dispatch(S.n2, [&](auto NC) {
         constexpr int N = decltype(NC)::value, E = WfCfg<N>::E, TB = WfCfg<N>::TB;
@@ -398,10 +402,10 @@ int wlaunch_rows_inv(const Solver2d &S, const double2 *spec0, const double2 *spe
         // One 256^2 wake (64 or 128 blocks, latency bound) was slower staged,
         // 268.7 -> 282.2 ms per pass, so small launches read directly.
         if (N >= 1024 || grid.x * grid.y >= 1024)
-            hipLaunchKernelGGL((kw_rows_inv<N, E, TB, Sink, true>), grid, dim3(TB), 0, s, spec0, spec1, sink, S.n1,
+            hipLaunchKernelGGL((kw_rows_inv<N, E, TB, Sink, true, C>), grid, dim3(TB), 0, s, spec0, spec1, sink, S.n1,
                                (const double2 *)S.ax2.dev.tw, ctl, skip_mode, nspec, sstride);
         else
-            hipLaunchKernelGGL((kw_rows_inv<N, E, TB, Sink, false>), grid, dim3(TB), 0, s, spec0, spec1, sink, S.n1,
+            hipLaunchKernelGGL((kw_rows_inv<N, E, TB, Sink, false, C>), grid, dim3(TB), 0, s, spec0, spec1, sink, S.n1,
                                (const double2 *)S.ax2.dev.tw, ctl, skip_mode, nspec, sstride);
     });
     QP_HIP_CHECK(hipGetLastError());
