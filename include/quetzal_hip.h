@@ -169,8 +169,8 @@ int qp_wake_window_stats(qp_wake w, int member, long long *overflow_blocks, long
  * instantiated tiles is in qp_wake_describe.  No reference counterpart. */
 int qp_wake_set_tile(qp_wake w, int threads_per_block, int window_nodes);
 /* JSON description of the launch shapes the library picked for this wake
- * (particle tile and the list of instantiated tiles; FFT rows/columns per
- * block of the generic kernels). */
+ * (particle tile and the list of instantiated tiles; the generic kernels' FFT
+ * rows/columns per block, always 1). */
 int qp_wake_describe(qp_wake w, char *buf, size_t len);
 /* Copy the current particle state back (FP64 SoA; any pointer may be NULL). */
 int qp_wake_get_particles(qp_wake w, size_t np, double *y, double *z, double *py, double *pz);

@@ -570,12 +570,12 @@ int wake_alloc_common(Wake *w) {
     const size_t nn = w->nn();
     const size_t nw = (size_t)w->nw;
     QP_TRY(w->S.init(p.ny, p.nz, p.dy, p.dz, w->nw));
-    const int ngrids = 27;
-    QP_HIP_CHECK(hipMalloc(&w->g_base, sizeof(double) * nn * nw * ngrids));
-    QP_HIP_CHECK(hipMemset(w->g_base, 0, sizeof(double) * nn * nw * ngrids));
     double **grids[] = {&w->src, &w->psi, &w->psi_prev, &w->psim, &w->rho, &w->jx, &w->jy, &w->jz, &w->jyn,
                         &w->jzn, &w->rho_ion, &w->by, &w->bz, &w->chi, &w->ex, &w->ey,
-                        &w->ez, &w->src2, &w->asq2, &w->psi_b[0], &w->psi_b[1], &w->zero2, &w->bx};
+                        &w->ez, &w->asq2, &w->psi_b[0], &w->psi_b[1], &w->zero2, &w->bx};
+    const size_t ngrids = sizeof(grids) / sizeof(*grids);
+    QP_HIP_CHECK(hipMalloc(&w->g_base, sizeof(double) * nn * nw * ngrids));
+    QP_HIP_CHECK(hipMemset(w->g_base, 0, sizeof(double) * nn * nw * ngrids));
     int gi = 0;
     for (double **g : grids) *g = w->g_base + nn * nw * (gi++);
     QP_HIP_CHECK(hipMalloc(&w->ctl, sizeof(Ctl) * nw));

@@ -30,7 +30,6 @@ void set_error(const std::string &msg);
 // ------------------------------------------------------------ FFT plan
 constexpr int kMaxStages = 12;
 constexpr int kMaxN = 1024;          // longest transform the LDS kernels take
-constexpr int kLdsComplex = 1024;    // complex doubles per LDS data buffer (16 KiB; two buffers)
 
 // One transform axis as the kernels see it (passed by value).
 struct FftAxisDev {
@@ -91,7 +90,6 @@ struct Ctl {
 };
 
 __device__ __forceinline__ bool ctl_skip(const Ctl *c) { return c->stop_acc != 0; }
-__device__ __forceinline__ bool ctl_skip_b(const Ctl *c) { return c->stop_now != 0; }
 // c is the control block of the launching block's wake.  Every skipping block
 // latches (the same value): in a group launch blockIdx.x is a flat index over
 // all batches and members, so no single block index is present for each wake.

@@ -295,19 +295,6 @@ __device__ __forceinline__ int rel_idx(int j, int ref, int n) {
     return d;
 }
 
-// Sum over the block (blockDim.x a multiple of 64, <= 1024); result in every thread.
-__device__ inline double block_sum(double v) {
-    __shared__ double part[16];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) part[wv] = v;
-    __syncthreads();
-    double s = 0.0;
-    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += part[i];
-    return s;
-}
-
 // Min over the wavefront, the same value in every lane: four DPP steps inside
 // each 16-lane row (lane ^ 1, lane ^ 2, half-row mirror, row mirror) leave the
 // row's min in all of its lanes, then the four rows are read out.  Every lane

@@ -69,7 +69,7 @@ struct Wake {
     double *src = nullptr, *psi = nullptr, *psi_prev = nullptr, *psim = nullptr, *rho = nullptr,
            *jx = nullptr, *jy = nullptr, *jz = nullptr, *jyn = nullptr, *jzn = nullptr,
            *rho_ion = nullptr, *by = nullptr, *bz = nullptr, *chi = nullptr, *ex = nullptr,
-           *ey = nullptr, *ez = nullptr, *src2 = nullptr, *asq2 = nullptr, *psi_b[2] = {nullptr, nullptr},
+           *ey = nullptr, *ez = nullptr, *asq2 = nullptr, *psi_b[2] = {nullptr, nullptr},
            *zero2 = nullptr, *bx = nullptr;
     // driver inputs (the 3D arrays only for a single wake)
     double *a_sqr3 = nullptr;            // nx*ny*nz or null
