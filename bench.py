@@ -420,14 +420,20 @@ def bench_c5(args, capi, workloads):
     print(json.dumps(line), flush=True)
 
 
+def pushed_slices(nx, slices, stop):
+    """Slices of a pass that push particles: all but slice 0, those down to the stop
+    slice where the pass stopped (stop >= 0)."""
+    return slices - 1 if stop < 0 else nx - stop
+
+
 def pass_rate(capi, ctx, wl, steps):
-    """Whole-pass rate of one wake (mixed, hipGraph slice step): (ms, pushes/s)."""
+    """Whole-pass rate of one wake (mixed, hipGraph slice step): (ms, pushes/s, stop slice)."""
     wk = make_wake(capi, ctx, wl, capi.QP_PREC_MIXED)
-    wk.run()
+    _, _, stop = wk.run()
     t = timed_steps(ctx, steps, lambda k: wk.run())
     wk.close()
     ms = 1e3 * t / steps
-    return ms, wl.n_particles * (wl.nx - 1) / (ms * 1e-3)
+    return ms, wl.n_particles * pushed_slices(wl.nx, wl.nx, stop) / (ms * 1e-3), stop
 
 
 def bench_extras(args, capi, workloads):
@@ -437,9 +443,11 @@ def bench_extras(args, capi, workloads):
     ctx = capi.Context(0)
     for name, steps in (("C2", 3), ("C3", 2)):
         wl = workloads.get(name)
-        ms, rate = pass_rate(capi, ctx, wl, steps)
-        out[name] = {"ms_per_pass": ms, "pushes_per_s": rate, "particles": wl.n_particles, "slices": wl.nx}
-        log(f"[bench] {name}: {ms:.1f} ms per pass -> {rate:.3e} pushes/s")
+        ms, rate, stop = pass_rate(capi, ctx, wl, steps)
+        out[name] = {"ms_per_pass": ms, "pushes_per_s": rate, "particles": wl.n_particles, "slices": wl.nx,
+                     "stop_slice": stop}
+        log(f"[bench] {name}: {ms:.1f} ms per pass -> {rate:.3e} pushes/s"
+            + (f" (stops at slice {stop})" if stop >= 0 else ""))
         if name == "C3" and not args.no_profile:
             out[name]["deposit_windows"] = window_report(capi, ctx, wl)
     ctx.close()
@@ -684,16 +692,17 @@ def bench_single(args, capi, workloads):
                    slice_limit=args.slice_limit)
     for _ in range(args.warmup):
         wk.run()
-    dev_ms = []
+    dev_ms, stop = [], -1
 
     def step(k):
-        wk.run()
+        nonlocal stop
+        _, _, stop = wk.run()
         dev_ms.append(wk.last_time_ms())
 
     t = timed_steps(ctx, args.steps, step)
     ms_per_step = 1e3 * t / args.steps
-    slices = args.slice_limit or wl.nx
-    value = wl.n_particles * (slices - 1) / (ms_per_step * 1e-3)
+    pushed = pushed_slices(wl.nx, args.slice_limit or wl.nx, stop)
+    value = wl.n_particles * pushed / (ms_per_step * 1e-3)
     log(f"[bench] mixed: {ms_per_step:.2f} ms/pass wall, device {np.median(dev_ms):.2f} ms -> {value:.3e} pushes/s")
     tuning = json.loads(wk.describe())
     classes, roofline, sroof = {}, None, None
@@ -719,8 +728,8 @@ def bench_single(args, capi, workloads):
         "metric": "particle-slice pushes/s (mixed precision, 1 MI355X, <=1e-5 rel err in psi and Ez vs FP64)",
         "value": value, "unit": "particle-slice pushes/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64",
-        "data": "synthetic", "config": wl.describe(),
-        "solves_per_s": ((1 + 3 * wl.K) * (slices - 1) + 1) / (ms_per_step * 1e-3),
+        "data": "synthetic", "config": wl.describe(), "stop_slice": stop,
+        "solves_per_s": ((1 + 3 * wl.K) * pushed + (stop < 0)) / (ms_per_step * 1e-3),
         "device_ms_per_step": float(np.median(dev_ms)), "kernel_classes": classes, "launch_shapes": tuning,
         "roofline": roofline, "solve_roofline": sroof, "fp64_gpu_pushes_per_s_leading": fp64_rate,
         "err_vs_fp64_gpu_leading": err64, "cpu_baseline": cpu,
