@@ -63,8 +63,7 @@ struct MxPart {
     double *w;
     double2 *ps;   // p* (y, z)
     double *iv;    // 1/(1 + psi) at the slice's position, from the first B to every C of a slice
-    int4 *wq;      // per particle block: the node window of its cells (origin j, k; rows,
-                   // columns), from A to the slice's B and C
+    int4 *wq;      // per particle block: its windows for the slice's B and C, from A (win_entry)
     int np;
     int pstride;
     const int *npw;
@@ -372,41 +371,54 @@ __device__ inline Win block_window(int rmin, int rmax, int cmin, int cmax, int j
     return w;
 }
 
-// A window kept for a later launch of the same block, with `lo` rows and columns
-// more ahead of it and `hi` more behind it (each below the grid's sides): padded.  Where
-// that does not fit the sides or the capacity, the kept window itself, if it does: it
-// holds the deposits at the cells and most of those a half step away (the others, at its
-// rim, take global atomics).  So blocks that straddle two tiles, as after a re-binning
-// (17 x 33 nodes, padded 19 x 35 or 20 x 36), keep their window: of a 1024^2 x 120-slice
-// wake re-binned every 20 slices 3.2 % of the blocks had none, now 0.09 % (152.5 -> 138.8 ms).
+// The block's cell window as the A phase keeps it for the slice's B and C launches, one
+// entry each: with a margin of `lo` rows and columns ahead of it and `hi` behind it (each
+// below the grid's sides), padded; where that does not fit the sides or the capacity, the
+// cell window itself, if it does.  It holds the deposits at the cells and most of those a
+// half step away (the others, at its rim, take global atomics).  So blocks that straddle
+// two tiles, as after a re-binning (17 x 33 nodes, padded 19 x 35 or 20 x 36), keep their
+// window: of a 1024^2 x 120-slice wake re-binned every 20 slices 3.2 % of the blocks had
+// none, now 0.09 % (152.5 -> 138.8 ms).
+// Entry: x = j0 | k0 << 16, y = rows | columns << 11 | padded << 22 | fits << 23 (sides up
+// to 1024, so a window has at most 1027 rows).
 template <int CAP>
-__device__ __forceinline__ Win win_load(const int4 *t, int blk, int lo, int hi, int n1, int n2, bool &padded) {
-    const int4 d = t[blk];
-    Win w;
-    w.j0 = __builtin_amdgcn_readfirstlane(d.x);
-    w.k0 = __builtin_amdgcn_readfirstlane(d.y);
-    w.wj = __builtin_amdgcn_readfirstlane(d.z);
-    w.wk = __builtin_amdgcn_readfirstlane(d.w);
-    if (w.wj == 0) {  // a block without particles
-        w.j0 = w.k0 = 0;
-        w.lds = padded = true;
-        return w;
+__device__ __forceinline__ int2 win_entry(const Win &c, int lo, int hi, int n1, int n2) {
+    Win w = c;
+    bool padded = true, fits = true;
+    if (c.wj != 0) {  // (0: a block without particles)
+        const int pj = c.wj + lo + hi, pk = c.wk + lo + hi;
+        padded = pj <= n1 && pk <= n2 && pj * pk <= CAP;
+        if (padded) {
+            w.j0 -= lo;
+            w.k0 -= lo;
+            if (w.j0 < 0) w.j0 += n1;
+            if (w.k0 < 0) w.k0 += n2;
+            w.wj = pj;
+            w.wk = pk;
+        }
+        fits = padded || c.lds;
     }
-    const int pj = w.wj + lo + hi, pk = w.wk + lo + hi;
-    padded = pj <= n1 && pk <= n2 && pj * pk <= CAP;
-    if (padded) {
-        w.j0 -= lo;
-        w.k0 -= lo;
-        if (w.j0 < 0) w.j0 += n1;
-        if (w.k0 < 0) w.k0 += n2;
-        w.wj = pj;
-        w.wk = pk;
-    }
-    w.lds = (w.wj <= n1 && w.wk <= n2 && w.wj * w.wk <= CAP);
-    return w;
+    return make_int2(w.j0 | w.k0 << 16, w.wj | w.wk << 11 | (int)padded << 22 | (int)fits << 23);
 }
-__device__ __forceinline__ void win_store(int4 *t, int blk, const Win &w) {
-    if (threadIdx.x == 0) t[blk] = make_int4(w.j0, w.k0, w.wj, w.wk);
+template <int CAP>
+__device__ __forceinline__ void win_store(int4 *t, int blk, const Win &c, int n1, int n2) {
+    if (threadIdx.x == 0) {
+        const int2 b = win_entry<CAP>(c, 1, 1, n1, n2), d = win_entry<CAP>(c, 2, 1, n1, n2);
+        t[blk] = make_int4(b.x, b.y, d.x, d.y);
+    }
+}
+// which: 0 for B, 1 for C.
+__device__ __forceinline__ Win win_load(const int4 *t, int blk, int which, bool &padded) {
+    const int2 d = reinterpret_cast<const int2 *>(t)[2 * blk + which];
+    const int x = __builtin_amdgcn_readfirstlane(d.x), y = __builtin_amdgcn_readfirstlane(d.y);
+    Win w;
+    w.j0 = x & 0xffff;
+    w.k0 = x >> 16;
+    w.wj = y & 0x7ff;
+    w.wk = y >> 11 & 0x7ff;
+    padded = y >> 22 & 1;
+    w.lds = y >> 23 & 1;
+    return w;
 }
 
 // Count a block that deposits but whose window exceeds its capacity (it falls back

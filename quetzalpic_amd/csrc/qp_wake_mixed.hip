@@ -131,7 +131,7 @@ __device__ __forceinline__ void mx_A(MxPart P, MxGeom g, MxSliceIn si, const dou
     int rmin = INT_MAX, rmax = INT_MIN, cmin = INT_MAX, cmax = INT_MIN;
     if (valid) range_add(q.j, q.k, jref, kref, n1, n2, rmin, rmax, cmin, cmax);
     const Win win = block_window<CAP>(rmin, rmax, cmin, cmax, jref, kref, n1, n2, sh);
-    win_store(P.wq, mx_blk<PT>(P, wk, bx), win);
+    win_store<CAP>(P.wq, mx_blk<PT>(P, wk, bx), win, n1, n2);
     win_note_overflow(win.lds, ctl);
     win_zero<CAP>(lds, 1, win);
     __syncthreads();
@@ -235,7 +235,7 @@ __device__ __forceinline__ void mx_B(MxPart P, MxGeom g, MxSliceIn si, const dou
     double2 pst = make_double2(0.0, 0.0);
     if (!CHI) pst = P.ps[p];  // P6 of the previous iteration (:503-505)
     bool padded;
-    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 1, 1, n1, n2, padded);
+    const Win win = win_load(P.wq, mx_blk<PT>(P, wk, bx), 0, padded);
     if (stop) {
         ctl_latch(ctl);
         return;
@@ -382,7 +382,7 @@ __device__ __forceinline__ void mx_C(MxPart P, MxGeom g, const double *psim, dou
     const double w = P.w[p], iv = P.iv[p];
     const double2 pst = P.ps[p];
     bool padded;
-    const Win win = win_load<CAP>(P.wq, mx_blk<PT>(P, wk, bx), 2, 1, n1, n2, padded);
+    const Win win = win_load(P.wq, mx_blk<PT>(P, wk, bx), 1, padded);
     if (stop) {
         ctl_latch(ctl);
         return;
