@@ -216,7 +216,6 @@ int qp_wake_destroy(qp_wake h) {
     if (w->h_out) (void)hipHostFree(w->h_out);
     if (w->ev0) (void)hipEventDestroy(w->ev0);
     if (w->ev1) (void)hipEventDestroy(w->ev1);
-    if (w->ev_mark) (void)hipEventDestroy(w->ev_mark);
     for (hipEvent_t e : w->prof_ev) (void)hipEventDestroy(e);
     delete h;
     return QP_OK;
@@ -582,7 +581,9 @@ int wake_alloc_common(Wake *w) {
     QP_HIP_CHECK(hipMemset(w->ctl, 0, sizeof(Ctl) * nw));
     QP_HIP_CHECK(hipMalloc(&w->d_laser, sizeof(LaserGauss) * nw));
     QP_HIP_CHECK(hipMemset(w->d_laser, 0, sizeof(LaserGauss) * nw));
-    QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * (nn * kOutPlanes + kCtlWords + 1), hipHostMallocDefault));
+    const size_t words = nn * kOutPlanes + kCtlWords;
+    QP_HIP_CHECK(hipHostMalloc(&w->h_out, sizeof(double) * words + sizeof(int) * nw, hipHostMallocDefault));
+    w->h_prog = reinterpret_cast<int *>(w->h_out + words);
     QP_HIP_CHECK(hipEventCreate(&w->ev0));
     QP_HIP_CHECK(hipEventCreate(&w->ev1));
     return QP_OK;

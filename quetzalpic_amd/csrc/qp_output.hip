@@ -1,7 +1,9 @@
 // qp_output.hip -- what a pass hands to the host while it runs: per-slice output, where the
 // planes of a view leave the device in one launch (output_step, src/System_3d.cpp:629-666,
 // writes them slice by slice), and the number of members that have not stopped.
+#include <climits>
 #include <string>
+#include <thread>
 
 #include "qp_wake.h"
 
@@ -27,32 +29,42 @@ __global__ __launch_bounds__(kPackT) void k_pack(OutPlanes o, size_t plane, cons
         d[t] = src ? src[t] : 0.0;
 }
 
-// Members of the batches that have not stopped.
-__global__ __launch_bounds__(64) void k_running(CtlSets c, int *count) {
-    int n = 0;
-    for (int b = 0; b < c.nb; ++b)
-        for (int m = threadIdx.x; m < c.nw[b]; m += 64) n += c.ctl[b][m].stop_acc == 0;
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
-    if (threadIdx.x == 0) *count = n;
-}
-
 }  // namespace
 
-int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t &ev, hipStream_t s, int &running) {
-    if (done == 0 || done % kWatchSlices != 0) return QP_OK;
-    if (!ev) QP_HIP_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    if (done > kWatchSlices) {  // the mark before this one
-        QP_HIP_CHECK(hipEventSynchronize(ev));
-        running = *count;
-        if (!running) return QP_OK;
-    }
-    hipLaunchKernelGGL(k_running, dim3(1), dim3(64), 0, s, c, count);
-    QP_HIP_CHECK(hipGetLastError());
-    QP_HIP_CHECK(hipEventRecord(ev, s));
-    return QP_OK;
+void watch_reset(Wake *w) {
+    for (int m = 0; m < w->nw; ++m) w->h_prog[m] = INT_MAX;
 }
 
-int *Wake::h_running() const { return reinterpret_cast<int *>(h_out + kOutPlanes * nn() + kCtlWords); }
+int watch_stops(Wake *const *b, int nb, int i, hipStream_t s, int &running) {
+    int first = INT_MAX;  // the slice that the device has reached
+    auto read = [&] {
+        running = 0;
+        for (int k = 0; k < nb; ++k)
+            for (int m = 0; m < b[k]->nw; ++m) {
+                const int p = __atomic_load_n(b[k]->h_prog + m, __ATOMIC_RELAXED);
+                if (p == kStopped) continue;
+                ++running;
+                first = p < first ? p : first;
+            }
+    };
+    read();
+    // slice i + 1 set a mark: wait for the one before it, i + 1 + kWatchSlices
+    const int mark = i + 1 + kWatchSlices;
+    if ((i + 1) % kWatchSlices != 0 || mark >= b[0]->p.nx) return QP_OK;
+    for (unsigned turn = 1; running && first > mark; ++turn) {
+        if (turn % 65536 == 0) {  // the wait ends with the stream, whatever ended it
+            const hipError_t e = hipStreamQuery(s);
+            if (e != hipErrorNotReady) {
+                read();
+                QP_HIP_CHECK(e);
+                return QP_OK;
+            }
+        }
+        std::this_thread::yield();
+        read();
+    }
+    return QP_OK;
+}
 
 int pack_planes(const OutPlanes &o, size_t plane, const Ctl *ctl, int nctl, double *dst, hipStream_t s) {
     const size_t blocks = (plane + kPackT - 1) / kPackT;

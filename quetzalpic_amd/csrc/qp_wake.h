@@ -22,25 +22,23 @@ struct PartFP64 {
            *ym = nullptr, *zm = nullptr, *pyn = nullptr, *pzn = nullptr;
 };
 
-// What a pass without a callback learns of its members while it runs: every kWatchSlices
-// slices a launch counts the members that still run into a pinned word, and the host waits
-// for the count before the last one before it enqueues more.  So it stays at most
+// What a pass without a callback learns of its members while it runs: the launch that ends a
+// slice stores, every kWatchSlices slices, each member's slice into pinned memory, kStopped
+// once the member has stopped.  Before it enqueues a slice the host reads these words, and
+// every kWatchSlices slices it waits for the mark before the last one.  So it stays at most
 // 2 kWatchSlices slices ahead of the device, which never runs dry, and a pass whose members
 // have all stopped ends there instead of skipping launch by launch through its remaining slices
 // (a skipped launch still loads its inputs beside the flag).  512^2 x 300 slices that stop at
-// the 111th: 86.8 -> 49.1 ms, 256^2 x 500 at the 111th 65.5 -> 25.3; passes that do not stop
-// as before (256^2 x 500 slices 109.5 and 109.7 ms).
+// the 111th: 86.8 -> 48.7 ms, 256^2 x 500 at the 111th 65.5 -> 25.4; passes that do not stop
+// take as long as before (with a launch and an event for every mark 0.3-0.4 % longer).
 constexpr int kWatchSlices = 8;
+constexpr int kStopped = -1;
 constexpr int kGroupMax = 16;  // batches of a group
-struct CtlSets {               // the control blocks of a launch's batches
-    const Ctl *ctl[kGroupMax];
-    int nw[kGroupMax];
-    int nb;
-};
-// Before slice number `done` (from 0) of a pass: sets `running` to the members that ran at
-// the last mark, where a mark is due.  `count` is pinned; `ev` is made at the first mark
-// (45 us; without time stamps: with them each mark took 14 us, not 3).
-int watch_stops(const CtlSets &c, int done, int *count, hipEvent_t &ev, hipStream_t s, int &running);
+// Stores member wk's progress at the end of slice `slice` (one thread of the launch).
+__device__ __forceinline__ void note_progress(int *prog, int wk, int slice) {
+    if (slice % kWatchSlices == 0 || slice == kStopped)
+        __hip_atomic_store(prog + wk, slice, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Host data of one member of a batch of wakes (a single wake is a batch of
 // one): the initial particles (FP64, re-uploaded every pass) and the laser.
@@ -77,9 +75,9 @@ struct Wake {
     double *rho_b3 = nullptr, *jx_b3 = nullptr;  // nx*ny*nz or null
 
     Ctl *ctl = nullptr;                  // nw control blocks
-    double *h_out = nullptr;             // pinned host staging, 12 planes, a control block, a count of members
+    double *h_out = nullptr;             // pinned host staging, 12 planes and a control block
+    int *h_prog = nullptr;               // behind them: the members' progress (note_progress)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    hipEvent_t ev_mark = nullptr;        // watch_stops
     double last_ms = 0.0;
     // mixed path: particle tile (threads per block, LDS window nodes per grid),
     // from the tile autotuner on the first pass unless set by QP_TILE
@@ -112,8 +110,6 @@ struct Wake {
 
     size_t nn() const { return (size_t)p.ny * p.nz; }
     size_t np() const { return mem[0].np; }  // particles of a single wake
-    CtlSets ctl_set() const { return CtlSets{{ctl}, {nw}, 1}; }
-    int *h_running() const;  // the count in h_out
     bool any_laser() const {
         for (const WakeMember &m : mem)
             if (m.laser_set) return true;
@@ -152,6 +148,11 @@ const double *wake_jx_b(Wake *w, int i);
 // Profiling bracket helpers (no-ops unless a profile pass is active).
 void prof_begin(Wake *w, const char *cls);
 void prof_end(Wake *w, const char *cls);
+
+// Before slice i of a pass without a callback: the members of the nb batches that have not
+// stopped, after a wait where one is due.
+int watch_stops(Wake *const *b, int nb, int i, hipStream_t s, int &running);
+void watch_reset(Wake *w);  // before a pass, its stream drained
 
 // Stage the output planes of slice i to host and call cb (bx may be null).
 // Per-slice output (qp_output.hip).  The planes of one view, in its order.

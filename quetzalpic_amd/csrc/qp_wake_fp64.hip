@@ -169,8 +169,10 @@ struct SinkB64 {
 // output_step's fields (src/System_3d.cpp:633-661).
 __global__ void k_output(double *ex, double *ey, double *ez, const double *psi, const double *psi_prev,
                          const double *by, const double *bz, int n1, int n2, double dx, double dy, double dz,
-                         int with_ex, Ctl *ctl, int final_step) {
+                         int with_ex, Ctl *ctl, int final_step, int *prog, int slice) {
     if (!final_step) {
+        const bool stopped = ctl_skip(ctl);
+        if (blockIdx.x == 0 && threadIdx.x == 0) note_progress(prog, 0, stopped ? kStopped : slice);
         SKIP_OR_LATCH(ctl);
     } else if (ctl->stop_acc) {
         by = nullptr;  // after a stop, by(0)/bz(0) are still the pass's zeros
@@ -475,11 +477,11 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
         return OutPlanes{{w->psi, w->rho, w->jx, w->jy, w->jz, w->ex, w->ey, w->ez, w->by, w->bz, w->chi, nullptr}};
     };
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
-    const CtlSets cs = w->ctl_set();
+    watch_reset(w);
     for (int i = p.nx - 1; i >= i_end; --i) {
         if (!cb) {
             int running = 1;
-            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev_mark, s, running));
+            QP_TRY(watch_stops(&w, 1, i, s, running));
             if (!running) break;
         }
         const double *asq;
@@ -521,7 +523,7 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
         if (np) LAUNCH(k_advance, pb, P, w->psim, np, g, ctl);
         prof_end(w, "push");
         LAUNCH(k_output, gb, w->ex, w->ey, w->ez, w->psi, w->psi_prev, w->by, w->bz, n1, n2, p.dx, p.dy, p.dz,
-               i < p.nx - 1 ? 1 : 0, ctl, 0);
+               i < p.nx - 1 ? 1 : 0, ctl, 0, w->h_prog, i);
         if (w->bunch) QP_TRY(bunch_slice_gather(w->bunch, w->ex, w->ey, w->ez, w->by, w->bz, ctl, -1, i, s));
         if (cb) {
             Ctl hc;
@@ -537,7 +539,7 @@ int wake_run_fp64(Wake *w, qp_slice_cb cb, void *user, int *stop_slice) {
     if (i_end == 0) {
         // output_step(0) after the loop (src/System_3d.cpp:622)
         LAUNCH(k_output, gb, w->ex, w->ey, w->ez, w->psi, w->psi_prev, w->by, w->bz, n1, n2, p.dx, p.dy, p.dz,
-               p.nx > 1 ? 1 : 0, ctl, 1);
+               p.nx > 1 ? 1 : 0, ctl, 1, w->h_prog, 0);
         // bunch bucket 0: slice 0's fields are final only after output_step(0)
         if (w->bunch) QP_TRY(bunch_slice_gather(w->bunch, w->ex, w->ey, w->ez, w->by, w->bz, ctl, -1, 0, s));
         // the envelope step after the pass (the plain path keeps the launches in order)

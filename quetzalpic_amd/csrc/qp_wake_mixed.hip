@@ -546,9 +546,11 @@ __global__ __launch_bounds__(kPT) void k_mx_ion(MxPart P, MxGeom g, double *rho_
 // the final output_step(0) the slot follows each member's own stop slice.
 __device__ __forceinline__ void mx_out(double *ex, double *ey, double *ez, const double *psi_b0, const double *psi_b1,
                          const double *by, const double *bz, int n1, int n2, double dx, double dy, double dz,
-                         int with_ex, Ctl *ctl, int slot, int final_step, int bx, int wk) {
+                         int with_ex, Ctl *ctl, int slot, int final_step, int *prog, int bx, int wk) {
     ctl += wk;
+    const bool lead = !final_step && bx == 0 && threadIdx.x == 0;
     if (!final_step) {
+        if (lead && ctl_skip(ctl)) note_progress(prog, wk, kStopped);
         MX_SKIP(ctl);
     } else {
         slot = (ctl->stop_acc ? ctl->stop_slice : 0) & 1;
@@ -565,7 +567,11 @@ __device__ __forceinline__ void mx_out(double *ex, double *ey, double *ez, const
     ez += go;
     if (by) by += go;
     if (bz) bz += go;
-    if (!final_step && bx == 0 && threadIdx.x == 0) ctl->slice_of[1 - slot] = ctl->slice_of[slot] - 1;
+    if (lead) {
+        const int slice = ctl->slice_of[slot];
+        ctl->slice_of[1 - slot] = slice - 1;
+        note_progress(prog, wk, slice);
+    }
     const size_t t = (size_t)bx * blockDim.x + threadIdx.x;
     if (t >= (size_t)n1 * n2) return;
     const int j = (int)(t / n2), k = (int)(t % n2);
@@ -577,8 +583,8 @@ __device__ __forceinline__ void mx_out(double *ex, double *ey, double *ez, const
 }
 __global__ void k_mx_out(double *ex, double *ey, double *ez, const double *psi_b0, const double *psi_b1,
                          const double *by, const double *bz, int n1, int n2, double dx, double dy, double dz,
-                         int with_ex, Ctl *ctl, int slot, int final_step) {
-    mx_out(ex, ey, ez, psi_b0, psi_b1, by, bz, n1, n2, dx, dy, dz, with_ex, ctl, slot, final_step, blockIdx.x,
+                         int with_ex, Ctl *ctl, int slot, int final_step, int *prog) {
+    mx_out(ex, ey, ez, psi_b0, psi_b1, by, bz, n1, n2, dx, dy, dz, with_ex, ctl, slot, final_step, prog, blockIdx.x,
            blockIdx.y);
 }
 
@@ -949,6 +955,7 @@ struct GArgsOut {
     int n1, n2;
     double dx, dy, dz;
     Ctl *ctl;
+    int *prog;
 };
 template <class Src>
 struct GArgsRowsF {
@@ -1019,7 +1026,7 @@ __global__ void kg_mx_out(GrpMap m, const GArgsOut *__restrict__ t, int with_ex,
     grp_locate(m, b, bx, wk);
     const GArgsOut &a = t[b];
     mx_out(a.ex, a.ey, a.ez, a.psi_b0, a.psi_b1, a.by, a.bz, a.n1, a.n2, a.dx, a.dy, a.dz, with_ex, a.ctl, slot,
-           final_step, bx, wk);
+           final_step, a.prog, bx, wk);
 }
 
 // Grid sides a group launch takes: the register-resident lengths whose
@@ -1597,7 +1604,7 @@ int enqueue_slice_t(MxRun &R, hipStream_t s, int i) {
     }
     MLAUNCH(k_mx_out, dim3(R.gb, R.nw), 256, 0, w->ex, w->ey, w->ez, (const double *)w->psi_b[0],
             (const double *)w->psi_b[1], (const double *)w->by, (const double *)w->bz, p.ny, p.nz, p.dx, p.dy, p.dz,
-            first ? 0 : 1, w->ctl, slot, 0);
+            first ? 0 : 1, w->ctl, slot, 0, w->h_prog);
     if (w->bunch)
         QP_TRY(bunch_slice_gather(w->bunch, w->ex, w->ey, w->ez, w->by, w->bz, (const Ctl *)w->ctl, slot, 0, s));
     return QP_OK;
@@ -1794,6 +1801,7 @@ int pass_setup(Wake *w, MxRun &R) {
     const qp_wake_params &p = w->p;
     hipStream_t s = w->stream();
     QP_TRY(wake_upload_mixed(w));
+    watch_reset(w);
     MixedState *m = mstate(w);
     const int nw = w->nw;
     R.w = w;
@@ -1885,7 +1893,7 @@ int pass_final_launch(Wake *w, MxRun &R) {
     // member's psi slot from its own stop slice
     hipLaunchKernelGGL(k_mx_out, dim3(R.gb, nw), dim3(256), 0, s, w->ex, w->ey, w->ez,
                        (const double *)w->psi_b[0], (const double *)w->psi_b[1], (const double *)w->by,
-                       (const double *)w->bz, p.ny, p.nz, p.dx, p.dy, p.dz, p.nx > 1 ? 1 : 0, w->ctl, 0, 1);
+                       (const double *)w->bz, p.ny, p.nz, p.dx, p.dy, p.dz, p.nx > 1 ? 1 : 0, w->ctl, 0, 1, w->h_prog);
     QP_HIP_CHECK(hipGetLastError());
     // bunch bucket 0: slice 0's fields are final only after output_step(0)
     if (w->bunch)
@@ -2081,12 +2089,11 @@ int wake_run_mixed(Wake *w, batch_cb cb, void *user, int *stop_slices) {
         }
     } join{q, writer};
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
-    const CtlSets cs = w->ctl_set();
     int running = nw;
     for (int i = p.nx - 1; i >= i_end; --i) {
         const int slot = i & 1;
         if (!cb) {
-            QP_TRY(watch_stops(cs, p.nx - 1 - i, w->h_running(), w->ev_mark, s, running));
+            QP_TRY(watch_stops(&w, 1, i, s, running));
             if (!running) break;
         }
         R.flag_first = running < nw;
@@ -2259,7 +2266,7 @@ void group_tables(Group *G, std::vector<MxRun> &R, GroupTabs &T, GroupMaps &M) {
                                                 R[b].sstride};
         }
         T.O[b] = GArgsOut{w->ex, w->ey, w->ez, w->psi_b[0], w->psi_b[1], w->by, w->bz, p.ny, p.nz, p.dx, p.dy, p.dz,
-                          w->ctl};
+                          w->ctl, w->h_prog};
         T.PC[b] = GArgsCols{S.spec[0], S.spec[0], S.n1, S.nh, S.n2, S.ax1.dev.tw, S.d_lam1, S.d_lam2, 0.0, m->bpart,
                             w->ctl, R[b].sstride, m->bstride};
         T.BC[b] = GArgsCols{S.spec[0], S.spec[1], S.n1, S.nh, S.n2, S.ax1.dev.tw, S.d_lam1, S.d_lam2, p.D, nullptr,
@@ -2475,18 +2482,13 @@ int group_run_mixed(Group *G, group_cb cb, void *user, int *stop_slices) {
         cctx[b] = GroupCbCtx{cb, user, b};
     }
     const int i_end = (p.slice_limit > 0 && p.slice_limit < p.nx) ? p.nx - p.slice_limit : 0;
-    CtlSets cs{};
     int members = 0;
-    for (Wake *w : G->b) {
-        cs.ctl[cs.nb] = w->ctl;
-        cs.nw[cs.nb++] = w->nw;
-        members += w->nw;
-    }
+    for (Wake *w : G->b) members += w->nw;
     int running = members;
     for (int i = p.nx - 1; i >= i_end; --i) {
         const int slot = i & 1;
         if (!cb) {
-            QP_TRY(watch_stops(cs, p.nx - 1 - i, G->b[0]->h_running(), G->b[0]->ev_mark, s, running));
+            QP_TRY(watch_stops(G->b.data(), nb, i, s, running));
             if (!running) break;
         }
         const int flag_first = running < members;
