@@ -144,16 +144,21 @@ def envelope_bytes_per_point(m):
 
 def bench_envelope(capi, ctx, wl, steps, use_graph=1):
     """Envelope advance on the workload's grid: chi from one mixed wake pass with
-    the attached Gaussian envelope, then `steps` steps (graph-replayed sweeps
-    unless use_graph = 0)."""
+    the attached Gaussian envelope, then `steps` calls of one step, and one call of
+    `steps` steps (graph-replayed sweeps unless use_graph = 0)."""
     env = capi.Envelope(ctx, wl.nx, wl.ny, wl.nz, wl.dx, wl.dy, wl.dz, ENV_K0)
     env.set_gaussian(*wl.laser)
     wk = make_wake(capi, ctx, wl, capi.QP_PREC_MIXED, use_graph=use_graph)
     wk.attach_envelope(env)
     wk.run()
     wk.close()
-    env.advance(ENV_DTAU, steps=1, chi_iterations=ENV_CHI_IT, use_graph=use_graph)   # graph capture
-    ms = env.advance(ENV_DTAU, steps=steps, chi_iterations=ENV_CHI_IT, use_graph=use_graph) / steps
+    def advance(n):
+        return env.advance(ENV_DTAU, steps=n, chi_iterations=ENV_CHI_IT, use_graph=use_graph)
+
+    for n in (1, 1, steps, steps):   # direct, captured
+        advance(n)
+    ms = sum(advance(1) for _ in range(steps)) / steps
+    ms_pipe = advance(steps) / steps
     # one coupled time step (wake pass + envelope step): two host calls, and the
     # step enqueued by the pass itself (qp_wake_set_envelope_step)
     wk = make_wake(capi, ctx, wl, capi.QP_PREC_MIXED, use_graph=use_graph)
@@ -161,12 +166,12 @@ def bench_envelope(capi, ctx, wl, steps, use_graph=1):
     coupled = {}
     for mode in ("two_calls", "in_pass"):
         wk.set_envelope_step(ENV_DTAU if mode == "in_pass" else 0.0, ENV_CHI_IT)
-        for rep in range(2):   # first: capture
+        for rep in range(3):   # direct, captured, replayed
             ctx.synchronize()
             t0 = time.perf_counter()
             wk.run()
             if mode == "two_calls":
-                env.advance(ENV_DTAU, steps=1, chi_iterations=ENV_CHI_IT, use_graph=use_graph)
+                advance(1)
             ctx.synchronize()
             coupled[mode] = 1e3 * (time.perf_counter() - t0)
     wk.close()
@@ -178,11 +183,12 @@ def bench_envelope(capi, ctx, wl, steps, use_graph=1):
     launches = wl.nx * 3 * (ENV_CHI_IT + 1) + 1
     achieved = byts / (ms * 1e-3) / 1e9
     res = {"k0": ENV_K0, "dtau": ENV_DTAU, "chi_iterations": ENV_CHI_IT, "graph": use_graph, "ms_per_step": ms,
+           "steps_in_one_call": steps, "ms_per_step_in_one_call": ms_pipe,
            "slices_per_s": wl.nx / (ms * 1e-3), "launches_per_step": launches,
            "us_per_launch": 1e3 * ms / launches, "algorithmic_bytes_per_step": byts,
            "achieved_GBs": achieved, "frac_hbm": achieved / HBM_PEAK_GBS, "coupled_step_ms": coupled}
     log(f"[bench] envelope: {ms:.2f} ms/step ({launches} launches, {1e3 * ms / launches:.2f} us each), "
-        f"{achieved:.0f} GB/s algorithmic")
+        f"{achieved:.0f} GB/s algorithmic; {ms_pipe:.2f} ms/step in one call of {steps}")
     return res
 
 

@@ -1,6 +1,6 @@
 // qp_mixed_kernels.h -- device code of the fused mixed-precision slice step.
 //
-// Particle layout (structure of arrays, 36 B persistent + 16 B scratch):
+// Particle layout (structure of arrays, 36 B persistent + 24 B scratch):
 //   cell  uint32   (j << 16) | k          node-origin cell of the particle
 //   off   uint2    in-cell offsets (y, z) in units of 2^-32 cell (Y = j + off.x 2^-32)
 //   p     double2  transverse momenta (y, z) (they accumulate over every slice)
@@ -12,6 +12,8 @@
 //                  an FP32 increment p* - p its rounding alone moved e_x of a
 //                  256^2 x 800-slice wake at a0 = 2.3 by 1.1e-5 of its maximum
 //                  against the FP64 oracle (the rounding enters every commit)
+//   iv   double   1/(1 + psi) at the slice's position (scratch, from B to C); wq: 16 B
+//                  of windows per particle block (scratch, from A to B and C)
 // Arithmetic is FP64 throughout (without packed FP32, FP32 and FP64 add, mul
 // and FMA issue at the same rate on gfx950); only the position is narrowed.
 // Positions are advanced in FP64 cell units and re-split with round-to-nearest
@@ -25,7 +27,7 @@
 // slice, rho in the last) and C (transverse current at the half step).  The node
 // deposits sit in B because B holds their inputs: C then gathers psi_middle only
 // and reads 1/(1 + psi) (8 B) where it gathered psi and <a^2>, divided and read p
-// (16 B).  With the shared window (see k_mx_B) one iteration's B + C took 77 + 48 us
+// (16 B).  With the shared window (see k_mx_B) one iteration's B + C takes 77 + 47 us
 // against 83 + 70 us at 1024^2 with 4.2 M particles, 23 + 16 against 26 + 22 us at
 // 512^2 with 1 M.
 #pragma once

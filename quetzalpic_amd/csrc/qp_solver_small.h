@@ -7,13 +7,15 @@
 // inverse), rows inverse, on the transforms of qp_wave_fft.h.  A transform lies inside one
 // wavefront, so the block meets twice only, at the transposes.  Same sources and sinks,
 // same member convention (blockIdx.y = wake * nspec + which).
-// Results are those of the three launches, bit for bit.
+// The transforms give the three launches' bits; psi's border mean sums the same terms in
+// another order (wavefront by wavefront), so psi agrees to rounding.
 // One CU's LDS bandwidth, its loads and FP64 rate bound it now (64^2: 9 us in a slice, its
 // sources coming from other CUs' deposits), so it ends at sides of 64.  Eight elements to a
 // lane instead of four (half the exchanges, half the wavefronts) took as long.
 // A chain of plain solves: 32^2 8.6 -> 4.3 us, 48^2 10.5 -> 7.4, 64^2 9.6-10.4 -> 7.4.  A 200-slice
 // wake of 48^2 48.0 -> 37.4 ms, of 64^2 42.5 -> 39.0 (FP64 61.7 -> 57.9); batches of 24 wakes of
-// 48^2 15.3 -> 13.2 ms, of 64^2 16.7 -> 16.2, of two wakes of 64^2 9.6 -> 10.0.
+// 48^2 15.3 -> 13.2 ms, of 64^2 16.7 -> 16.2, of two wakes of 64^2 9.6 -> 10.0 (12.1 before the
+// three launches were shortened).  Sides of 16 keep the three launches: not measured.
 #pragma once
 
 #include <type_traits>

@@ -186,8 +186,8 @@ __device__ __forceinline__ double gamma_of(double p2, double a, double ps, doubl
 // the same in every iteration (:526), so the first deposits it; a pass that stops
 // in a later iteration then still has it.
 // Waves per SIMD the B phase is bounded to, where the LDS of as many blocks fits a CU
-// (160 KB).  Unbounded the compiler takes 88 VGPRs (5 waves: 109 us at 1024^2 against
-// 89 us).  The first iteration fits 64 VGPRs (8 waves) without scratch, the others,
+// (160 KB).  Unbounded the compiler takes more registers and fewer waves: 86-95 us at 1024^2
+// against 77-80 us.  The first iteration fits 64 VGPRs (8 waves) without scratch, the others,
 // which also hold the previous p*, 72 (7 waves).
 constexpr int b_lds(int CAP, bool RHO, bool CHI) {  // doubles: the staged grids or the deposit windows
     return std::max(4 * kGwCap, (2 + RHO + CHI) * CAP);
@@ -454,7 +454,7 @@ __device__ __forceinline__ void mx_S(MxPart P, MxGeom g, MxSliceIn si, const dou
         const double inv1ps = 1.0 / (1 + ps);
         const double gm = gamma_of(py * py + pz * pz, a, ps, inv1ps);
         const double px = 0.5 * (1 + py * py + pz * pz + a - (1 + ps) * (1 + ps)) * inv1ps;
-        // S5 (:390-397) with 1/(1-vx) = gamma/(1+psi), as in the C phase
+        // S5 (:390-397) with 1/(1-vx) = gamma/(1+psi), as in the B phase
         vjx = w * px * inv1ps;
         vrho = w * gm * inv1ps;
         vchi = -w * inv1ps;
@@ -1404,8 +1404,8 @@ struct MxRun {
 };
 
 // The instantiated particle tiles (threads per block, window nodes per grid).
-// The LDS of the C phase is (2 + grids) x CAP doubles: 25.6 KB at (256, 640),
-// 40 KB at (256, 1024).
+// LDS at (256, 640) and (256, 1024): A 5 and 8 KB, C 10 and 16 KB (2 x CAP doubles), B
+// 12-20 and 16-32 KB (the staged grids or its two to four windows, b_lds).
 constexpr int kTiles[][2] = {{256, 640}, {128, 640}, {256, 1024}, {128, 384}};
 constexpr int kNumTiles = 4;
 
